@@ -1207,17 +1207,12 @@ static int ivf_candidates(bv_index *idx, const float *d_q, uint32_t nq, uint64_t
 }
 
 // ---------------------------------------------------------------- queries
-// Scanning workgroups per query: at least 256 rows each, and at most
-// 2 * CUs - 1 so that the scanning workgroups plus the threshold helper fit
-// the device at two workgroups per CU whatever the kernel's register count.
 // The fused scan's grid for n rows: one workgroup per 256 rows, at most as
 // many as the device holds at once next to the threshold helper (two per
 // CU, or one when a workgroup's LDS -- the per-wave lists, which grow with
-// the fetch -- leaves room for one only).  The helper is the grid's last
-// workgroup: with more workgroups than fit, it would start only after the
-// others, the scan would run without its bound, and every wave would flush
-// and exactly re-score all of its rows (measured 27 ms instead of 0.2 ms at
-// fetch 1024 over 1M rows).
+// the fetch -- leaves room for one only): a persistent scan with more
+// workgroups than places runs the rest after the dynamic share is gone, a
+// second round of static shares on a half-empty device.
 static uint32_t grid_for(const bv_index *idx, uint64_t n, uint32_t kprime, uint32_t rr_dim) {
     uint64_t g = (n + 255) / 256;
     const int cus = idx->dev->prop.multiProcessorCount > 0 ? idx->dev->prop.multiProcessorCount : 128;

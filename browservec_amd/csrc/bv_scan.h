@@ -2021,11 +2021,10 @@ __device__ void threshold_helper(const ScanArgs &a, uint32_t qi, TopkLds &L) {
     }
 }
 
-// Fused scan + top-k (one launch per query batch).  Workgroups 0..grid-1
-// take row blocks round-robin (block b goes to workgroup b % grid); each of
+// Fused scan + top-k (one launch per query batch).  Workgroup 0 is the
+// threshold helper; workgroups 1..grid take row blocks round-robin; each of
 // their waves keeps keys at or above its running bound in a private LDS list
-// and publishes its running maximum.  Workgroup `grid` is the threshold
-// helper.  At the end every wave flushes its keys at or above the freshest
+// and publishes its running maximum.  At the end every wave flushes its keys at or above the freshest
 // bound to a global array; the last workgroup to finish selects the best
 // kprime of the flushes.  Dynamic LDS: max(sizeof(TopkLds), 4 * wcap * 8).
 template <int C, int LPR, int UPL, bool IDX, bool PREP>
@@ -2042,7 +2041,13 @@ __device__ __forceinline__ void scan_topk_body(ScanArgs a) {
     QState *qs = a.qs + qi;
     const uint32_t kp = a.kprime;
 
-    if (blockIdx.x == a.grid) {
+    // The helper is each query's first workgroup: workgroups start in order,
+    // so it runs from the start even when another launch holds part of the
+    // device (several indexes queried at once on their own streams).  As the
+    // last one it started after every scanning workgroup had a place, and
+    // until then the scan ran without its bound: three 1M x 768 int8 indexes
+    // queried in turn took 341 us per query, one alone 184.
+    if (blockIdx.x == 0) {
         threshold_helper(a, qi, L);
         __syncthreads();
         if (tid == 0) L.last = atomicAdd(&qs->fin, 1u) == 1;
@@ -2050,6 +2055,7 @@ __device__ __forceinline__ void scan_topk_body(ScanArgs a) {
         if (L.last) reset_query(a, qi);
         return;
     }
+    const uint32_t bx = blockIdx.x - 1;  // the scanning workgroup's index
 
     const int p = lane % LPR;
     ScanRegs<C, UPL> R;
@@ -2069,7 +2075,7 @@ __device__ __forceinline__ void scan_topk_body(ScanArgs a) {
         cand = a.cand + (uint64_t)qi * a.cand_stride;
         n = a.cand_n[qi] < a.cand_stride ? a.cand_n[qi] : (uint32_t)a.cand_stride;
     }
-    uint64_t *wslot = a.wmax + (((uint64_t)qi * a.grid + blockIdx.x) * SH::WAVES + wave) * a.pub_m;
+    uint64_t *wslot = a.wmax + (((uint64_t)qi * a.grid + bx) * SH::WAVES + wave) * a.pub_m;
     uint64_t lmax = 0;
 
     const uint32_t wcap = a.wcap;
@@ -2081,7 +2087,7 @@ __device__ __forceinline__ void scan_topk_body(ScanArgs a) {
     const uint32_t ng = a.grid < (uint32_t)NGROUP ? a.grid : (uint32_t)NGROUP;
 
     // ---- a wave's stream of steps ----
-    // Static part: grabs g = blockIdx.x + gi*grid for gi < sgrabs, each wave
+    // Static part: grabs g = bx + gi*grid for gi < sgrabs, each wave
     // taking GRAB_STEPS steps of every grab (rows wofs + s * wstep..).
     // Dynamic part: the steps of rows [d0, n), cut into ng slices that each
     // have their own ticket counter.  A slice hands out chunks of DSTEPS
@@ -2112,7 +2118,7 @@ __device__ __forceinline__ void scan_topk_body(ScanArgs a) {
         return nb + (ls - nb * dsteps);
     };
     uint32_t gi = 0;
-    uint32_t sub = 0, ds = 0, dlen = 0, slice = (blockIdx.x * SH::WAVES + wave) % ng, pend = 0;
+    uint32_t sub = 0, ds = 0, dlen = 0, slice = (bx * SH::WAVES + wave) % ng, pend = 0;
     bool dynamic = false, has_pend = false;
     uint32_t c0 = 0, clim = 0;
     // takes the next dynamic ticket: its first row in c0 and end in clim;
@@ -2150,7 +2156,7 @@ __device__ __forceinline__ void scan_topk_body(ScanArgs a) {
     auto next_step = [&](uint32_t &base, uint32_t &lim) -> bool {
         if (!dynamic) {
             while (gi < sgrabs) {
-                const uint32_t r0 = (blockIdx.x + gi * a.grid) * SH::GRAB_ROWS;
+                const uint32_t r0 = (bx + gi * a.grid) * SH::GRAB_ROWS;
                 base = r0 + wofs + sub * wstep;
                 lim = r0 + SH::GRAB_ROWS < n ? r0 + SH::GRAB_ROWS : n;
                 if (++sub == (uint32_t)SH::GRAB_STEPS) {
@@ -2281,7 +2287,7 @@ __device__ __forceinline__ void scan_topk_body(ScanArgs a) {
         // the workgroup's first static grab is full: the wave's first two
         // steps are its two steps in that grab (next_step's state moves on
         // to the second grab)
-        const uint32_t r0 = blockIdx.x * SH::GRAB_ROWS;
+        const uint32_t r0 = bx * SH::GRAB_ROWS;
         ab = r0 + wofs;
         al = r0 + SH::GRAB_ROWS;
         bb = ab + wstep;
@@ -2394,7 +2400,7 @@ __device__ __forceinline__ void scan_topk_body(ScanArgs a) {
     // the grid are still scanning.  The slot reservation is issued first and
     // read only when the pairs are stored, so its round trip overlaps the
     // re-rank's row loads.
-    const uint32_t grp = blockIdx.x % ng;
+    const uint32_t grp = bx % ng;
     const uint64_t region = a.cand_cap / ng;  // pairs per group region
     if (wc) {
         uint32_t b0 = 0;
