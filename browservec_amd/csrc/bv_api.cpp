@@ -173,6 +173,7 @@ struct bv_index {
     uint64_t pm_rows = 0;                      // rows expanded into pm_codes
     DevBuf ivb_base, ivb_pcount, ivb_poff, ivb_fill, ivb_pq, ivb_pbase, ivb_tmp;  // list-major IVF batches
     DevBuf ivb_chunks, ivb_choff;             // list-major IVF batches: work items per list, their offsets
+    DevBuf sl_ord, sl_best, sl_part, sl_top;  // slot scans: order words, slots' best keys, parts' order words, 1-bit upper bounds
     DevBuf sel_list, sel_popc, sel_off, sel_misc;  // listed rows; mask word counts and offsets; flag + count
     HostBuf h_cnt;
     HostBuf h_rows, h_scores, h_n, h_flag;
@@ -1323,6 +1324,28 @@ static int lanes_mark(bv_index *idx) {
     return BV_OK;
 }
 
+// Rotated queries (qrot) and their layout for codec `layout` (qscan).
+static int prepare_layout(bv_index *idx, const float *d_q, uint32_t nq, int layout, const void **qscan,
+                          uint64_t *qstride) {
+    const uint32_t P = idx->P;
+    const size_t st = level_stride(layout, P);
+    HIPX(idx->dev, idx->qrot.ensure((size_t)nq * P * 4, 0, idx->stream), "query buffer");
+    HIPX(idx->dev, idx->qscan.ensure((size_t)nq * st, 0, idx->stream), "query buffer");
+    PrepArgs a{};
+    a.q = d_q;
+    a.dim = idx->dim;
+    a.P = P;
+    a.signs = idx->signs.as<float>();
+    a.rounds = idx->d.rounds;
+    a.qrot = idx->qrot.as<float>();
+    a.out = idx->qscan.as<unsigned char>();
+    a.stride = st;
+    HIPX(idx->dev, launch_query_prep(layout, a, nq, idx->stream), "query transform kernel");
+    *qscan = idx->qscan.p;
+    *qstride = st;
+    return BV_OK;
+}
+
 // Query transform for the scan: device-resident queries d_q (nq x dim) ->
 // qscan (per-codec layout), and for quantized kinds qrot (nq x P).
 static int prepare_queries(bv_index *idx, const float *d_q, uint32_t nq, const void **qscan, uint64_t *qstride) {
@@ -1343,40 +1366,12 @@ static int prepare_queries(bv_index *idx, const float *d_q, uint32_t nq, const v
     a.rotated = idx->qrot.as<float>();
     switch (idx->codec) {
     case C_Q8:
-    case C_Q4: {
-        const size_t st = level_stride(idx->codec, P);
-        HIPX(idx->dev, idx->qscan.ensure((size_t)nq * st, 0, idx->stream), "query buffer");
-        HIPX(idx->dev, launch_encode(a, idx->stream), "query rotate kernel");
-        LevelArgs la{};
-        la.qrot = idx->qrot.as<float>();
-        la.P = P;
-        la.codec = idx->codec;
-        la.out = idx->qscan.as<unsigned char>();
-        la.stride = st;
-        HIPX(idx->dev, launch_levels(la, nq, idx->stream), "query levels kernel");
-        *qscan = idx->qscan.p;
-        *qstride = st;
-        return BV_OK;
-    }
+    case C_Q4:
+    case C_Q1P: return prepare_layout(idx, d_q, nq, idx->codec, qscan, qstride);
     case C_Q1A:
         *qscan = idx->qrot.p;
         *qstride = (uint64_t)P * 4;
         break;
-    case C_Q1P: {
-        const size_t st = level_stride(C_Q1P, P);
-        HIPX(idx->dev, idx->qscan.ensure((size_t)nq * st, 0, idx->stream), "query buffer");
-        HIPX(idx->dev, launch_encode(a, idx->stream), "query rotate kernel");
-        LevelArgs la{};
-        la.qrot = idx->qrot.as<float>();
-        la.P = P;
-        la.codec = C_Q1P;
-        la.out = idx->qscan.as<unsigned char>();
-        la.stride = st;
-        HIPX(idx->dev, launch_q1p_layout(la, nq, idx->stream), "query bit-plane kernel");
-        *qscan = idx->qscan.p;
-        *qstride = st;
-        return BV_OK;
-    }
     case C_HAM:
     case C_I8S: {
         const uint32_t per = idx->codec == C_HAM ? 32 : 4;
@@ -1530,7 +1525,7 @@ static int run_fused(bv_index *idx, const float *d_q, uint32_t nq, uint32_t kpri
 // Keys are the single-query scan's keys, so results equal the same queries
 // run one at a time.  A query whose appended keys overflow their buffer (a
 // bound left loose by the sample) is re-run through the fused scan.
-constexpr uint32_t MQ_MIN_Q = 8;  // smallest batch for the matrix-core path
+constexpr uint32_t MQ_MIN_Q = 8;  // smallest batch for the matrix-core path (it waits once; fewer queries never do)
 
 static bool mq_eligible(const bv_index *idx, uint32_t nq, const uint32_t *d_mask) {
     if (idx->ivf || d_mask || nq < MQ_MIN_Q || idx->rows == 0) return false;
@@ -1551,30 +1546,11 @@ static bool mq_eligible(const bv_index *idx, uint32_t nq, const uint32_t *d_mask
 // the batched scan reads (int4 indexes: levels without the 1/127 scale).
 static int prepare_levels16(bv_index *idx, const float *d_q, uint32_t nq, const unsigned char **qlev,
                             uint64_t *qstride, int layout = -1) {
-    const uint32_t P = idx->P;
     if (layout < 0) layout = idx->codec == C_Q4 ? C_Q4M : C_Q8;
-    const size_t st = level_stride(layout, P);
-    HIPX(idx->dev, idx->qrot.ensure((size_t)nq * P * 4, 0, idx->stream), "query buffer");
-    HIPX(idx->dev, idx->qscan.ensure((size_t)nq * st, 0, idx->stream), "query buffer");
-    EncodeArgs e{};
-    e.src = d_q;
-    e.rows = nq;
-    e.dim = idx->dim;
-    e.P = P;
-    e.signs = idx->signs.as<float>();
-    e.rounds = idx->d.rounds;
-    e.rotated = idx->qrot.as<float>();
-    HIPX(idx->dev, launch_encode(e, idx->stream), "query rotate kernel");
-    LevelArgs la{};
-    la.qrot = idx->qrot.as<float>();
-    la.P = P;
-    la.codec = layout;
-    la.out = idx->qscan.as<unsigned char>();
-    la.stride = st;
-    HIPX(idx->dev, launch_levels(la, nq, idx->stream), "query levels kernel");
-    *qlev = idx->qscan.as<unsigned char>();
-    *qstride = st;
-    return BV_OK;
+    const void *q = nullptr;
+    const int rc = prepare_layout(idx, d_q, nq, layout, &q, qstride);
+    *qlev = (const unsigned char *)q;
+    return rc;
 }
 
 // Workgroups per (XCD, query block) of the persistent batched scan: about
@@ -2361,6 +2337,116 @@ static int run_ivf_batched(bv_index *idx, const float *d_q, uint32_t nq, uint32_
     return BV_OK;
 }
 
+// ------------------------------------------------------------- slot scans
+// Small batches and short scans: scan_slots (the rows read once for up to
+// four queries) and pick_topk (one workgroup per query).
+// Which calls take them.  Measured on one MI355X, us a call alone (slot scan
+// against the other path):
+//   against one fused scan per query (2 to 7 queries, or no batch path):
+//     every size and codec, 1M x 768 int8 4 queries 286 / 702, 1-bit 219 /
+//     8,234, 100,000 x 384 int4 fetch 160 one query 57 / 1,108, 100,000 x 300
+//     fp32 256 queries 1,660 / 8,360;
+//   single queries likewise, but for the int8 scan from half a GB on, which
+//     the fused scan's one launch serves in 192 us against 212 (1M x 768;
+//     500,000 rows: 132 / 130);
+//   against the batched passes: those cost about 140 us of launches and
+//     0.24 us per million codes whatever the batch, a slot scan 45 us and a
+//     time per query, row and 16-byte unit set by its dot products (below):
+//     1M x 768 int8 crosses between 4 and 5 queries, 100,000 x 384 at 40,
+//     20,000 x 300 at 140.
+static bool slots_route(const bv_index *idx, uint32_t nq, uint32_t kprime, bool rerank, bool batchable) {
+    if (idx->ivf || idx->rows == 0 || idx->rows >= (1ull << 30)) return false;
+    if (!pick_supported(idx->codec, idx->P, rerank ? idx->dim : 0)) return false;
+    if (nq == 1) return !(idx->codec == C_Q8 && idx->rows * idx->row_bytes >= (512ull << 20) && kprime <= 256);
+    if (!batchable) return true;
+    double per;  // us per million (row, unit)
+    switch (idx->codec) {
+    case C_Q8: per = 0.95; break;
+    case C_Q4: per = 1.4; break;
+    case C_Q1P: per = 3.6; break;
+    case C_Q1A: per = 2.0; break;
+    case C_HAM: per = 1.0; break;
+    case C_I8S: per = 0.5; break;
+    case C_F32DOT_S:
+    case C_F32L2_S: per = 0.18; break;
+    default: per = 0.7; break;
+    }
+    const double mrows = (double)idx->rows * 1e-6;
+    const double slots = 45.0 + (double)nq * mrows * idx->units * per;
+    const double batch = idx->quant ? 140.0 + 0.24 * mrows * idx->P
+                                    : 120.0 + 0.82 * mrows * idx->dim * std::max(1.0, (double)nq / 48.0);
+    return slots < batch;
+}
+
+static int run_slots(bv_index *idx, const float *d_q, uint32_t nq, uint32_t kprime, uint32_t k_out, bool rerank,
+                     const uint32_t *d_mask, uint64_t mask_bits, uint32_t *d_rows, float *d_scores, uint32_t *d_n) {
+    hipStream_t s = idx->stream;
+    const void *qscan = nullptr;
+    uint64_t qstride = 0;
+    int rc = prepare_queries(idx, d_q, nq, &qscan, &qstride);
+    if (rc) return rc;
+    // rows per slot: two wave steps at least (one where the fetch is large
+    // next to the slots: their best keys then still give a bound), and so
+    // many that the slots fit half of what pick_topk holds
+    const uint32_t step = scan_step_rows(idx->units);
+    uint32_t rw = 2 * step;
+    if (idx->rows / rw < 2ull * kprime) rw = step;
+    while ((idx->rows + rw - 1) / rw > SLOTS_MAX / 2) rw *= 2;
+    const uint32_t nslots = (uint32_t)((idx->rows + rw - 1) / rw);
+    uint32_t nsub = 1;
+    while (nsub < 8 && rw / (nsub * 2) >= 2 * step) nsub *= 2;
+    const uint64_t per = (uint64_t)nslots * rw;
+    const uint32_t chunk = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(nq, (256ull << 20) / (per * 4)));
+    HIPX(idx->dev, idx->sl_ord.ensure((size_t)chunk * per * 4, 0, s), "scratch");
+    HIPX(idx->dev, idx->sl_best.ensure((size_t)chunk * nslots * 8, 0, s), "scratch");
+    HIPX(idx->dev, idx->sl_part.ensure((size_t)chunk * nslots * nsub * 4, 0, s), "scratch");
+    const bool q1p = idx->codec == C_Q1P;
+    if (q1p) HIPX(idx->dev, idx->sl_top.ensure((size_t)chunk * nslots * 4, 0, s), "scratch");
+    PickArgs p{};
+    SlotArgs &a = p.s;
+    a.codes = idx->quant ? idx->codes.p : idx->raw.p;
+    a.row_bytes = idx->row_bytes;
+    a.units = idx->units;
+    a.padded_dim = idx->P;
+    a.scales = (idx->codec == C_Q8 || idx->codec == C_Q4 || idx->codec == C_Q1A || q1p) ? idx->scales.as<float>() : nullptr;
+    a.scale_mul = idx->codec == C_Q4 ? 1.0f / 7.0f : 1.0f;
+    a.q_stride = qstride;
+    a.mask = d_mask;
+    a.mask_bits = mask_bits;
+    a.n = (uint32_t)idx->rows;
+    a.rw = rw;
+    a.nsub = nsub;
+    a.part = idx->sl_part.as<uint32_t>();
+    a.nslots = nslots;
+    a.ord = idx->sl_ord.as<uint32_t>();
+    a.best = idx->sl_best.as<uint64_t>();
+    a.top = q1p ? idx->sl_top.as<uint32_t>() : nullptr;
+    p.q1p = q1p;
+    p.is_int = idx->codec == C_HAM || idx->codec == C_I8S;
+    p.kk = kprime;
+    p.k_out = k_out;
+    timing_begin(idx);
+    for (uint32_t q0 = 0; q0 < nq; q0 += chunk) {
+        a.nq = std::min(chunk, nq - q0);
+        a.q = (const char *)qscan + (uint64_t)q0 * qstride;
+        p.qrot = q1p ? idx->qrot.as<float>() + (size_t)q0 * idx->P : nullptr;
+        if (rerank) {
+            p.rr_src = idx->raw.as<float>();
+            p.rr_dim = idx->dim;
+            p.rr_q = d_q + (size_t)q0 * idx->dim;
+            p.rr_q_stride = idx->dim;
+        }
+        p.out_rows = d_rows + (size_t)q0 * k_out;
+        p.out_scores = d_scores + (size_t)q0 * k_out;
+        p.out_n = d_n + q0;
+        HIPX(idx->dev, launch_scan_slots(idx->codec, a, s), "slot scan kernel");
+        HIPX(idx->dev, launch_pick_topk(p, s), "selection kernel");
+    }
+    timing_end(idx);
+    idx->last_scanned = idx->rows * nq;
+    return BV_OK;
+}
+
 static int run_pipeline(bv_index *idx, const float *d_q, uint32_t nq, uint32_t kprime, uint32_t k_out, bool rerank,
                         const uint32_t *d_mask, uint64_t mask_bits, uint32_t *d_rows, float *d_scores,
                         uint32_t *d_n, bool may_alternate = false) {
@@ -2368,6 +2454,14 @@ static int run_pipeline(bv_index *idx, const float *d_q, uint32_t nq, uint32_t k
         int rc = lanes_join(idx);
         if (rc) return rc;
         return run_ivf_batched(idx, d_q, nq, kprime, k_out, rerank, d_rows, d_scores, d_n);
+    }
+    // (single queries kept in flight on several query streams stay with the
+    // fused scan, whose scratch each stream has)
+    const bool streams = may_alternate && idx->query_streams >= 2 && nq < MQ_MIN_Q;
+    if (!streams && slots_route(idx, nq, kprime, rerank, mq_eligible(idx, nq, d_mask))) {
+        int rc = lanes_join(idx);
+        if (rc) return rc;
+        return run_slots(idx, d_q, nq, kprime, k_out, rerank, d_mask, mask_bits, d_rows, d_scores, d_n);
     }
     if (mq_eligible(idx, nq, d_mask)) {
         int rc = lanes_join(idx);  // the batch path shares the index stream's scratch and outputs
@@ -2379,9 +2473,10 @@ static int run_pipeline(bv_index *idx, const float *d_q, uint32_t nq, uint32_t k
 
 // Queries per device call for query batches: the matrix-core path takes
 // large batches (its scratch is about 32 * kprime * N / MQ_SAMPLE bytes per
-// query); the fused scan's scratch is sized per query in flight.
+// query; run_slots bounds its own); the fused scan's scratch is sized per
+// query in flight.
 static uint32_t batch_chunk(const bv_index *idx, uint32_t nq) {
-    return mq_eligible(idx, nq, nullptr) ? 1024u : 64u;
+    return mq_eligible(idx, nq, nullptr) || (nq > 1 && slots_route(idx, nq, 1, idx->quant, false)) ? 1024u : 64u;
 }
 
 // Host entry: upload queries (+mask), run, download.

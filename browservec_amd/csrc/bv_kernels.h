@@ -117,6 +117,57 @@ struct ScanArgs {
     uint32_t lean;            // 1: the register-lean build of the int8 transform scan (two queries in flight)
 };
 
+// The scan of short scans and small query batches (bv_slots.h): every row's
+// order word and every slot's best key, for pick_topk.
+constexpr uint32_t SLOTS_MAX = 16384;  // slots per query (pick_topk holds their best keys in registers)
+struct SlotArgs {
+    const void *codes;        // row-major rows, row_bytes each
+    uint64_t row_bytes;
+    uint32_t units, padded_dim;
+    const float *scales;      // per-row scale or null
+    float scale_mul;
+    const void *q;            // prepared queries, q_stride bytes apart
+    uint64_t q_stride;
+    const uint32_t *cand;     // indexed: query q scores rows cand[cand_off[q], cand_off[q + 1])
+    const uint64_t *cand_off;
+    const uint32_t *mask;     // row filter bits or null
+    uint64_t mask_bits;
+    uint32_t n;               // rows (indexed: the most candidates of a query)
+    uint32_t nq;
+    uint32_t rw;              // rows per slot: a power of two, whole wave steps
+    uint32_t nsub;            // parts per slot: a power of two; more than one: parts of whole step pairs
+    uint32_t nslots;          // nslots * rw >= n
+    uint32_t *ord;            // [nq][nslots * rw] order words (0: left out by the mask; C_Q1P: of an upper bound)
+    uint64_t *best;           // [nq][nslots] best keys (0: no row; C_Q1P: of lower bounds)
+    uint32_t *part;           // [nq][nslots * nsub] largest order word of each part
+    uint32_t *top;            // C_Q1P: [nq][nslots] largest order words
+};
+// Rows per wave step of the scan layout for rows of `units` units.
+uint32_t scan_step_rows(uint32_t units);
+hipError_t launch_scan_slots(int codec, const SlotArgs &a, hipStream_t s);
+
+// Per query: the kk best keys of a scan_slots pass, then (rr_src set) their
+// exact re-rank, and the best k_out into the outputs.
+struct PickArgs {
+    SlotArgs s;               // the pass (C_Q1P: codes, scales and row layout for the exact keys too)
+    bool q1p;
+    const float *qrot;        // C_Q1P: rotated fp32 queries, nq x padded_dim
+    bool is_int;              // integer scores
+    uint32_t kk;              // 1 .. MAX_KPRIME
+    const float *rr_src;      // stored fp32 rows (N x rr_dim), or null: no re-rank
+    uint32_t rr_dim;
+    const float *rr_q;        // fp32 queries, rr_q_stride floats apart
+    uint64_t rr_q_stride;
+    uint32_t k_out;
+    uint32_t *out_rows;       // [nq][k_out]
+    float *out_scores;
+    uint32_t *out_n;
+};
+// Whether pick_topk serves the codec at this padded dimension (C_Q1P: its
+// exact keys need the 4- and 8-lane layouts).
+bool pick_supported(int codec, uint32_t P, uint32_t rr_dim);
+hipError_t launch_pick_topk(const PickArgs &a, hipStream_t s);
+
 // Exact keys of listed rows of a 1-bit asymmetric (C_Q1P) index, one grid
 // row per query (q1p_exact_rows).
 struct Q1pRowsArgs {
@@ -466,6 +517,18 @@ hipError_t launch_zero(void *p, size_t bytes, hipStream_t s);
 bool scan_supported(int codec, uint32_t units);
 hipError_t launch_scan(int codec, uint32_t units, const ScanArgs &a, uint32_t nq, hipStream_t s);
 hipError_t launch_encode(const EncodeArgs &a, hipStream_t s);
+// The rotated queries (nq x P) and their layout for codec C_Q8, C_Q4, C_Q4M or
+// C_Q1P, level_stride(codec, P) bytes or more apart.
+struct PrepArgs {
+    const float *q;           // nq x dim fp32 queries
+    uint32_t dim, P;
+    const float *signs;       // rounds x P
+    uint32_t rounds;
+    float *qrot;
+    unsigned char *out;
+    uint64_t stride;
+};
+hipError_t launch_query_prep(int codec, const PrepArgs &a, uint32_t nq, hipStream_t s);
 hipError_t launch_rerank(const RerankArgs &a, uint32_t nq, hipStream_t s);
 hipError_t launch_levels(const LevelArgs &a, uint32_t nq, hipStream_t s);
 // C_Q1P query layout (bit planes + Q1Tail + fp32 query) from rotated queries.

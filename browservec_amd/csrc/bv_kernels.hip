@@ -7,6 +7,36 @@
 namespace bvk {
 namespace {
 
+// ------------------------------------------------------- query transform --
+// A query's rotation and its codec layout (int8 / int4 levels, 1-bit planes)
+// in one launch, one workgroup of four waves per query, by the code the fused
+// scan runs in its own workgroups: 4-5 us where the row encoder and then the
+// level split (one wave each) took 9-12 (P = 1024).
+template <int C, int EP> __global__ __launch_bounds__(SCAN_WG) void query_prep(PrepArgs a) {
+    extern __shared__ __align__(16) unsigned char prep_lds[];
+    const int tid = threadIdx.x;
+    const uint32_t P = 256 * EP, q = blockIdx.x;
+    ScanArgs sa{};
+    sa.padded_dim = P;
+    sa.qdim = a.dim;
+    sa.rounds = a.rounds;
+    sa.signs = a.signs;
+    RotInWG<EP> in;
+    rotate_load_wg<EP>(a.q + (uint64_t)q * a.dim, a.dim, P, a.signs, a.rounds, in, tid);
+    prep_query_wg<C, EP, false>(sa, in, prep_lds, tid);
+    __syncthreads();
+    const size_t lay = query_layout_bytes(C, P);
+    const float *xs = (const float *)(prep_lds + prep_wg_xs_offset(lay));  // the rotated query
+    for (uint32_t i = (uint32_t)tid; i < P; i += SCAN_WG) {
+        const float v = xs[i];
+        a.qrot[(uint64_t)q * P + i] = v;
+        if (C == C_Q1P) ((float *)(a.out + (uint64_t)q * a.stride + q1p_f_off(P)))[i] = v;
+    }
+    const uint32_t words = (uint32_t)((C == C_Q1P ? q1p_f_off(P) : lay) / 4);
+    for (uint32_t i = (uint32_t)tid; i < words; i += SCAN_WG)
+        ((uint32_t *)(a.out + (uint64_t)q * a.stride))[i] = ((const uint32_t *)prep_lds)[i];
+}
+
 // ---------------------------------------------------------------- rerank --
 // Re-rank of an explicit candidate list: one wave per candidate computes
 // Store.dotRow exactly (exact_key_wave); the last wave of each query ranks
@@ -116,6 +146,39 @@ hipError_t launch_scan(int codec, uint32_t units, const ScanArgs &a, uint32_t nq
     }
 }
 
+uint32_t scan_step_rows(uint32_t units) {
+    Layout L;
+    if (!pick_layout(units, L)) return 0;
+    // (ScanShape::RPS; the codec does not enter)
+    switch (L.lpr) {
+    case 4: return ScanShape<C_Q8, 4, 1>::RPS;
+    case 8: return ScanShape<C_Q8, 8, 1>::RPS;
+    case 16: return ScanShape<C_Q8, 16, 1>::RPS;
+    case 32: return ScanShape<C_Q8, 32, 1>::RPS;
+    default:
+        return L.upl >= 4 ? ScanShape<C_Q8, 64, 4>::RPS : L.upl >= 2 ? ScanShape<C_Q8, 64, 2>::RPS
+                                                                     : ScanShape<C_Q8, 64, 1>::RPS;
+    }
+}
+
+hipError_t launch_scan_slots(int codec, const SlotArgs &a, hipStream_t s) {
+    Layout L;
+    if (!pick_layout(a.units, L) || !scan_supported(codec, a.units)) return hipErrorInvalidValue;
+    switch (codec) {
+    case C_F32DOT: return slots_codec_f32dot(L.lpr, L.upl, a, s);
+    case C_F32L2: return slots_codec_f32l2(L.lpr, L.upl, a, s);
+    case C_Q8: return slots_codec_q8(L.lpr, L.upl, a, s);
+    case C_Q4: return slots_codec_q4(L.lpr, L.upl, a, s);
+    case C_Q1A: return slots_codec_q1a(L.lpr, L.upl, a, s);
+    case C_Q1P: return slots_codec_q1p(L.lpr, L.upl, a, s);
+    case C_HAM: return slots_codec_ham(L.lpr, L.upl, a, s);
+    case C_I8S: return slots_codec_i8s(L.lpr, L.upl, a, s);
+    case C_F32DOT_S: return slots_codec_f32dot_s(L.lpr, L.upl, a, s);
+    case C_F32L2_S: return slots_codec_f32l2_s(L.lpr, L.upl, a, s);
+    default: return hipErrorInvalidValue;
+    }
+}
+
 hipError_t launch_encode(const EncodeArgs &a, hipStream_t s) {
     if (a.rows == 0) return hipSuccess;
     const uint32_t E = a.P >= 64 ? a.P / 64 : 1;
@@ -151,6 +214,48 @@ hipError_t launch_levels(const LevelArgs &a, uint32_t nq, hipStream_t s) {
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
+}
+
+template <int C> static hipError_t prep_go(const PrepArgs &a, uint32_t nq, hipStream_t s) {
+    const size_t lds = (query_prep_lds(C == C_Q4M ? C_Q8 : C, a.P) + 15) & ~(size_t)15;
+    switch (a.P) {
+    case 256: hipLaunchKernelGGL((query_prep<C, 1>), dim3(nq), dim3(SCAN_WG), lds, s, a); break;
+    case 512: hipLaunchKernelGGL((query_prep<C, 2>), dim3(nq), dim3(SCAN_WG), lds, s, a); break;
+    case 1024: hipLaunchKernelGGL((query_prep<C, 4>), dim3(nq), dim3(SCAN_WG), lds, s, a); break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+hipError_t launch_query_prep(int codec, const PrepArgs &a, uint32_t nq, hipStream_t s) {
+    if (nq == 0) return hipSuccess;
+    // the workgroup-wide transform's sizes; other ones take the row encoder
+    // and the level split
+    if (a.P == 256 || a.P == 512 || a.P == 1024) {
+        switch (codec) {
+        case C_Q8: return prep_go<C_Q8>(a, nq, s);
+        case C_Q4: return prep_go<C_Q4>(a, nq, s);
+        case C_Q4M: return prep_go<C_Q4M>(a, nq, s);
+        case C_Q1P: return prep_go<C_Q1P>(a, nq, s);
+        default: return hipErrorInvalidValue;
+        }
+    }
+    EncodeArgs e{};
+    e.src = a.q;
+    e.rows = nq;
+    e.dim = a.dim;
+    e.P = a.P;
+    e.signs = a.signs;
+    e.rounds = a.rounds;
+    e.rotated = a.qrot;
+    hipError_t r = launch_encode(e, s);
+    if (r != hipSuccess) return r;
+    LevelArgs la{};
+    la.qrot = a.qrot;
+    la.P = a.P;
+    la.codec = codec;
+    la.out = a.out;
+    la.stride = a.stride;
+    return codec == C_Q1P ? launch_q1p_layout(la, nq, s) : launch_levels(la, nq, s);
 }
 
 size_t level_stride(int codec, uint32_t P) { return query_layout_bytes(codec, P); }

@@ -27,6 +27,8 @@
 #include "bv_kernels.h"
 #include "bv_device.h"
 #include "bv_mfma.h"
+#include "bv_exact.h"
+#include "bv_sort.h"
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -69,29 +71,6 @@ __device__ __forceinline__ float next_up(float x) {
     return __uint_as_float((b & 0x80000000u) ? b - 1 : b + 1);
 }
 __device__ __forceinline__ float next_down(float x) { return -next_up(-x); }
-
-// Descending bitonic sort of keys[0, npow) (npow a power of two), whole
-// workgroup.
-__device__ void sort_desc(uint64_t *keys, uint32_t npow) {
-    const uint32_t tid = threadIdx.x, nt = blockDim.x;
-    for (uint32_t k = 2; k <= npow; k <<= 1) {
-        for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-            for (uint32_t i = tid; i < npow; i += nt) {
-                const uint32_t ixj = i ^ j;
-                if (ixj > i) {
-                    const uint64_t x = keys[i], y = keys[ixj];
-                    const bool desc = (i & k) == 0;
-                    if (desc ? (x < y) : (x > y)) {
-                        keys[i] = y;
-                        keys[ixj] = x;
-                    }
-                }
-            }
-            __syncthreads();
-        }
-    }
-}
-
 
 // Per-query constants of the epilogue, in LDS: the level scales in f64
 // (exact keys) and in f32 with the level-3 bound (prefilter), and the bound
@@ -1415,7 +1394,8 @@ constexpr int SEL_CAP = 4096;
 constexpr int SEL_KPT = 16;  // keys per thread held in registers (lists up to 16,384 keys)
 
 __global__ __launch_bounds__(SEL_THREADS) void mq_select(MqSelArgs a) {
-    __shared__ uint32_t hist[SEL_BINS];
+    // (a pad word per 32 bins: the scan's lanes start 32 bins apart)
+    __shared__ uint32_t hist[SEL_BINS + SEL_BINS / 32];
     __shared__ uint64_t sel[SEL_CAP];
     __shared__ uint64_t red[2][SEL_THREADS / 64];
     __shared__ uint32_t s_bin, s_excl, s_cnt;
@@ -1458,6 +1438,7 @@ __global__ __launch_bounds__(SEL_THREADS) void mq_select(MqSelArgs a) {
             for (uint32_t i = tid; i < n; i += SEL_THREADS) f(keys[i]);
         }
     };
+    auto hbin = [](uint32_t b) { return b + (b >> 5); };
     uint32_t lim = 256;
     while (lim < 2 * kk && lim < (uint32_t)SEL_CAP) lim <<= 1;
     uint64_t G = 0;  // keys >= G are gathered
@@ -1489,16 +1470,16 @@ __global__ __launch_bounds__(SEL_THREADS) void mq_select(MqSelArgs a) {
         for (;;) {
             const uint64_t span = hi - lo;
             const int shift = (span >> 11) ? 64 - __clzll((long long)(span >> 11)) : 0;  // (span >> shift) < 2048
-            for (uint32_t i = tid; i < SEL_BINS; i += SEL_THREADS) hist[i] = 0;
+            for (uint32_t i = tid; i < SEL_BINS + SEL_BINS / 32; i += SEL_THREADS) hist[i] = 0;
             __syncthreads();
             each([&](uint64_t k) {
-                if (k >= lo && k <= hi) atomicAdd(&hist[(uint32_t)((k - lo) >> shift)], 1u);
+                if (k >= lo && k <= hi) atomicAdd(&hist[hbin((uint32_t)((k - lo) >> shift))], 1u);
             });
             __syncthreads();
             if (wave == 0) {
                 // lane l holds bins 2047 - 32l - j (j < 32): counts from the top
                 uint32_t loc = 0;
-                for (int j = 0; j < 32; ++j) loc += hist[SEL_BINS - 1 - (32 * lane + j)];
+                for (int j = 0; j < 32; ++j) loc += hist[hbin(SEL_BINS - 1 - (32 * lane + j))];
                 uint32_t inc = loc;
 #pragma unroll
                 for (int o = 1; o < 64; o <<= 1) {
@@ -1511,7 +1492,7 @@ __global__ __launch_bounds__(SEL_THREADS) void mq_select(MqSelArgs a) {
                     uint32_t acc = exc;
                     for (int j = 0; j < 32; ++j) {
                         const uint32_t bin = SEL_BINS - 1 - (32 * lane + j);
-                        const uint32_t cb = hist[bin];
+                        const uint32_t cb = hist[hbin(bin)];
                         if (acc + cb >= rem) {
                             s_bin = bin;
                             s_excl = acc;
@@ -1568,7 +1549,7 @@ __global__ __launch_bounds__(SEL_THREADS) void mq_select(MqSelArgs a) {
     while (npow < got) npow <<= 1;
     for (uint32_t i = got + tid; i < npow; i += SEL_THREADS) sel[i] = 0;
     __syncthreads();
-    sort_desc(sel, npow);
+    sort_desc_lds<SEL_THREADS>(sel, npow);
     const uint32_t m = got < kk ? got : kk;
     if (tid == 0) {
         if (a.tau) {
@@ -1591,56 +1572,25 @@ __global__ __launch_bounds__(SEL_THREADS) void mq_select(MqSelArgs a) {
 }
 
 // Exact re-rank of each query's selected candidates (Store.dotRow,
-// src/store/store.ts:114-130) and the final top-k_out, one workgroup per
-// query.  Lane 4c + m of a wave runs accumulator m of candidate c: the f64
-// sum over elements 4j + m in order (each f32 x f32 product is exact in f64,
-// so fma adds it with the reference's single rounding); lanes 4c .. 4c + 3
-// then combine as ((a0 + a1) + a2) + a3 and add the tail elements in order.
-// Sixteen candidates per wave run at once.
+// src/store/store.ts:114-130; bv_exact.h) and the final top-k_out, one
+// workgroup per query, sixteen candidates per wave at once.
 constexpr int RR_THREADS = 1024;
 __global__ __launch_bounds__(RR_THREADS) void mq_rerank(MqRerankArgs a) {
-    extern __shared__ float qv[];  // the query, dim floats
+    extern __shared__ __align__(16) float qv[];  // the transposed query
+    __shared__ __align__(16) float tiles[RR_THREADS / 64][EXACT_TILE];
     __shared__ uint64_t ek[MAX_KPRIME];
     const uint32_t q = blockIdx.x, tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
-    const uint32_t dim = a.dim, vec = dim & ~3u;
     const float *qs = a.q + (uint64_t)q * a.q_stride;
-    for (uint32_t i = tid; i < dim; i += RR_THREADS) qv[i] = qs[i];
+    exact_load_query(qs, a.dim, qv, tid, RR_THREADS);
     __syncthreads();
     const uint32_t m = a.merged_n[q];
     const uint64_t *mk = a.merged + (uint64_t)q * a.kprime;
-    const int ci = lane >> 2, ai = lane & 3;
     for (uint32_t c0 = (uint32_t)wave * 16; c0 < m; c0 += (RR_THREADS / 64) * 16) {
-        const uint32_t cand = c0 + ci;
-        const bool have = cand < m;
-        const uint32_t row = have ? key_row(mk[cand]) : 0u;
-        const float *x = a.rows + (uint64_t)row * dim;
-        double acc = 0.0;
-        uint32_t j = ai;
-        // 32 of the lane's elements loaded at once, then summed in order
-        for (; j + 124 < vec; j += 128) {
-            float xv[32];
-#pragma unroll
-            for (int u = 0; u < 32; ++u) xv[u] = x[j + 4 * u];
-#pragma unroll
-            for (int u = 0; u < 32; ++u) acc = fma((double)xv[u], (double)qv[j + 4 * u], acc);
-        }
-        for (; j + 28 < vec; j += 32) {
-            float xv[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) xv[u] = x[j + 4 * u];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) acc = fma((double)xv[u], (double)qv[j + 4 * u], acc);
-        }
-        for (; j < vec; j += 4) acc = fma((double)x[j], (double)qv[j], acc);
-        const double a1 = __shfl_down(acc, 1), a2 = __shfl_down(acc, 2), a3 = __shfl_down(acc, 3);
-        if (have && ai == 0) {
-            double sum = acc + a1;
-            sum = sum + a2;
-            sum = sum + a3;
-            for (uint32_t i = vec; i < dim; ++i) sum = fma((double)x[i], (double)qv[i], sum);
-            ek[cand] = make_key(ord_f32((float)sum), row);
-        }
+        const uint32_t cand = c0 + (uint32_t)(lane >> 2);
+        const uint32_t row = key_row(mk[cand < m ? cand : c0]);
+        const uint64_t k = exact_keys16(a.rows, a.dim, qs, qv, row, tiles[wave], lane);
+        if ((lane & 3) == 0 && cand < m) ek[cand] = k;
     }
     __syncthreads();
     // rank: key i goes to slot #{keys greater than it} (keys are unique)
@@ -2548,9 +2498,8 @@ hipError_t launch_mq_select(const MqSelArgs &a, uint32_t nq, hipStream_t s) {
 
 hipError_t launch_mq_rerank(const MqRerankArgs &a, uint32_t nq, hipStream_t s) {
     if (nq == 0) return hipSuccess;
-    if (a.kprime == 0 || a.kprime > (uint32_t)MAX_KPRIME || a.dim == 0 || (size_t)a.dim * 4 > 96 * 1024)
-        return hipErrorInvalidValue;
-    hipLaunchKernelGGL(mq_rerank, dim3(nq), dim3(RR_THREADS), (size_t)a.dim * 4, s, a);
+    if (a.kprime == 0 || a.kprime > (uint32_t)MAX_KPRIME || a.dim == 0 || a.dim > 4096) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(mq_rerank, dim3(nq), dim3(RR_THREADS), 16 * (size_t)exact_q_stride(a.dim), s, a);
     return hipGetLastError();
 }
 

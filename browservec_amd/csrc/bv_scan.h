@@ -744,6 +744,17 @@ __device__ __forceinline__ uint64_t wave_max_u64(uint64_t v) {
     return swap_max_u64<true>(v);
 }
 
+__device__ __forceinline__ uint32_t wave_max_u32_dpp(uint32_t v) {
+    v = max(v, dpp<DPP_XOR1>(v));
+    v = max(v, dpp<DPP_XOR2>(v));
+    v = max(v, dpp<DPP_HALF_MIRROR>(v));
+    v = max(v, dpp<DPP_MIRROR>(v));
+    const auto a = __builtin_amdgcn_permlane16_swap((int)v, (int)v, false, false);
+    v = max((uint32_t)a[0], (uint32_t)a[1]);
+    const auto b = __builtin_amdgcn_permlane32_swap((int)v, (int)v, false, false);
+    return max((uint32_t)b[0], (uint32_t)b[1]);
+}
+
 // wave_append for (key, companion) pairs stored at the same index.
 __device__ __forceinline__ void wave_append2(uint64_t *keys, uint64_t *comp, uint32_t *cnt, uint32_t cap, bool take,
                                              uint64_t key, uint64_t c, int lane) {
@@ -1373,7 +1384,8 @@ __device__ __forceinline__ void rotate_load_wg(const float *src, uint32_t dim, u
     }
 }
 
-template <int C, int EP>
+// (LUT: C_Q1P builds its re-score table too, at lds + a.qf_off)
+template <int C, int EP, bool LUT = true>
 __device__ __forceinline__ void prep_query_wg(const ScanArgs &a, RotInWG<EP> &in, unsigned char *lds, int tid) {
 #pragma clang fp contract(off)
     const uint32_t P = a.padded_dim;  // == 256 * EP
@@ -1462,7 +1474,7 @@ __device__ __forceinline__ void prep_query_wg(const ScanArgs &a, RotInWG<EP> &in
         }
         __syncthreads();
         q1p_planes(lv, P, (uint32_t *)lds, (uint32_t)tid, SCAN_WG);
-        q1p_lut_build(xs, P, (float *)(lds + a.qf_off), (uint32_t)tid, SCAN_WG);
+        if constexpr (LUT) q1p_lut_build(xs, P, (float *)(lds + a.qf_off), (uint32_t)tid, SCAN_WG);
         if (tid == 0) {
             Q1Tail *tl = (Q1Tail *)(lds + q1p_tail_off(P));
             tl->s1 = s1;
@@ -1509,7 +1521,7 @@ __device__ __forceinline__ void prep_query_wg(const ScanArgs &a, RotInWG<EP> &in
         uint32_t *w = (uint32_t *)lds;
         const unsigned char *lb = (const unsigned char *)lv;
         uint32_t qwords;
-        if constexpr (C == C_Q8) {
+        if constexpr (C == C_Q8 || C == C_Q4M) {
             const uint32_t units = P / 16;
             qwords = units * 12;
             for (uint32_t i = tid; i < qwords; i += SCAN_WG) {
@@ -2957,5 +2969,17 @@ hipError_t scan_codec_ham(int lpr, int upl, const ScanArgs &a, uint32_t nq, hipS
 hipError_t scan_codec_i8s(int lpr, int upl, const ScanArgs &a, uint32_t nq, hipStream_t s);
 hipError_t scan_codec_f32dot_s(int lpr, int upl, const ScanArgs &a, uint32_t nq, hipStream_t s);
 hipError_t scan_codec_f32l2_s(int lpr, int upl, const ScanArgs &a, uint32_t nq, hipStream_t s);
+
+// and of its two-kernel form (bv_slots.h)
+hipError_t slots_codec_f32dot(int lpr, int upl, const SlotArgs &a, hipStream_t s);
+hipError_t slots_codec_f32l2(int lpr, int upl, const SlotArgs &a, hipStream_t s);
+hipError_t slots_codec_q8(int lpr, int upl, const SlotArgs &a, hipStream_t s);
+hipError_t slots_codec_q4(int lpr, int upl, const SlotArgs &a, hipStream_t s);
+hipError_t slots_codec_q1a(int lpr, int upl, const SlotArgs &a, hipStream_t s);
+hipError_t slots_codec_q1p(int lpr, int upl, const SlotArgs &a, hipStream_t s);
+hipError_t slots_codec_ham(int lpr, int upl, const SlotArgs &a, hipStream_t s);
+hipError_t slots_codec_i8s(int lpr, int upl, const SlotArgs &a, hipStream_t s);
+hipError_t slots_codec_f32dot_s(int lpr, int upl, const SlotArgs &a, hipStream_t s);
+hipError_t slots_codec_f32l2_s(int lpr, int upl, const SlotArgs &a, hipStream_t s);
 
 }  // namespace bvk

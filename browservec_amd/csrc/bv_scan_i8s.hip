@@ -1,10 +1,13 @@
 // Fused scan instantiations for codec C_I8S (see bv_scan.h).
-#include "bv_scan.h"
+#include "bv_slots.h"
 
 namespace bvk {
 
 hipError_t scan_codec_i8s(int lpr, int upl, const ScanArgs &a, uint32_t nq, hipStream_t s) {
     return dispatch_layout<C_I8S>(Layout{lpr, upl}, a, nq, s);
+}
+hipError_t slots_codec_i8s(int lpr, int upl, const SlotArgs &a, hipStream_t s) {
+    return slots_layout<C_I8S>(Layout{lpr, upl}, a, s);
 }
 
 }  // namespace bvk
