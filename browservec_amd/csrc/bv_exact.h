@@ -1,8 +1,9 @@
-// Exact re-rank scores of sixteen rows per wave (Store.dotRow,
-// src/store/store.ts:114-130) with coalesced row reads.
+// Exact scores of sixteen rows per wave (Store.dotRow and, L2, Store.l2Row,
+// src/store/store.ts:114-160) with coalesced row reads.
 //
-// Lane 4c + m runs accumulator m of candidate c: the f64 sum of the exact
-// products of elements 4j + m in order.  Read straight from memory each lane
+// Lane 4c + m runs accumulator m of candidate c over elements 4j + m in order,
+// in f64 (dot: each product is exact, so fma adds it with the reference's one
+// rounding; l2: the difference, its square and the sum each rounded).  Read straight from memory each lane
 // would take one element in four (16 rows x 16 bytes per load instruction,
 // 192 instructions at 768 dimensions: the address unit, shared by a
 // workgroup's waves, bounds it); here a row's 64-element chunks come in as
@@ -45,8 +46,18 @@ struct __attribute__((packed, aligned(4))) f32x4_u {
 
 // The (score, row) key of candidate lane >> 2 in lanes 4c; every lane of the
 // wave calls it with its candidate's row (absent candidates: any valid row).
-// tile: the wave's EXACT_TILE floats.  Padded elements multiply 0 by 0: the
-// sums are unchanged.
+// tile: the wave's EXACT_TILE floats.  Padded elements are 0 on both sides:
+// the sums are unchanged.
+template <bool L2> __device__ __forceinline__ double exact_add(double acc, float x, float q) {
+    if constexpr (L2) {
+#pragma clang fp contract(off)
+        const double d = (double)x - (double)q;
+        return acc + d * d;
+    } else {
+        return fma((double)x, (double)q, acc);
+    }
+}
+template <bool L2 = false>
 __device__ __forceinline__ uint64_t exact_keys16(const float *rows, uint32_t dim, const float *q, const float *qt,
                                                  uint32_t row, float *tile, int lane) {
     const uint32_t vec = dim & ~3u, nch = (vec + 63) / 64, qst = exact_q_stride(dim);
@@ -95,10 +106,10 @@ __device__ __forceinline__ uint64_t exact_keys16(const float *rows, uint32_t dim
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
                     const float4 a = xr[t], b = qr[t];
-                    acc = fma((double)a.x, (double)b.x, acc);
-                    acc = fma((double)a.y, (double)b.y, acc);
-                    acc = fma((double)a.z, (double)b.z, acc);
-                    acc = fma((double)a.w, (double)b.w, acc);
+                    acc = exact_add<L2>(acc, a.x, b.x);
+                    acc = exact_add<L2>(acc, a.y, b.y);
+                    acc = exact_add<L2>(acc, a.z, b.z);
+                    acc = exact_add<L2>(acc, a.w, b.w);
                 }
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             }
@@ -109,8 +120,8 @@ __device__ __forceinline__ uint64_t exact_keys16(const float *rows, uint32_t dim
     sum = sum + a2;
     sum = sum + a3;
     if (m == 0)
-        for (uint32_t i = vec; i < dim; ++i) sum = fma((double)x[i], (double)q[i], sum);
-    return make_key(ord_f32((float)sum), row);
+        for (uint32_t i = vec; i < dim; ++i) sum = exact_add<L2>(sum, x[i], q[i]);
+    return make_key(ord_f32(L2 ? (float)(-sum) : (float)sum), row);
 }
 
 }  // namespace

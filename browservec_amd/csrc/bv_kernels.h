@@ -129,7 +129,7 @@ struct SlotArgs {
     const void *q;            // prepared queries, q_stride bytes apart
     uint64_t q_stride;
     const uint32_t *cand;     // indexed: query q scores rows cand[cand_off[q], cand_off[q + 1])
-    const uint64_t *cand_off;
+    const uint64_t *cand_off; // (pick_topk: null for one query's rows cand[0, n))
     const uint32_t *mask;     // row filter bits or null
     uint64_t mask_bits;
     uint32_t n;               // rows (indexed: the most candidates of a query)
@@ -163,6 +163,10 @@ struct PickArgs {
     float *out_scores;
     uint32_t *out_n;
 };
+// Store.dotRow / Store.l2Row of the rows cand[0, n) (a.codes the fp32 rows of
+// a.padded_dim floats; slots of a multiple of 16 rows, one part each) against
+// q, as scan_slots leaves its scores.  A row at or past nrows sets *bad.
+hipError_t launch_rows_exact(const SlotArgs &a, const float *q, uint64_t nrows, bool l2, uint32_t *bad, hipStream_t s);
 // Whether pick_topk serves the codec at this padded dimension (C_Q1P: its
 // exact keys need the 4- and 8-lane layouts).
 bool pick_supported(int codec, uint32_t P, uint32_t rr_dim);

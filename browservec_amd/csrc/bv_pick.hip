@@ -76,7 +76,7 @@ template <int LPR> __global__ __launch_bounds__(PICK_THREADS) void pick_topk(Pic
     const uint32_t *ord = a.s.ord + (uint64_t)q * nslots * a.s.rw;
     const uint32_t *cand = a.s.cand;
     uint32_t n = a.s.n;
-    if (cand) {
+    if (cand && a.s.cand_off) {
         cand += a.s.cand_off[q];
         n = (uint32_t)(a.s.cand_off[q + 1] - a.s.cand_off[q]);
     }
@@ -330,7 +330,53 @@ template <int LPR> __global__ __launch_bounds__(PICK_THREADS) void pick_topk(Pic
     if (tid == 0) a.out_n[q] = ko;
 }
 
+// The exact score of each listed row (bv_exact.h) in scan_slots' form: one
+// wave per sixteen rows, a slot of a.rw / 16 of its passes.  A listed row at
+// or past nrows scores nothing and sets *bad.  Bound by the latency of one
+// wave's row reads and its f64 chain (a quarter of the dimension) for lists
+// of a few thousand rows, by HBM from about 50,000 (dim * 4 bytes each).
+constexpr uint32_t ROWS_WAVES = 4;
+template <bool L2>
+__global__ __launch_bounds__(ROWS_WAVES * 64) void rows_exact(SlotArgs a, const float *q, uint64_t nrows,
+                                                             uint32_t *bad) {
+    extern __shared__ __align__(16) float rows_smem[];  // the transposed query
+    __shared__ __align__(16) float tiles[ROWS_WAVES][EXACT_TILE];
+    const uint32_t dim = a.padded_dim;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    exact_load_query(q, dim, rows_smem, threadIdx.x, ROWS_WAVES * 64);
+    __syncthreads();
+    const uint32_t slot = blockIdx.x * ROWS_WAVES + (uint32_t)wave;
+    if (slot >= a.nslots) return;
+    uint64_t best = 0;
+    for (uint32_t r0 = slot * a.rw; r0 < (slot + 1) * a.rw && r0 < a.n; r0 += 16) {
+        const uint32_t i = r0 + (uint32_t)(lane >> 2);
+        const uint32_t row = a.cand[i < a.n ? i : r0];
+        const bool ok = row < nrows;
+        const uint64_t key =
+            exact_keys16<L2>((const float *)a.codes, dim, q, rows_smem, ok ? row : 0u, tiles[wave], lane);
+        if ((lane & 3) == 0 && i < a.n) {
+            const uint32_t w = (uint32_t)(key >> 32);
+            a.ord[i] = ok ? (w ? w : 1u) : 0u;
+            if (ok) best = key > best ? key : best;
+            else *bad = 1u;
+        }
+    }
+    best = wave_max_u64(best);
+    if (lane == 0) a.best[slot] = best;
+}
+
 }  // namespace
+
+hipError_t launch_rows_exact(const SlotArgs &a, const float *q, uint64_t nrows, bool l2, uint32_t *bad, hipStream_t s) {
+    const size_t lds = 16 * (size_t)exact_q_stride(a.padded_dim);
+    if (a.n == 0 || nrows == 0 || a.nq != 1 || a.nsub != 1 || a.rw < 16 || a.rw % 16 || !a.cand ||
+        (uint64_t)a.nslots * a.rw < a.n || lds + ROWS_WAVES * EXACT_TILE * 4 > 160 * 1024)
+        return hipErrorInvalidValue;
+    const dim3 g((a.nslots + ROWS_WAVES - 1) / ROWS_WAVES), wg(ROWS_WAVES * 64);
+    if (l2) hipLaunchKernelGGL(rows_exact<true>, g, wg, lds, s, a, q, nrows, bad);
+    else hipLaunchKernelGGL(rows_exact<false>, g, wg, lds, s, a, q, nrows, bad);
+    return hipGetLastError();
+}
 
 bool pick_supported(int codec, uint32_t P, uint32_t rr_dim) {
     return (codec != C_Q1P || (P >= 128 && P <= 1024)) && rr_dim <= 4096;

@@ -117,3 +117,30 @@ def test_slots_masked(ctx, kind, n, keep):
     assert [h.row for h in hits] == order.tolist()
     assert np.array_equal(np.array([h.score for h in hits], np.float32).view(np.uint32), scores[order].view(np.uint32))
     idx.destroy()
+
+
+@pytest.mark.parametrize("metric,dim,n_list,k", [("cosine", 768, 1, 1), ("l2", 300, 15, 10), ("dot", 37, 17, 17),
+                                                 ("cosine", 3, 200, 100), ("l2", 1001, 4097, 1000),
+                                                 ("cosine", 96, 140_000, 20)])
+def test_listed_rows_equal_dot_row(ctx, metric, dim, n_list, k):
+    """Listed rows (a duplicate among them) score Store.dotRow / l2Row bit for
+    bit and come back in canonical order."""
+    from browservec_amd import FlatIndex
+    from oracle import oracle as o
+
+    say("listed rows", metric, dim, n_list, k)
+    rng = np.random.default_rng(dim)
+    n = max(n_list + 5, 50)
+    x = rng.standard_normal((n, dim)).astype(np.float32)
+    idx = FlatIndex(ctx, dim, metric)
+    idx.append(x, n)
+    lst = rng.permutation(n)[:n_list].astype(np.uint32)
+    if n_list > 2:
+        lst[-1] = lst[0]
+    q = rng.standard_normal(dim).astype(np.float32)
+    hits = idx.query_rows(q, lst, k)
+    s = np.array([o.l2_row(x[r], q) if metric == "l2" else o.dot_row(x[r], q) for r in lst], np.float64).astype(np.float32)
+    order = np.lexsort((lst, -s.astype(np.float64)))[:k]
+    assert [h.row for h in hits] == lst[order].tolist()
+    assert np.array_equal(np.array([h.score for h in hits], np.float32).view(np.uint32), s[order].view(np.uint32))
+    idx.destroy()
