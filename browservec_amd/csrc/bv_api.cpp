@@ -134,6 +134,51 @@ struct HostBuf {
     }
 };
 
+// The inputs and results of a host call.  Inputs are gathered in one pinned
+// buffer and brought to the device by one small kernel; the last kernels of
+// the call write their results to pinned memory (coherent, so they are in
+// place when the stream is).  A pageable copy each way cost 8-12 us a piece:
+// 3,000 listed rows took 116 us a call, 36 of them kernels.  The buffers are
+// free again when the call has waited for its stream.
+struct PinnedBuf {
+    void *p = nullptr;
+    size_t cap = 0;
+    ~PinnedBuf() {
+        if (p) (void)hipHostFree(p);
+    }
+    hipError_t ensure(size_t bytes) {
+        if (bytes <= cap) return hipSuccess;
+        if (p) (void)hipHostFree(p);
+        p = nullptr;
+        const size_t ncap = std::max<size_t>(std::max(bytes, cap * 2), 4096);
+        cap = 0;
+        const hipError_t e = hipHostMalloc(&p, ncap, hipHostMallocMapped | hipHostMallocCoherent);
+        if (e == hipSuccess) cap = ncap;
+        else p = nullptr;
+        return e;
+    }
+};
+struct HostIo {
+    PinnedBuf in, out;
+    DevBuf dev;
+    size_t used = 0;
+    static size_t pad(size_t bytes) { return (bytes + 255) & ~size_t(255); }
+    // room for a call's inputs: the padded sizes' sum
+    hipError_t begin(size_t bytes, hipStream_t s) {
+        used = 0;
+        const hipError_t e = in.ensure(bytes);
+        return e == hipSuccess ? dev.ensure(bytes, 0, s) : e;
+    }
+    // the input's place on the device, valid after send()
+    void *put(const void *src, size_t bytes) {
+        std::memcpy((char *)in.p + used, src, bytes);
+        void *d = (char *)dev.p + used;
+        used += pad(bytes);
+        return d;
+    }
+    hipError_t send(hipStream_t s) { return launch_copy_in(dev.p, in.p, used, s); }
+};
+
 // ------------------------------------------------------------------ index
 // query streams a caller may keep single queries in flight on
 // (bv_index_set_query_streams)
@@ -176,7 +221,8 @@ struct bv_index {
     DevBuf sl_ord, sl_best, sl_part, sl_top;  // slot scans: order words, slots' best keys, parts' order words, 1-bit upper bounds
     DevBuf sel_list, sel_popc, sel_off, sel_misc;  // listed rows; mask word counts and offsets; flag + count
     HostBuf h_cnt;
-    HostBuf h_rows, h_scores, h_n, h_flag;
+    HostBuf h_flag;
+    HostIo io;                                // inputs and results of host calls
     // host appends: rows staged through two pinned buffers on a copy stream
     hipStream_t copy_stream = nullptr;
     hipEvent_t up_ev[2] = {nullptr, nullptr};
@@ -405,8 +451,9 @@ extern "C" int bv_index_create(bv_device *dev, const bv_index_desc *desc, bv_ind
     }
     hipError_t e = hipSetDevice(dev->ordinal);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&x->stream, hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipEventCreate(&x->ev0);
-    if (e == hipSuccess) e = hipEventCreate(&x->ev1);
+    // (timing only: without the system-scope fence a record does not write L2 back)
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&x->ev0, hipEventDisableSystemFence);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&x->ev1, hipEventDisableSystemFence);
     if (e == hipSuccess && !quant && !x->ivf) {
         e = x->rsq_max.ensure(256, 0, x->stream, false);
         if (e == hipSuccess) e = hipMemset(x->rsq_max.p, 0, 256);
@@ -2491,42 +2538,30 @@ static int host_query(bv_index *idx, const float *q, uint32_t nq, uint32_t kprim
     }
     int rc = ensure_built(idx);
     if (rc) return rc;
-    const size_t qbytes = (size_t)nq * idx->dim * 4;
-    HIPX(idx->dev, idx->qin.ensure(qbytes, 0, idx->stream), "query buffer");
-    HIPX(idx->dev, hipEventRecord(idx->ev0, idx->stream), "event");
-    HIPX(idx->dev, hipMemcpyAsync(idx->qin.p, q, qbytes, hipMemcpyHostToDevice, idx->stream), "query upload");
-    const uint32_t *d_mask = nullptr;
-    uint64_t mask_bits = 0;
-    if (mask) {
-        HIPX(idx->dev, idx->mask.ensure(mask_words * 4, 0, idx->stream), "mask buffer");
-        HIPX(idx->dev, hipMemcpyAsync(idx->mask.p, mask, mask_words * 4, hipMemcpyHostToDevice, idx->stream),
-             "mask upload");
-        d_mask = idx->mask.as<uint32_t>();
-        mask_bits = mask_words * 32;
+    hipStream_t st = idx->stream;
+    const size_t qbytes = (size_t)nq * idx->dim * 4, mbytes = mask ? mask_words * 4 : 0;
+    const size_t rbytes = HostIo::pad((size_t)nq * k_out * 4);
+    HIPX(idx->dev, idx->io.begin(HostIo::pad(qbytes) + HostIo::pad(mbytes), st), "query buffer");
+    HIPX(idx->dev, idx->io.out.ensure(2 * rbytes + (size_t)nq * 4), "pinned buffer");
+    uint32_t *o_rows = (uint32_t *)idx->io.out.p, *o_n = (uint32_t *)((char *)idx->io.out.p + 2 * rbytes);
+    float *o_scores = (float *)((char *)idx->io.out.p + rbytes);
+    const float *d_q = (const float *)idx->io.put(q, qbytes);
+    const uint32_t *d_mask = mask ? (const uint32_t *)idx->io.put(mask, mbytes) : nullptr;
+    HIPX(idx->dev, hipEventRecord(idx->ev0, st), "event");
+    HIPX(idx->dev, idx->io.send(st), "query upload");
+    rc = run_pipeline(idx, d_q, nq, kprime, k_out, rerank, d_mask, mask ? mask_words * 32 : 0, o_rows, o_scores, o_n);
+    if (rc) {
+        (void)hipStreamSynchronize(st);  // (launched kernels may still read the buffers)
+        return rc;
     }
-    HIPX(idx->dev, idx->out_rows.ensure((size_t)nq * k_out * 4, 0, idx->stream), "output buffer");
-    HIPX(idx->dev, idx->out_scores.ensure((size_t)nq * k_out * 4, 0, idx->stream), "output buffer");
-    HIPX(idx->dev, idx->out_n.ensure((size_t)nq * 4, 0, idx->stream), "output buffer");
-    rc = run_pipeline(idx, idx->qin.as<float>(), nq, kprime, k_out, rerank, d_mask, mask_bits,
-                      idx->out_rows.as<uint32_t>(), idx->out_scores.as<float>(), idx->out_n.as<uint32_t>());
-    if (rc) return rc;
-    HIPX(idx->dev, idx->h_rows.ensure((size_t)nq * k_out * 4), "pinned buffer");
-    HIPX(idx->dev, idx->h_scores.ensure((size_t)nq * k_out * 4), "pinned buffer");
-    HIPX(idx->dev, idx->h_n.ensure((size_t)nq * 4), "pinned buffer");
-    HIPX(idx->dev, hipMemcpyAsync(idx->h_rows.p, idx->out_rows.p, (size_t)nq * k_out * 4, hipMemcpyDeviceToHost,
-                                  idx->stream), "result download");
-    HIPX(idx->dev, hipMemcpyAsync(idx->h_scores.p, idx->out_scores.p, (size_t)nq * k_out * 4,
-                                  hipMemcpyDeviceToHost, idx->stream), "result download");
-    HIPX(idx->dev, hipMemcpyAsync(idx->h_n.p, idx->out_n.p, (size_t)nq * 4, hipMemcpyDeviceToHost, idx->stream),
-         "result download");
-    HIPX(idx->dev, hipEventRecord(idx->ev1, idx->stream), "event");
-    HIPX(idx->dev, hipStreamSynchronize(idx->stream), "query");
+    HIPX(idx->dev, hipEventRecord(idx->ev1, st), "event");
+    HIPX(idx->dev, hipStreamSynchronize(st), "query");
     timing_collect(idx);
     float gms = 0;
     (void)hipEventElapsedTime(&gms, idx->ev0, idx->ev1);
-    std::memcpy(rows, idx->h_rows.p, (size_t)nq * k_out * 4);
-    std::memcpy(scores, idx->h_scores.p, (size_t)nq * k_out * 4);
-    std::memcpy(n_out, idx->h_n.p, (size_t)nq * 4);
+    std::memcpy(rows, o_rows, (size_t)nq * k_out * 4);
+    std::memcpy(scores, o_scores, (size_t)nq * k_out * 4);
+    std::memcpy(n_out, o_n, (size_t)nq * 4);
     idx->last_query_gpu_ms = gms;
     idx->last_query_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     return BV_OK;
@@ -2781,12 +2816,12 @@ extern "C" int bv_index_rerank(bv_index *idx, const float *q, const uint32_t *ca
         return BV_OK;
     }
     const size_t qb = (size_t)idx->dim * 4;
-    HIPX(idx->dev, idx->qin.ensure(qb, 0, idx->stream), "query buffer");
-    HIPX(idx->dev, hipMemcpyAsync(idx->qin.p, q, qb, hipMemcpyHostToDevice, idx->stream), "upload");
-    HIPX(idx->dev, idx->cand.ensure((size_t)n_cand * 4, 0, idx->stream), "scratch");
-    HIPX(idx->dev, hipMemcpyAsync(idx->cand.p, cand, (size_t)n_cand * 4, hipMemcpyHostToDevice, idx->stream), "upload");
-    HIPX(idx->dev, idx->cand_n.ensure(4, 0, idx->stream), "scratch");
-    HIPX(idx->dev, hipMemcpyAsync(idx->cand_n.p, &n_cand, 4, hipMemcpyHostToDevice, idx->stream), "upload");
+    HIPX(idx->dev, idx->io.begin(HostIo::pad(qb) + HostIo::pad((size_t)n_cand * 4) + HostIo::pad(4), idx->stream),
+         "query buffer");
+    const float *d_q = (const float *)idx->io.put(q, qb);
+    const uint32_t *d_cand = (const uint32_t *)idx->io.put(cand, (size_t)n_cand * 4);
+    const uint32_t *d_cand_n = (const uint32_t *)idx->io.put(&n_cand, 4);
+    HIPX(idx->dev, idx->io.send(idx->stream), "upload");
     HIPX(idx->dev, idx->rr_keys.ensure((size_t)n_cand * 8, 0, idx->stream), "scratch");
     {
         const size_t old = idx->rr_tickets.cap;
@@ -2794,45 +2829,39 @@ extern "C" int bv_index_rerank(bv_index *idx, const float *q, const uint32_t *ca
         if (idx->rr_tickets.cap != old)
             HIPX(idx->dev, hipMemsetAsync(idx->rr_tickets.p, 0, idx->rr_tickets.cap, idx->stream), "scratch");
     }
-    HIPX(idx->dev, idx->out_rows.ensure((size_t)kk * 4, 0, idx->stream), "output");
-    HIPX(idx->dev, idx->out_scores.ensure((size_t)kk * 4, 0, idx->stream), "output");
-    HIPX(idx->dev, idx->out_n.ensure(4, 0, idx->stream), "output");
+    const size_t rb = HostIo::pad((size_t)kk * 4);
+    HIPX(idx->dev, idx->io.out.ensure(2 * rb + 4), "pinned buffer");
+    char *out = (char *)idx->io.out.p;
     RerankArgs r{};
     r.rows = idx->raw.as<float>();
     r.dim = idx->dim;
-    r.q = idx->qin.as<float>();
+    r.q = d_q;
     r.q_stride = idx->dim;
-    r.cand_rows = idx->cand.as<uint32_t>();
-    r.cand_n = idx->cand_n.as<uint32_t>();
+    r.cand_rows = d_cand;
+    r.cand_n = d_cand_n;
     r.kprime = n_cand;
     r.k_out = kk;
     r.rr_keys = idx->rr_keys.as<uint64_t>();
     r.tickets = idx->rr_tickets.as<uint32_t>();
-    r.out_rows = idx->out_rows.as<uint32_t>();
-    r.out_scores = idx->out_scores.as<float>();
-    r.out_n = idx->out_n.as<uint32_t>();
+    r.out_rows = (uint32_t *)out;
+    r.out_scores = (float *)(out + rb);
+    r.out_n = (uint32_t *)(out + 2 * rb);
     HIPX(idx->dev, launch_rerank(r, 1, idx->stream), "rerank kernel");
-    HIPX(idx->dev, hipMemcpyAsync(rows, idx->out_rows.p, (size_t)kk * 4, hipMemcpyDeviceToHost, idx->stream), "download");
-    HIPX(idx->dev, hipMemcpyAsync(scores, idx->out_scores.p, (size_t)kk * 4, hipMemcpyDeviceToHost, idx->stream),
-         "download");
-    HIPX(idx->dev, hipMemcpyAsync(n_out, idx->out_n.p, 4, hipMemcpyDeviceToHost, idx->stream), "download");
     HIPX(idx->dev, hipStreamSynchronize(idx->stream), "rerank");
+    *n_out = *r.out_n;
+    std::memcpy(rows, r.out_rows, (size_t)*n_out * 4);
+    std::memcpy(scores, r.out_scores, (size_t)*n_out * 4);
     return BV_OK;
 }
 
 // Exact scores of the n_list rows at idx->sel_list against q (Store.dotRow /
 // Store.l2Row order), then their top k by a device sort.
-static int exact_list_topk(bv_index *idx, const float *q, uint64_t n_list, uint32_t k, uint32_t *rows, float *scores,
-                           uint32_t *n_out) {
+// (d_q and d_list on the device)
+static int exact_list_topk(bv_index *idx, const float *d_q, const uint32_t *d_list, uint64_t n_list, uint32_t k,
+                           uint32_t *rows, float *scores, uint32_t *n_out) {
     hipStream_t s = idx->stream;
-    const size_t qb = (size_t)idx->dim * 4;
-    HIPX(idx->dev, idx->qin.ensure(qb, 0, s), "query buffer");
-    HIPX(idx->dev, hipMemcpyAsync(idx->qin.p, q, qb, hipMemcpyHostToDevice, s), "upload");
-    HIPX(idx->dev, idx->sel_misc.ensure(8, 0, s), "scratch");
-    HIPX(idx->dev, launch_zero(idx->sel_misc.p, 4, s), "scratch clear");
     const bool l2 = idx->d.metric == BV_METRIC_L2;
     const uint32_t kk = (uint32_t)std::min<uint64_t>(k, n_list);
-    uint32_t bad = 0;
     const auto bad_row = [&]() {
         return fail(BV_E_INVALID, "a listed row is out of range (the index holds %llu rows)",
                     (unsigned long long)idx->rows);
@@ -2848,7 +2877,7 @@ static int exact_list_topk(bv_index *idx, const float *q, uint64_t n_list, uint3
         SlotArgs &a = p.s;
         a.codes = idx->raw.p;
         a.padded_dim = idx->dim;
-        a.cand = idx->sel_list.as<uint32_t>();
+        a.cand = d_list;
         a.n = (uint32_t)n_list;
         a.nq = 1;
         a.rw = rw;
@@ -2858,37 +2887,31 @@ static int exact_list_topk(bv_index *idx, const float *q, uint64_t n_list, uint3
         HIPX(idx->dev, idx->sl_best.ensure((size_t)a.nslots * 8, 0, s), "scratch");
         a.ord = idx->sl_ord.as<uint32_t>();
         a.best = idx->sl_best.as<uint64_t>();
-        HIPX(idx->dev, idx->out_rows.ensure((size_t)kk * 4, 0, s), "scratch");
-        HIPX(idx->dev, idx->out_scores.ensure((size_t)kk * 4, 0, s), "scratch");
-        HIPX(idx->dev, idx->out_n.ensure(4, 0, s), "scratch");
+        const size_t rb = HostIo::pad((size_t)kk * 4);
+        HIPX(idx->dev, idx->io.out.ensure(2 * rb + 8), "pinned buffer");
+        char *out = (char *)idx->io.out.p;
+        uint32_t *o_n = (uint32_t *)(out + 2 * rb);
+        o_n[1] = 0;  // set when a listed row is out of range
         p.kk = kk;
         p.k_out = kk;
-        p.out_rows = idx->out_rows.as<uint32_t>();
-        p.out_scores = idx->out_scores.as<float>();
-        p.out_n = idx->out_n.as<uint32_t>();
-        HIPX(idx->dev,
-             launch_rows_exact(a, idx->qin.as<float>(), idx->rows, l2, idx->sel_misc.as<uint32_t>(), s),
-             "exact row kernel");
+        p.out_rows = (uint32_t *)out;
+        p.out_scores = (float *)(out + rb);
+        p.out_n = o_n;
+        HIPX(idx->dev, launch_rows_exact(a, d_q, idx->rows, l2, o_n + 1, s), "exact row kernel");
         HIPX(idx->dev, launch_pick_topk(p, s), "selection kernel");
-        uint32_t n = 0;
-        std::vector<uint32_t> r(kk);
-        std::vector<float> sc(kk);
-        HIPX(idx->dev, hipMemcpyAsync(&bad, idx->sel_misc.p, 4, hipMemcpyDeviceToHost, s), "download");
-        HIPX(idx->dev, hipMemcpyAsync(&n, idx->out_n.p, 4, hipMemcpyDeviceToHost, s), "download");
-        HIPX(idx->dev, hipMemcpyAsync(r.data(), idx->out_rows.p, (size_t)kk * 4, hipMemcpyDeviceToHost, s), "download");
-        HIPX(idx->dev, hipMemcpyAsync(sc.data(), idx->out_scores.p, (size_t)kk * 4, hipMemcpyDeviceToHost, s),
-             "download");
         HIPX(idx->dev, hipStreamSynchronize(s), "exact rows");
-        if (bad) return bad_row();
-        std::memcpy(rows, r.data(), (size_t)n * 4);
-        std::memcpy(scores, sc.data(), (size_t)n * 4);
-        *n_out = n;
+        if (o_n[1]) return bad_row();
+        std::memcpy(rows, p.out_rows, (size_t)o_n[0] * 4);
+        std::memcpy(scores, p.out_scores, (size_t)o_n[0] * 4);
+        *n_out = o_n[0];
         return BV_OK;
     }
+    uint32_t bad = 0;
+    HIPX(idx->dev, idx->sel_misc.ensure(8, 0, s), "scratch");
+    HIPX(idx->dev, launch_zero(idx->sel_misc.p, 4, s), "scratch clear");
     HIPX(idx->dev, idx->sel_keys.ensure(n_list * 8, 0, s), "scratch");
-    HIPX(idx->dev, sel_exact_row_keys(idx->raw.as<float>(), idx->rows, idx->dim, l2, idx->qin.as<float>(),
-                                      idx->sel_list.as<uint32_t>(), n_list, idx->sel_keys.as<uint64_t>(),
-                                      idx->sel_misc.as<uint32_t>(), s),
+    HIPX(idx->dev, sel_exact_row_keys(idx->raw.as<float>(), idx->rows, idx->dim, l2, d_q, d_list, n_list,
+                                      idx->sel_keys.as<uint64_t>(), idx->sel_misc.as<uint32_t>(), s),
          "exact row kernel");
     HIPX(idx->dev, hipMemcpyAsync(&bad, idx->sel_misc.p, 4, hipMemcpyDeviceToHost, s), "download");
     HIPX(idx->dev, hipStreamSynchronize(s), "exact rows");
@@ -2916,9 +2939,12 @@ extern "C" int bv_index_query_rows(bv_index *idx, const float *q, const uint32_t
         *n_out = 0;
         return BV_OK;
     }
-    HIPX(idx->dev, idx->sel_list.ensure(n_list * 4, 0, idx->stream), "scratch");
-    HIPX(idx->dev, hipMemcpyAsync(idx->sel_list.p, list, n_list * 4, hipMemcpyHostToDevice, idx->stream), "upload");
-    return exact_list_topk(idx, q, n_list, k, rows, scores, n_out);
+    const size_t qb = (size_t)idx->dim * 4;
+    HIPX(idx->dev, idx->io.begin(HostIo::pad(qb) + HostIo::pad(n_list * 4), idx->stream), "query buffer");
+    const float *d_q = (const float *)idx->io.put(q, qb);
+    const uint32_t *d_list = (const uint32_t *)idx->io.put(list, n_list * 4);
+    HIPX(idx->dev, idx->io.send(idx->stream), "upload");
+    return exact_list_topk(idx, d_q, d_list, n_list, k, rows, scores, n_out);
 }
 
 extern "C" int bv_index_query_rows_masked(bv_index *idx, const float *q, const uint32_t *mask_words, uint64_t n_words,
@@ -2936,12 +2962,15 @@ extern "C" int bv_index_query_rows_masked(bv_index *idx, const float *q, const u
         return BV_OK;
     }
     hipStream_t s = idx->stream;
-    HIPX(idx->dev, idx->mask.ensure(words * 4, 0, s), "mask buffer");
-    HIPX(idx->dev, hipMemcpyAsync(idx->mask.p, mask_words, words * 4, hipMemcpyHostToDevice, s), "upload");
+    const size_t qb = (size_t)idx->dim * 4;
+    HIPX(idx->dev, idx->io.begin(HostIo::pad(qb) + HostIo::pad(words * 4), s), "query buffer");
+    const float *d_q = (const float *)idx->io.put(q, qb);
+    const uint32_t *d_mask = (const uint32_t *)idx->io.put(mask_words, words * 4);
+    HIPX(idx->dev, idx->io.send(s), "upload");
     HIPX(idx->dev, idx->sel_popc.ensure(words * 4, 0, s), "scratch");
     HIPX(idx->dev, idx->sel_off.ensure(words * 4, 0, s), "scratch");
     HIPX(idx->dev, idx->sel_misc.ensure(8, 0, s), "scratch");
-    HIPX(idx->dev, sel_mask_counts(idx->mask.as<uint32_t>(), words, idx->rows, idx->sel_popc.as<uint32_t>(), s),
+    HIPX(idx->dev, sel_mask_counts(d_mask, words, idx->rows, idx->sel_popc.as<uint32_t>(), s),
          "mask count kernel");
     size_t tb = 0;
     HIPX(idx->dev, sel_exclusive_scan(nullptr, tb, nullptr, nullptr, words, s), "scan sizing");
@@ -2952,7 +2981,7 @@ extern "C" int bv_index_query_rows_masked(bv_index *idx, const float *q, const u
          "scan");
     // the list can hold every row: sized before its length is known
     HIPX(idx->dev, idx->sel_list.ensure(words * 32 * 4, 0, s), "scratch");
-    HIPX(idx->dev, sel_mask_rows(idx->mask.as<uint32_t>(), words, idx->rows, idx->sel_popc.as<uint32_t>(),
+    HIPX(idx->dev, sel_mask_rows(d_mask, words, idx->rows, idx->sel_popc.as<uint32_t>(),
                                  idx->sel_off.as<uint32_t>(), idx->sel_list.as<uint32_t>(),
                                  idx->sel_misc.as<uint32_t>() + 1, s),
          "mask row kernel");
@@ -2963,7 +2992,7 @@ extern "C" int bv_index_query_rows_masked(bv_index *idx, const float *q, const u
         *n_out = 0;
         return BV_OK;
     }
-    return exact_list_topk(idx, q, n_list, k, rows, scores, n_out);
+    return exact_list_topk(idx, d_q, idx->sel_list.as<uint32_t>(), n_list, k, rows, scores, n_out);
 }
 
 // Dense scores of one query for every row (the scan's score for each row),
@@ -3527,7 +3556,8 @@ struct bv_graph {
     hipStream_t stream = nullptr;
     uint32_t dim = 0, metric = 0, degree = 0;
     uint64_t corpus_rows = 0, graph_rows = 0;
-    DevBuf corpus, graph, queries, entries, out_rows, out_scores, out_n, beam_d, beam_i;
+    DevBuf corpus, graph, beam_d, beam_i;
+    HostIo io;
 };
 
 namespace {
@@ -3553,12 +3583,11 @@ uint32_t graph_seeds(uint32_t entry, uint64_t rows, uint32_t *out) {
 int graph_run(bv_graph *g, const float *queries, uint32_t nq, const uint32_t *entries, uint32_t n_entries,
               uint32_t ef_active, uint32_t iter_cap, uint32_t k, uint32_t stride, bool beams) {
     hipStream_t s = g->stream;
-    const size_t qb = (size_t)nq * g->dim * 4;
-    HIPX(g->dev, g->queries.ensure(qb, 0, s), "query buffer");
-    HIPX(g->dev, hipMemcpyAsync(g->queries.p, queries, qb, hipMemcpyHostToDevice, s), "upload");
-    HIPX(g->dev, g->entries.ensure(std::max<size_t>(n_entries, 1) * 4, 0, s), "scratch");
-    if (n_entries)
-        HIPX(g->dev, hipMemcpyAsync(g->entries.p, entries, (size_t)n_entries * 4, hipMemcpyHostToDevice, s), "upload");
+    const size_t qb = (size_t)nq * g->dim * 4, eb = (size_t)n_entries * 4;
+    HIPX(g->dev, g->io.begin(HostIo::pad(qb) + HostIo::pad(eb), s), "query buffer");
+    const float *d_q = (const float *)g->io.put(queries, qb);
+    const uint32_t *d_e = (const uint32_t *)g->io.put(entries, eb);
+    HIPX(g->dev, g->io.send(s), "upload");
     GraphArgs a{};
     a.corpus = g->corpus.as<float>();
     a.dim = g->dim;
@@ -3566,8 +3595,8 @@ int graph_run(bv_graph *g, const float *queries, uint32_t nq, const uint32_t *en
     a.graph = g->graph.as<uint32_t>();
     a.K = g->degree;
     a.graph_rows = g->graph_rows;
-    a.queries = g->queries.as<float>();
-    a.entries = g->entries.as<uint32_t>();
+    a.queries = d_q;
+    a.entries = d_e;
     a.n_entries = n_entries;
     a.efA = ef_active;
     a.iter_cap = iter_cap;
@@ -3577,14 +3606,14 @@ int graph_run(bv_graph *g, const float *queries, uint32_t nq, const uint32_t *en
         a.beam_dist = g->beam_d.as<float>();
         a.beam_id = g->beam_i.as<uint32_t>();
     } else {
-        HIPX(g->dev, g->out_rows.ensure((size_t)nq * std::max(stride, 1u) * 4, 0, s), "scratch");
-        HIPX(g->dev, g->out_scores.ensure((size_t)nq * std::max(stride, 1u) * 4, 0, s), "scratch");
-        HIPX(g->dev, g->out_n.ensure((size_t)nq * 4, 0, s), "scratch");
+        const size_t rb = HostIo::pad((size_t)nq * stride * 4);
+        HIPX(g->dev, g->io.out.ensure(2 * rb + (size_t)nq * 4), "pinned buffer");
+        char *out = (char *)g->io.out.p;
         a.k = k;
         a.out_stride = stride;
-        a.out_rows = g->out_rows.as<uint32_t>();
-        a.out_scores = g->out_scores.as<float>();
-        a.out_n = g->out_n.as<uint32_t>();
+        a.out_rows = (uint32_t *)out;
+        a.out_scores = (float *)(out + rb);
+        a.out_n = (uint32_t *)(out + 2 * rb);
     }
     HIPX(g->dev, launch_graph_beam(a, nq, g->metric == BV_METRIC_L2, s), "graph search kernel");
     return BV_OK;
@@ -3682,11 +3711,15 @@ extern "C" int bv_graph_search(bv_graph *g, const float *queries, uint32_t nq, u
     const uint32_t ns = graph_seeds(entry, g->graph_rows, seeds);
     rc = graph_run(g, queries, nq, seeds, ns, efA, efA, kk, k, false);
     if (rc) return rc;
-    HIPX(g->dev, hipMemcpyAsync(rows, g->out_rows.p, (size_t)nq * k * 4, hipMemcpyDeviceToHost, g->stream), "download");
-    HIPX(g->dev, hipMemcpyAsync(scores, g->out_scores.p, (size_t)nq * k * 4, hipMemcpyDeviceToHost, g->stream),
-         "download");
-    HIPX(g->dev, hipMemcpyAsync(n_out, g->out_n.p, (size_t)nq * 4, hipMemcpyDeviceToHost, g->stream), "download");
     HIPX(g->dev, hipStreamSynchronize(g->stream), "graph search");
+    // (a query's hits past its count are left as the caller had them)
+    const size_t rb = HostIo::pad((size_t)nq * k * 4);
+    const char *out = (const char *)g->io.out.p;
+    std::memcpy(n_out, out + 2 * rb, (size_t)nq * 4);
+    for (uint32_t i = 0; i < nq; i++) {
+        std::memcpy(rows + (size_t)i * k, out + (size_t)i * k * 4, (size_t)n_out[i] * 4);
+        std::memcpy(scores + (size_t)i * k, out + rb + (size_t)i * k * 4, (size_t)n_out[i] * 4);
+    }
     return BV_OK;
 }
 

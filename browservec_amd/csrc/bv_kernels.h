@@ -518,6 +518,10 @@ hipError_t launch_mq_select(const MqSelArgs &a, uint32_t nq, hipStream_t s);
 // so the launch is safe to record in a captured graph).
 hipError_t launch_zero(void *p, size_t bytes, hipStream_t s);
 
+// dst[0, bytes) = src[0, bytes) (a multiple of 16; src in pinned host memory
+// the device maps), by a kernel.
+hipError_t launch_copy_in(void *dst, const void *src, size_t bytes, hipStream_t s);
+
 bool scan_supported(int codec, uint32_t units);
 hipError_t launch_scan(int codec, uint32_t units, const ScanArgs &a, uint32_t nq, hipStream_t s);
 hipError_t launch_encode(const EncodeArgs &a, hipStream_t s);

@@ -107,7 +107,24 @@ __global__ __launch_bounds__(256) void zero_words(uint32_t *p, uint64_t words) {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < words; i += stride) p[i] = 0u;
 }
 
+// Host memory over PCIe: bound by its latency for a few queries (2-3 us), by
+// its bandwidth for large batches.
+__global__ __launch_bounds__(256) void copy_in(uint4 *dst, const uint4 *src, uint64_t n) {
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) dst[i] = src[i];
+}
+
 }  // namespace
+
+hipError_t launch_copy_in(void *dst, const void *src, size_t bytes, hipStream_t s) {
+    if (bytes == 0) return hipSuccess;
+    if (bytes & 15) return hipErrorInvalidValue;
+    const uint64_t n = bytes / 16;
+    uint64_t blocks = (n + 255) / 256;
+    if (blocks > 1024) blocks = 1024;
+    hipLaunchKernelGGL(copy_in, dim3((uint32_t)blocks), dim3(256), 0, s, (uint4 *)dst, (const uint4 *)src, n);
+    return hipGetLastError();
+}
 
 hipError_t launch_zero(void *p, size_t bytes, hipStream_t s) {
     if (bytes == 0) return hipSuccess;
