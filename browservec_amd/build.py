@@ -21,7 +21,7 @@ ARCH = os.environ.get("BV_OFFLOAD_ARCH", "gfx950")
 # (bv_scan_*.hip) so that they compile in parallel.
 SCAN_CODECS = ["f32dot", "f32l2", "q8", "q4", "q1a", "q1p", "ham", "i8s", "f32dot_s", "f32l2_s"]
 SOURCES = (["bv_kernels.hip"] + [f"bv_scan_{c}.hip" for c in SCAN_CODECS] +
-           ["bv_ivf.hip", "bv_mq.hip", "bv_pick.hip", "bv_select.hip", "bv_graph.hip", "bv_api.cpp"])
+           ["bv_ivf.hip", "bv_mq.hip", "bv_mqf.hip", "bv_pick.hip", "bv_select.hip", "bv_graph.hip", "bv_api.cpp"])
 HEADERS = ["bv_kernels.h", "bv_device.h", "bv_scan.h", "bv_slots.h", "bv_mfma.h", "bv_exact.h", "bv_sort.h"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

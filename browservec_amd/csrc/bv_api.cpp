@@ -209,8 +209,8 @@ struct bv_index {
     DevBuf out_rows, out_scores, out_n;
     DevBuf cand, cand_n, dense;
     DevBuf mq_cand, mq_cnt, mq_tau, mq_tau2, mq_flag;  // batched matrix-core scans
-    DevBuf rsq, rsq_max;                      // flat fp32: squared row norms and their maximum (float bits)
-    DevBuf mq_qsq, mq_slack, mq_rows;         // exact fp32 batches: query norms, slack, surviving rows
+    DevBuf rsq, bf16_ratio;                   // flat fp32: squared row norms; the largest relative bf16 rounding of a row (float bits)
+    DevBuf mq_qbf, mq_qk, mq_rows;            // fp32 batches: bf16 queries, constants of their bounds; surviving rows
     DevBuf cnorm, mq_rq, mq_up, mq_kept;       // flat int8 level-one batches: row code norms, query bounds, upper bounds, kept counts
     DevBuf mq_bk, mq_bu, mq_bc;               // level-one batches: per-workgroup buckets (lower keys, upper bounds, lengths)
     DevBuf sel_keys, sel_sorted, sel_tmp;     // selection by sort: keys, sorted keys, hipCUB scratch
@@ -455,8 +455,8 @@ extern "C" int bv_index_create(bv_device *dev, const bv_index_desc *desc, bv_ind
     if (e == hipSuccess) e = hipEventCreateWithFlags(&x->ev0, hipEventDisableSystemFence);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&x->ev1, hipEventDisableSystemFence);
     if (e == hipSuccess && !quant && !x->ivf) {
-        e = x->rsq_max.ensure(256, 0, x->stream, false);
-        if (e == hipSuccess) e = hipMemset(x->rsq_max.p, 0, 256);
+        e = x->bf16_ratio.ensure(256, 0, x->stream, false);
+        if (e == hipSuccess) e = hipMemset(x->bf16_ratio.p, 0, 256);
     }
     if (e == hipSuccess && quant) {
         std::vector<float> s;
@@ -781,7 +781,8 @@ static int append_common(bv_index *idx, const float *data, bool device_src, uint
     }
     const size_t taken = dst_slot.size();
     const bool extend = idx->ivf && idx->built_rows == base && idx->nlist && idx->d.ivf_incremental;
-    HIPX(idx->dev, idx->raw.ensure(total * rb, base * rb, idx->stream), "row buffer");
+    // (16 bytes more: mqf_scan reads rows in 16-byte pieces)
+    HIPX(idx->dev, idx->raw.ensure(total * rb + 16, base * rb, idx->stream), "row buffer");
     if (idx->quant) {
         HIPX(idx->dev, idx->codes.ensure(total * idx->row_bytes, base * idx->row_bytes, idx->stream), "code buffer");
         HIPX(idx->dev, idx->scales.ensure(total * 4, base * 4, idx->stream), "scale buffer");
@@ -842,7 +843,7 @@ static int append_common(bv_index *idx, const float *data, bool device_src, uint
         if (norms)
             HIPX(idx->dev,
                  launch_row_sqnorms(idx->raw.as<float>() + r0 * idx->dim, m, idx->dim, idx->rsq.as<float>() + r0,
-                                    idx->rsq_max.as<uint32_t>(), idx->stream),
+                                    idx->bf16_ratio.as<uint32_t>(), idx->stream),
                  "norm kernel");
         if (idx->quant) {
             EncodeArgs e{};
@@ -1576,11 +1577,9 @@ constexpr uint32_t MQ_MIN_Q = 8;  // smallest batch for the matrix-core path (it
 
 static bool mq_eligible(const bv_index *idx, uint32_t nq, const uint32_t *d_mask) {
     if (idx->ivf || d_mask || nq < MQ_MIN_Q || idx->rows == 0) return false;
-    // fp32: dot / cosine / l2 above the sample size (smaller corpora: one fused
-    // launch for the whole batch is already exact and cheap)
+    // fp32: above the sample size (smaller corpora: slot scans)
     if (!idx->quant)
-        return (idx->codec == C_F32DOT || idx->codec == C_F32L2) && mq_f32_supported(idx->dim) &&
-               idx->rows > MQ_SAMPLE;
+        return mqf_supported(idx->dim) && idx->rows > MQ_SAMPLE;
     const uint32_t u16 = idx->P / 16;  // 16-code units per row
     const bool shape = u16 >= 2 && (u16 % 2) == 0 && u16 / 2 <= MQ_MAX_STEPS;
     // Hamming and 1-bit asymmetric: the first-level pass over +1 / -1 rows,
@@ -1606,116 +1605,6 @@ static uint32_t mq_groups(const bv_index *idx, uint32_t qblocks) {
     const int cus = idx->dev->prop.multiProcessorCount > 0 ? idx->dev->prop.multiProcessorCount : 256;
     const uint32_t g = (uint32_t)cus / (8u * qblocks);
     return g ? g : 1u;
-}
-
-// fp32 batches, exactly equal to single queries.  The matrix-core scan is a
-// prefilter: a dense pass over MQ_SAMPLE strided rows gives each query a
-// bound (its kprime-th best sample score), a pass over every row keeps the
-// ids of the rows whose matrix-core score reaches the bound minus the
-// slack 2E (E bounds the difference between a matrix-core score and the
-// single-query scan's), and the fused scan re-scores exactly those rows in
-// indexed mode with the single-query arithmetic and selects the top-k of the
-// same keys.  A query whose kept rows overflow their buffer runs the fused
-// scan over every row.
-static int run_batched_f32(bv_index *idx, const float *d_q, uint32_t nq, uint32_t kprime, uint32_t k_out,
-                           uint32_t *d_rows, float *d_scores, uint32_t *d_n) {
-    const uint64_t N = idx->rows, S = MQ_SAMPLE;  // N > S (mq_eligible)
-    const bool l2 = idx->codec == C_F32L2;
-    uint64_t cap = std::max<uint64_t>(S, 4ull * kprime * ((N + S - 1) / S));
-    cap = std::min<uint64_t>(cap, N);
-    hipStream_t s = idx->stream;
-    HIPX(idx->dev, idx->mq_cand.ensure((size_t)nq * std::max<uint64_t>(cap, S) * 8, 0, s), "scratch");
-    HIPX(idx->dev, idx->mq_rows.ensure((size_t)nq * cap * 4, 0, s), "scratch");
-    HIPX(idx->dev, idx->mq_cnt.ensure((size_t)nq * 4, 0, s), "scratch");
-    HIPX(idx->dev, idx->mq_tau.ensure((size_t)nq * 8, 0, s), "scratch");
-    HIPX(idx->dev, idx->mq_qsq.ensure((size_t)nq * 4, 0, s), "scratch");
-    HIPX(idx->dev, idx->mq_slack.ensure((size_t)nq * 4, 0, s), "scratch");
-    HIPX(idx->dev, idx->h_cnt.ensure((size_t)nq * 4), "pinned buffer");
-
-    timing_begin(idx);
-    HIPX(idx->dev,
-         launch_mq_f32_qconst(d_q, nq, idx->dim, idx->rsq_max.as<uint32_t>(), l2 ? 1 : 0, idx->mq_qsq.as<float>(),
-                              idx->mq_slack.as<float>(), s),
-         "query norm kernel");
-    MqArgs m{};
-    m.codes = idx->raw.as<uint32_t>();
-    m.W = idx->dim;
-    m.units = idx->dim / 8;
-    m.qlev = (const unsigned char *)d_q;
-    m.qstride = (uint64_t)idx->dim * 4;
-    m.nq = nq;
-    m.qblocks = (nq + MQ_QB - 1) / MQ_QB;
-    m.groups = mq_groups(idx, m.qblocks);
-    m.cand = idx->mq_cand.as<uint64_t>();
-    m.cnt = idx->mq_cnt.as<uint32_t>();
-    m.cap = std::max<uint64_t>(cap, S);
-    m.l2 = l2 ? 1 : 0;
-    m.rsq = idx->rsq.as<float>();
-    m.qsq = idx->mq_qsq.as<float>();
-    m.slack = idx->mq_slack.as<float>();
-    // sample pass: every (approximate) key of logical rows i < S
-    m.n = S;
-    m.row_step = N / S;
-    HIPX(idx->dev, hipMemsetD32Async((hipDeviceptr_t)idx->mq_cnt.p, (int)S, nq, s), "scratch");
-    HIPX(idx->dev, launch_mq_scan_f32(m, s), "batched scan kernel");
-    MqSelArgs sa{};
-    sa.cand = m.cand;
-    sa.cnt = m.cnt;
-    sa.cap = m.cap;
-    sa.kk = kprime;
-    sa.tau = idx->mq_tau.as<uint64_t>();
-    HIPX(idx->dev, launch_mq_select(sa, nq, s), "batched select kernel");
-    // full pass: ids of every row that can rank
-    HIPX(idx->dev, hipMemsetAsync(idx->mq_cnt.p, 0, (size_t)nq * 4, s), "scratch");
-    m.n = N;
-    m.row_step = 1;
-    m.tau = idx->mq_tau.as<uint64_t>();
-    m.cap = cap;
-    m.rows_out = idx->mq_rows.as<uint32_t>();
-    HIPX(idx->dev, launch_mq_scan_f32(m, s), "batched scan kernel");
-    HIPX(idx->dev, hipMemcpyAsync(idx->h_cnt.p, idx->mq_cnt.p, (size_t)nq * 4, hipMemcpyDeviceToHost, s),
-         "count download");
-    HIPX(idx->dev, hipStreamSynchronize(s), "batched scan");
-    const uint32_t *cnt = (const uint32_t *)idx->h_cnt.p;
-    uint64_t most = 1;
-    for (uint32_t i = 0; i < nq; i++) most = std::max<uint64_t>(most, std::min<uint64_t>(cnt[i], cap));
-    // exact re-score of the kept rows: the fused scan in indexed mode
-    ScanArgs a{};
-    const uint32_t grid = grid_for(idx, most, kprime, 0);
-    int rc = scan_scratch(idx, nq, grid, kprime, 0, a);
-    if (rc) return rc;
-    a.codes = idx->raw.p;
-    a.row_bytes = idx->row_bytes;
-    a.units = idx->units;
-    a.padded_dim = idx->P;
-    a.scale_mul = 1.0f;
-    a.q = d_q;
-    a.q_stride = (uint64_t)idx->dim * 4;
-    a.cand = idx->mq_rows.as<uint32_t>();
-    a.cand_n = idx->mq_cnt.as<uint32_t>();
-    a.cand_stride = cap;
-    a.n = cap;
-    a.kprime = kprime;
-    a.grid = grid;
-    a.k_out = k_out;
-    a.out_rows = d_rows;
-    a.out_scores = d_scores;
-    a.out_n = d_n;
-    HIPX(idx->dev, launch_scan(idx->codec, idx->units, a, nq, s), "scan kernel");
-    timing_end(idx);
-    uint64_t scanned = N + S;
-    for (uint32_t i = 0; i < nq; i++) scanned += std::min<uint64_t>(cnt[i], cap);
-    idx->last_scanned = scanned;
-    // queries whose kept rows overflowed: the fused scan over every row
-    std::vector<uint32_t> over;
-    for (uint32_t i = 0; i < nq; i++)
-        if (cnt[i] > cap) over.push_back(i);
-    for (uint32_t i : over) {
-        rc = run_fused(idx, d_q + (size_t)i * idx->dim, 1, kprime, k_out, false, nullptr, 0,
-                       d_rows + (size_t)i * k_out, d_scores + (size_t)i * k_out, d_n + i);
-        if (rc) return rc;
-    }
-    return BV_OK;
 }
 
 // int8 batches above the sample size, exactly equal to single queries.  The
@@ -1861,6 +1750,98 @@ static int finish_batched_indexed(bv_index *idx, const float *d_q, uint32_t nq, 
         if (rc) return rc;
     }
     return BV_OK;
+}
+
+// fp32 batches, exactly equal to single queries: the bf16 prefilter
+// (mqf_scan) bounds every row's score, and the passes are those of
+// run_batched_q8 below: a dense pass over MQ_SAMPLE strided rows gives each
+// query a bound (its kprime-th best lower bound), the first eighth of the rows
+// a tighter one, the rest run under the better of the two, and what reaches
+// the kprime-th best lower bound of the joined list is scored by the fused
+// scan in indexed mode with the single-query arithmetic.
+static int run_batched_f32(bv_index *idx, const float *d_q, uint32_t nq, uint32_t kprime, uint32_t k_out,
+                           uint32_t *d_rows, float *d_scores, uint32_t *d_n) {
+    const uint64_t N = idx->rows, S = MQ_SAMPLE;  // N > S (mq_eligible)
+    const uint32_t dim = idx->dim;
+    uint64_t cap = std::max<uint64_t>(S, 4ull * kprime * ((N + S - 1) / S));
+    cap = std::min<uint64_t>(cap, N);
+    hipStream_t s = idx->stream;
+    const uint32_t qblocks = (nq + mqf_block(dim) - 1) / mqf_block(dim);
+    const int cus = idx->dev->prop.multiProcessorCount > 0 ? idx->dev->prop.multiProcessorCount : 256;
+    const uint32_t nwg = std::min<uint32_t>(1024, std::max<uint32_t>(8, (uint32_t)cus / qblocks & ~7u));
+    const uint32_t capw = (uint32_t)((std::max<uint64_t>(128, (cap + nwg - 1) / nwg) + 15) & ~15ull);
+    const uint64_t qstride = mqf_qstride(dim);
+    HIPX(idx->dev, idx->mq_cand.ensure((size_t)nq * std::max<uint64_t>(cap, S) * 8, 0, s), "scratch");
+    HIPX(idx->dev, idx->mq_up.ensure((size_t)nq * cap * 4, 0, s), "scratch");
+    HIPX(idx->dev, idx->mq_bk.ensure((size_t)nq * nwg * capw * 8, 0, s), "scratch");
+    HIPX(idx->dev, idx->mq_bu.ensure((size_t)nq * nwg * capw * 4, 0, s), "scratch");
+    HIPX(idx->dev, idx->mq_bc.ensure((size_t)nq * nwg * 4, 0, s), "scratch");
+    HIPX(idx->dev, idx->mq_rows.ensure((size_t)nq * cap * 4, 0, s), "scratch");
+    HIPX(idx->dev, idx->mq_cnt.ensure((size_t)nq * 4, 0, s), "scratch");
+    HIPX(idx->dev, idx->mq_kept.ensure((size_t)nq * 4, 0, s), "scratch");
+    HIPX(idx->dev, idx->mq_tau.ensure((size_t)nq * 8, 0, s), "scratch");
+    HIPX(idx->dev, idx->mq_qbf.ensure((size_t)nq * qstride, 0, s), "scratch");
+    HIPX(idx->dev, idx->mq_qk.ensure((size_t)nq * sizeof(MqfQuery), 0, s), "scratch");
+    HIPX(idx->dev, idx->h_cnt.ensure((size_t)nq * 8), "pinned buffer");
+
+    timing_begin(idx);
+    MqfArgs m{};
+    m.dim = dim;
+    m.l2 = idx->d.metric == BV_METRIC_L2;
+    m.qbf = idx->mq_qbf.as<unsigned char>();
+    m.qstride = qstride;
+    m.qk = idx->mq_qk.as<MqfQuery>();
+    m.nq = nq;
+    m.qblocks = qblocks;
+    m.nwg = nwg;
+    m.capw = capw;
+    HIPX(idx->dev,
+         launch_mqf_prep(d_q, nq, dim, idx->bf16_ratio.as<uint32_t>(), m.l2 != 0, idx->mq_qbf.as<unsigned char>(),
+                         idx->mq_qk.as<MqfQuery>(), idx->mq_cnt.as<uint32_t>(), (uint32_t)S, s),
+         "query bound kernel");
+    // sample pass: the lower-bound key of every logical row i < S
+    m.rows = idx->raw.as<float>();
+    m.rsq = idx->rsq.as<float>();
+    m.n = S;
+    m.row_step = N / S;
+    m.cand = idx->mq_cand.as<uint64_t>();
+    m.cap = S;
+    HIPX(idx->dev, launch_mqf_scan(m, s), "batched scan kernel");
+    MqSelArgs sa{};
+    sa.cand = idx->mq_cand.as<uint64_t>();
+    sa.cnt = idx->mq_cnt.as<uint32_t>();
+    sa.cap = S;
+    sa.kk = kprime;
+    sa.tau = idx->mq_tau.as<uint64_t>();
+    HIPX(idx->dev, launch_mq_select(sa, nq, s), "batched select kernel");
+    const uint64_t NA = std::max<uint64_t>(MQ1_ROWS, N / 8 / MQ1_ROWS * MQ1_ROWS);
+    m.tau = idx->mq_tau.as<uint64_t>();
+    m.cand = idx->mq_bk.as<uint64_t>();
+    m.up_out = idx->mq_bu.as<uint32_t>();
+    m.cnt = idx->mq_bc.as<uint32_t>();
+    m.cap = cap;
+    m.row_step = 1;
+    sa.cap = cap;
+    sa.tau_max = true;
+    for (int part = 0; part < 2; ++part) {
+        const uint64_t r0 = part ? NA : 0;
+        m.n = part ? N - NA : NA;
+        m.row_base = r0;
+        m.rows = idx->raw.as<float>() + r0 * dim;
+        m.rsq = idx->rsq.as<float>() + r0;
+        HIPX(idx->dev, launch_mqf_scan(m, s), "batched scan kernel");
+        HIPX(idx->dev,
+             launch_mq1_compact(idx->mq_bk.as<uint64_t>(), idx->mq_bu.as<uint32_t>(), idx->mq_bc.as<uint32_t>(), nwg,
+                                capw, cap, idx->mq_cand.as<uint64_t>(), idx->mq_up.as<uint32_t>(),
+                                idx->mq_cnt.as<uint32_t>(), part > 0, nq, s),
+             "batched compact kernel");
+        HIPX(idx->dev, launch_mq_select(sa, nq, s), "batched select kernel");
+    }
+    HIPX(idx->dev,
+         launch_mq1_keep(idx->mq_cand.as<uint64_t>(), idx->mq_up.as<uint32_t>(), idx->mq_cnt.as<uint32_t>(), cap,
+                         idx->mq_tau.as<uint64_t>(), idx->mq_rows.as<uint32_t>(), idx->mq_kept.as<uint32_t>(), nq, s),
+         "batched keep kernel");
+    return finish_batched_indexed(idx, d_q, nq, kprime, k_out, false, cap, d_rows, d_scores, d_n);
 }
 
 static int run_batched_q8(bv_index *idx, const float *d_q, uint32_t nq, uint32_t kprime, uint32_t k_out,
@@ -2149,18 +2130,26 @@ static int run_batched_q8(bv_index *idx, const float *d_q, uint32_t nq, uint32_t
 
 static int run_batched(bv_index *idx, const float *d_q, uint32_t nq, uint32_t kprime, uint32_t k_out, bool rerank,
                        uint32_t *d_rows, float *d_scores, uint32_t *d_n) {
-    if (!idx->quant) return run_batched_f32(idx, d_q, nq, kprime, k_out, d_rows, d_scores, d_n);
+    if (!idx->quant) {
+        // (in calls of at most 1,024 queries, whose scratch is 0.65 MB a query)
+        uint64_t scanned = 0;
+        for (uint32_t q0 = 0; q0 < nq; q0 += 1024) {
+            const int rc = run_batched_f32(idx, d_q + (size_t)q0 * idx->dim, std::min(1024u, nq - q0), kprime, k_out,
+                                           d_rows + (size_t)q0 * k_out, d_scores + (size_t)q0 * k_out, d_n + q0);
+            if (rc) return rc;
+            scanned += idx->last_scanned;
+        }
+        idx->last_scanned = scanned;
+        return BV_OK;
+    }
     if ((idx->codec == C_Q8 || idx->codec == C_Q4 || idx->codec == C_HAM || idx->codec == C_Q1P ||
          idx->codec == C_Q1A) &&
         idx->rows > MQ_SAMPLE)
         return run_batched_q8(idx, d_q, nq, kprime, k_out, rerank, d_rows, d_scores, d_n);
-    const unsigned char *qscan = (const unsigned char *)d_q;  // fp32 rows: the queries as they are
-    uint64_t qstride = (uint64_t)idx->dim * 4;
-    int rc = BV_OK;
-    if (idx->quant) {
-        rc = prepare_levels16(idx, d_q, nq, &qscan, &qstride);
-        if (rc) return rc;
-    }
+    const unsigned char *qscan = nullptr;
+    uint64_t qstride = 0;
+    int rc = prepare_levels16(idx, d_q, nq, &qscan, &qstride);
+    if (rc) return rc;
     const uint64_t N = idx->rows;
     const uint64_t S = std::min<uint64_t>(N, MQ_SAMPLE);
     const bool one_pass = S == N;
@@ -2175,10 +2164,10 @@ static int run_batched(bv_index *idx, const float *d_q, uint32_t nq, uint32_t kp
     HIPX(idx->dev, idx->merged_n.ensure((size_t)nq * 4, 0, idx->stream), "scratch");
 
     MqArgs m{};
-    m.codes = idx->quant ? idx->codes.as<uint32_t>() : idx->raw.as<uint32_t>();
+    m.codes = idx->codes.as<uint32_t>();
     m.scales = idx->scales.as<float>();
-    m.W = idx->quant ? idx->words_per_row : idx->dim;
-    m.units = idx->quant ? idx->P / 16 : idx->dim / 8;
+    m.W = idx->words_per_row;
+    m.units = idx->P / 16;
     m.bits = idx->codec == C_Q4 ? 4 : 8;
     m.scale_mul = idx->codec == C_Q4 ? 1.0f / 7.0f : 1.0f;
     m.qlev = qscan;
@@ -2202,7 +2191,7 @@ static int run_batched(bv_index *idx, const float *d_q, uint32_t nq, uint32_t kp
     m.row_step = N / S;
     m.tau = nullptr;
     HIPX(idx->dev, hipMemsetD32Async((hipDeviceptr_t)idx->mq_cnt.p, (int)S, nq, idx->stream), "scratch");
-    HIPX(idx->dev, idx->quant ? launch_mq_scan(m, idx->stream) : launch_mq_scan_f32(m, idx->stream),
+    HIPX(idx->dev, launch_mq_scan(m, idx->stream),
          "batched scan kernel");
     if (!one_pass) {
         sa.tau = idx->mq_tau.as<uint64_t>();
@@ -2211,7 +2200,7 @@ static int run_batched(bv_index *idx, const float *d_q, uint32_t nq, uint32_t kp
         m.n = N;
         m.row_step = 1;
         m.tau = idx->mq_tau.as<uint64_t>();
-        HIPX(idx->dev, idx->quant ? launch_mq_scan(m, idx->stream) : launch_mq_scan_f32(m, idx->stream),
+        HIPX(idx->dev, launch_mq_scan(m, idx->stream),
          "batched scan kernel");
         sa.tau = nullptr;
     }
@@ -2400,7 +2389,10 @@ static int run_ivf_batched(bv_index *idx, const float *d_q, uint32_t nq, uint32_
 //     0.24 us per million codes whatever the batch, a slot scan 45 us and a
 //     time per query, row and 16-byte unit set by its dot products (below):
 //     1M x 768 int8 crosses between 4 and 5 queries, 100,000 x 384 at 40,
-//     20,000 x 300 at 140.
+//     20,000 x 300 at 140;
+//   fp32 batches cost 0.62 us per million elements on top: 100,000 x 384
+//     crosses at 20 (16 queries 129 / 161, 32 183 / 165), 20,000 x 384 at 75
+//     (64 queries 119 / 132).
 static bool slots_route(const bv_index *idx, uint32_t nq, uint32_t kprime, bool rerank, bool batchable) {
     if (idx->ivf || idx->rows == 0 || idx->rows >= (1ull << 30)) return false;
     if (!pick_supported(idx->codec, idx->P, rerank ? idx->dim : 0)) return false;
@@ -2420,8 +2412,7 @@ static bool slots_route(const bv_index *idx, uint32_t nq, uint32_t kprime, bool 
     }
     const double mrows = (double)idx->rows * 1e-6;
     const double slots = 45.0 + (double)nq * mrows * idx->units * per;
-    const double batch = idx->quant ? 140.0 + 0.24 * mrows * idx->P
-                                    : 120.0 + 0.82 * mrows * idx->dim * std::max(1.0, (double)nq / 48.0);
+    const double batch = idx->quant ? 140.0 + 0.24 * mrows * idx->P : 140.0 + 0.62 * mrows * idx->dim;
     return slots < batch;
 }
 
@@ -3459,7 +3450,7 @@ extern "C" int bv_index_load_section(bv_index *idx, const float *data, uint64_t 
     // every allocation first, so a failure leaves the index empty
     const size_t rb = (size_t)idx->dim * 4;
     hipStream_t s = idx->stream;
-    HIPX(idx->dev, idx->raw.ensure(std::max<uint64_t>(count, 1) * rb, 0, s), "row buffer");
+    HIPX(idx->dev, idx->raw.ensure(std::max<uint64_t>(count, 1) * rb + 16, 0, s), "row buffer");
     const bool norms = !idx->quant && !idx->ivf;
     const bool code_norms = idx->codec == C_Q8 && !idx->ivf;
     if (norms) HIPX(idx->dev, idx->rsq.ensure(std::max<uint64_t>(count, 1) * 4, 0, s), "norm buffer");
@@ -3486,7 +3477,7 @@ extern "C" int bv_index_load_section(bv_index *idx, const float *data, uint64_t 
     }
     if (norms)
         HIPX(idx->dev, launch_row_sqnorms(idx->raw.as<float>(), count, idx->dim, idx->rsq.as<float>(),
-                                          idx->rsq_max.as<uint32_t>(), s),
+                                          idx->bf16_ratio.as<uint32_t>(), s),
              "norm kernel");
     if (code_norms)
         HIPX(idx->dev, launch_row_code_norms(idx->codes.as<uint32_t>(), count, idx->words_per_row,

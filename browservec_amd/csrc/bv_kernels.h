@@ -377,26 +377,46 @@ struct MqArgs {
     uint64_t *cand;           // [nq][cap]
     uint32_t *cnt;            // [nq] appended keys (threshold pass)
     uint64_t cap;
-    // fp32 rows only.  l2: score 2 x.q - |x|^2 - |q|^2 (rsq per row, qsq per
-    // query) instead of x.q.  rows_out: the threshold pass appends the ids of
-    // rows whose score reaches tau's score minus slack[q] ([nq][cap] u32)
-    // instead of keys: a superset of the rows that can rank in the exact scan.
-    int l2;
-    const float *rsq;
-    const float *qsq;
-    const float *slack;
-    uint32_t *rows_out;
 };
-// Per-row squared norms of fp32 rows (f64 sums rounded to f32) and, in
-// *max_bits, the largest of them (float bits, rounded up; rsq >= 0 so the
-// bits order like the values).
-hipError_t launch_row_sqnorms(const float *rows, uint64_t n, uint32_t dim, float *rsq, uint32_t *max_bits,
+// Per-row squared norms of fp32 rows (f64 sums rounded to f32) and, raised in
+// *ratio_bits, the largest |x - bf16(x)| / |x| of the rows (float bits, rounded
+// up; the ratios are >= 0, so the bits order like the values).
+hipError_t launch_row_sqnorms(const float *rows, uint64_t n, uint32_t dim, float *rsq, uint32_t *ratio_bits,
                               hipStream_t s);
-// Per-query constants of the exact fp32 batch: qsq = |q|^2 and the slack
-// 2E, where E bounds |matrix-core score - single-query score| for every row:
-// dot 3(dim+2)u |x|max |q|, l2 4(dim+4)u (|x|max + |q|)^2 (u = 2^-24).
-hipError_t launch_mq_f32_qconst(const float *q, uint32_t nq, uint32_t dim, const uint32_t *max_bits, int l2,
-                                float *qsq, float *slack, hipStream_t s);
+// The bf16 prefilter of fp32 batches (mqf_scan): bounds s +- E of every row's
+// score, E = alpha |x| + beta + gamma |x|^2 per query.
+struct MqfQuery {
+    float alpha, beta, gamma;
+    float qsq;                // |q|^2 (l2: s = 2 x.q - |x|^2 - |q|^2)
+};
+struct MqfArgs {
+    const float *rows;        // logical row i at rows + i * row_step * dim (the buffer goes on for 12 bytes) ...
+    const float *rsq;         // ... its squared norm at rsq[i * row_step] ...
+    uint32_t dim;
+    int l2;
+    uint64_t n;               // logical rows in this pass
+    uint64_t row_step;
+    uint64_t row_base;        // ... and its row in the keys row_base + i * row_step
+    const unsigned char *qbf; // nq bf16 queries, qstride bytes apart (launch_mqf_prep)
+    uint64_t qstride;         // mqf_qstride(dim)
+    const MqfQuery *qk;
+    uint32_t nq;
+    uint32_t qblocks;         // ceil(nq / mqf_block(dim))
+    uint32_t nwg;             // workgroups per query block (a multiple of 8)
+    const uint64_t *tau;      // null: dense pass; else [nq] bound keys; outputs as in Mq1Args
+    uint64_t *cand;
+    uint32_t *up_out;
+    uint32_t *cnt;
+    uint64_t cap;
+    uint32_t capw;
+};
+bool mqf_supported(uint32_t dim);
+uint32_t mqf_block(uint32_t dim);    // queries per workgroup
+uint64_t mqf_qstride(uint32_t dim);
+// Queries to bf16 and their constants; cnt (if given) is filled with cnt_value.
+hipError_t launch_mqf_prep(const float *q, uint32_t nq, uint32_t dim, const uint32_t *ratio_bits, bool l2,
+                           unsigned char *qbf, MqfQuery *qk, uint32_t *cnt, uint32_t cnt_value, hipStream_t s);
+hipError_t launch_mqf_scan(const MqfArgs &a, hipStream_t s);
 // Per query: the best kk keys of cand[q][0, min(cnt[q], cap)).  Outputs are
 // optional: tau = the kk-th best key (0 when there are kk or fewer), the
 // selected keys (merged, merged_n), overflow = cnt[q] > cap, and the selected
@@ -506,11 +526,6 @@ hipError_t launch_mq1_qconst_l1(const float *qrot, uint32_t P, const unsigned ch
                                 hipStream_t s);
 hipError_t launch_mq1_scan(const Mq1Args &a, hipStream_t s);
 hipError_t launch_mq_scan(const MqArgs &a, hipStream_t s);
-// fp32 rows (dot / cosine): a.codes = the rows, a.W = dim, a.units = dim / 8,
-// a.qlev = fp32 queries (a.qstride bytes apart).  Dimensions 32 .. 1024 in
-// the set mq_f32_supported accepts (32 queries of up to 1024 floats stay in LDS).
-bool mq_f32_supported(uint32_t dim);
-hipError_t launch_mq_scan_f32(const MqArgs &a, hipStream_t s);
 hipError_t launch_mq_rerank(const MqRerankArgs &a, uint32_t nq, hipStream_t s);
 hipError_t launch_mq_select(const MqSelArgs &a, uint32_t nq, hipStream_t s);
 

@@ -9,13 +9,6 @@
 //                distanceQ4 dispatches + score buffers for query batches
 //                (src/engine/wgsl/distanceQ8.ts:56-82, distanceQ4.ts:44-78,
 //                src/index/quant.ts:178-245, src/index.ts:473-517).
-//   mq_scan_f32  fp32 rows x fp32 queries (dot / cosine / l2) on
-//                v_mfma_f32_32x32x2f32 (src/engine/wgsl/distance.ts:24-177,
-//                src/index/flat.ts:132-200 for query batches).  Its scores
-//                are within a proven bound of the single-query scan's, and
-//                serve as a prefilter: the rows that can rank are re-scored
-//                by the single-query scan's own arithmetic, so a batch
-//                returns exactly the single-query results.
 //   mq_select    exact selection of each query's best kk keys.
 //   mq_rerank    exact f64 re-rank of the selected candidates, 16 per wave.
 //
@@ -212,18 +205,6 @@ struct Mq1Stage {
     uint16_t ln[2][MQ_WAVES][64];          // entries of each lane
     uint8_t qovf[MQ1_QB];                  // a query's entries did not all fit
 };
-
-// Inclusive prefix sum over the wave's 64 lanes in VALU (DPP row shifts
-// within rows of 16, then the row broadcasts), no LDS traffic.
-__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x) {
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false);  // row_shr:1
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false);  // row_shr:2
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false);  // row_shr:4
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false);  // row_shr:8
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false);  // row_bcast:15
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false);  // row_bcast:31
-    return x;
-}
 
 // Keys of one wave's 32 queries x the tile's MQ1_ROWS (32) rows.  Dense
 // pass: the lower-bound key of every (row, query) (a NaN bound as order 0,
@@ -1156,228 +1137,6 @@ __global__ __launch_bounds__(1024) void mq1_compact(const uint64_t *bk, const ui
     if (tid == 0) cnt[q] = total;
 }
 
-// fp32 rows x fp32 queries on v_mfma_f32_32x32x2f32: the batched
-// counterpart of the fp32 flat scan.  Same structure as mq_scan: the block's
-// 32 queries stay in LDS, each wave streams 64 rows.  Lane l = 32h + c
-// supplies, over the four MFMA steps of chunk t, elements 8t + 4h .. 8t +
-// 4h + 3 of row c (A) and of query c (B), one 16-byte load each, so both
-// operands pair the same elements.  The sum runs in the matrix core's own
-// order, so a score differs from the single-query scan's by rounding only:
-// at most E (launch_mq_f32_qconst) for every row.  l2 scores are
-// 2 x.q - |x|^2 - |q|^2 from the rows' and queries' squared norms.
-// a.W = dim (floats per row), a.units = dim / 8 chunks, a.qlev = the fp32
-// queries, a.qstride their byte stride.
-//
-// Passes: dense (every key of logical row i at cand[q][i]); threshold with
-// keys (append keys at or above tau[q]); threshold with row ids (rows_out:
-// append every row whose score reaches tau's score minus slack[q], which
-// keeps every row the exact scan can rank: a row in the exact top-kk has
-// single-query score >= the kk-th best single-query score >= tau's score
-// - E, hence matrix-core score >= tau's score - 2E).
-template <int CHUNKS>
-__global__ __launch_bounds__(MQ_WAVES * 64) void mq_scan_f32(MqArgs a) {
-    constexpr int G = CHUNKS < 4 ? CHUNKS : 4;
-    __shared__ float4 qlds[CHUNKS][64];
-    __shared__ uint64_t qtau[MQ_QB];
-    __shared__ float qts[MQ_QB];
-    __shared__ float qn2[MQ_QB];
-    __shared__ float rn2[MQ_WAVES][64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int h = lane >> 5, c = lane & 31;
-    const uint32_t b = blockIdx.x, xcd = b & 7u, slot = b >> 3;
-    const uint32_t qb = slot % a.qblocks, grp = slot / a.qblocks;
-    const uint64_t tstride = 8ull * a.groups;
-    uint64_t tile = xcd + 8ull * grp;
-    if (tile * MQ_ROWS >= a.n) return;
-    {
-        uint32_t q = qb * MQ_QB + c;
-        if (q >= a.nq) q = a.nq - 1;
-        const float *src = (const float *)(a.qlev + (uint64_t)q * a.qstride);
-        for (int t = wave; t < CHUNKS; t += MQ_WAVES)
-            __builtin_amdgcn_global_load_lds((glb_void *)(src + 8 * t + 4 * h), (lds_void *)&qlds[t][0], 16, 0, 0);
-    }
-    if (threadIdx.x < MQ_QB) {
-        uint32_t q = qb * MQ_QB + threadIdx.x;
-        if (q >= a.nq) q = a.nq - 1;
-        const uint64_t t = a.tau ? a.tau[q] : 0ull;
-        qtau[threadIdx.x] = t;
-        float ts = t ? f32_from_ord((uint32_t)(t >> 32)) : -__builtin_inff();
-        if (a.rows_out && t) {
-            // tau's score minus the slack, rounded down
-            const float r = (float)((double)ts - (double)a.slack[q]);
-            ts = next_down(r);
-        }
-        qts[threadIdx.x] = ts;
-        qn2[threadIdx.x] = a.l2 ? a.qsq[q] : 0.0f;
-    }
-    auto row_sq = [&](uint64_t t) {
-        uint64_t li = t * MQ_ROWS + (uint64_t)wave * 64 + lane;
-        if (li >= a.n) li = a.n - 1;
-        return a.rsq[li * a.row_step];
-    };
-    float rsq_next = a.l2 ? row_sq(tile) : 0.0f;
-    auto row_ptrs = [&](uint64_t t, const float4 *(&ap)[2]) {
-        const uint64_t w0 = t * MQ_ROWS + (uint64_t)wave * 64;
-#pragma unroll
-        for (int fr = 0; fr < 2; ++fr) {
-            uint64_t li = w0 + fr * 32 + c;
-            if (li >= a.n) li = a.n - 1;  // rows past the end load a valid row; their results are dropped
-            ap[fr] = (const float4 *)((const float *)a.codes + li * a.row_step * a.W + 4 * h);
-        }
-    };
-    const float4 *ap[2];
-    row_ptrs(tile, ap);
-    float4 ring[2][G][2];
-#pragma unroll
-    for (int j = 0; j < G; ++j)
-#pragma unroll
-        for (int fr = 0; fr < 2; ++fr) ring[0][j][fr] = ap[fr][2 * j];
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-
-    const uint32_t q = qb * MQ_QB + c;
-    const bool qok = q < a.nq;
-    const uint32_t qq = qok ? q : a.nq - 1;
-    uint64_t *out = a.cand + (uint64_t)qq * a.cap;
-    for (;;) {
-        const uint64_t ntile = tile + tstride;
-        const bool more = ntile * MQ_ROWS < a.n;
-        const float4 *np[2];
-        row_ptrs(more ? ntile : tile, np);
-        v16f acc[2] = {v16f{}, v16f{}};
-#pragma unroll
-        for (int t = 0; t < CHUNKS; ++t) {
-            const int gp = (t / G) & 1, j = t % G;
-            if (j == 0) {
-                const int nt = t + G;
-#pragma unroll
-                for (int jj = 0; jj < G; ++jj)
-#pragma unroll
-                    for (int fr = 0; fr < 2; ++fr) {
-                        if (nt < CHUNKS) ring[gp ^ 1][jj][fr] = ap[fr][2 * (nt + jj)];
-                        else if (more) ring[gp ^ 1][jj][fr] = np[fr][2 * (nt - CHUNKS + jj)];
-                    }
-            }
-            const float4 B = qlds[t][lane];
-            const float bv[4] = {B.x, B.y, B.z, B.w};
-#pragma unroll
-            for (int fr = 0; fr < 2; ++fr) {
-                const float4 A = ring[gp][j][fr];
-                const float av[4] = {A.x, A.y, A.z, A.w};
-#pragma unroll
-                for (int e = 0; e < 4; ++e) acc[fr] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[e], bv[e], acc[fr], 0, 0, 0);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        if constexpr ((CHUNKS / G) & 1) {
-#pragma unroll
-            for (int j = 0; j < G; ++j)
-#pragma unroll
-                for (int fr = 0; fr < 2; ++fr) ring[0][j][fr] = ring[1][j][fr];
-        }
-        // l2: the score from the dot and the squared norms (this wave's 64
-        // rows' norms through wave-private LDS)
-        if (a.l2) {
-            rn2[wave][lane] = rsq_next;
-            if (more) rsq_next = row_sq(ntile);
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-            const float qs2 = qn2[c];
-#pragma unroll
-            for (int fr = 0; fr < 2; ++fr)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const float x2 = rn2[wave][fr * 32 + 8 * (r >> 2) + 4 * h + (r & 3)];
-                    acc[fr][r] = 2.0f * acc[fr][r] - x2 - qs2;
-                }
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        }
-        // keys: dense (logical row i at out[i]), appended at or above tau, or
-        // row ids appended at or above the slackened bound
-        const uint64_t w0 = tile * MQ_ROWS + (uint64_t)wave * 64;
-        const bool full = w0 + 64 <= a.n;
-        if (a.rows_out) {
-            const float ts = qts[c];
-            uint32_t pass = 0;
-#pragma unroll
-            for (int fr = 0; fr < 2; ++fr)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const uint64_t li = w0 + fr * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
-                    // a NaN score passes: the exact scan ranks it as it ranks any key
-                    if (qok && (full || li < a.n) && !(acc[fr][r] < ts)) pass |= 1u << (fr * 16 + r);
-                }
-            if (__ballot(pass != 0)) {
-                const uint32_t mine = __popc(pass);
-                const uint32_t other = __shfl_xor(mine, 32);
-                uint32_t base = 0;
-                if (h == 0 && mine + other) base = atomicAdd(&a.cnt[qq], mine + other);
-                base = __shfl(base, c);
-                if (pass) {
-                    uint32_t *ro = a.rows_out + (uint64_t)qq * a.cap;
-                    uint64_t pos = (uint64_t)base + (h ? other : 0u);
-#pragma unroll
-                    for (int fr = 0; fr < 2; ++fr)
-#pragma unroll
-                        for (int r = 0; r < 16; ++r)
-                            if (pass & (1u << (fr * 16 + r))) {
-                                const uint64_t li = w0 + fr * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
-                                if (pos < a.cap) ro[pos] = (uint32_t)(li * a.row_step);
-                                ++pos;
-                            }
-                }
-            }
-        } else if (!a.tau) {
-#pragma unroll
-            for (int fr = 0; fr < 2; ++fr)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const uint64_t li = w0 + fr * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
-                    if (qok && (full || li < a.n)) out[li] = make_key(ord_f32(acc[fr][r]), (uint32_t)(li * a.row_step));
-                }
-        } else {
-            const uint64_t tau = qtau[c];
-            const float ts = qts[c];
-            uint32_t pass = 0;
-#pragma unroll
-            for (int fr = 0; fr < 2; ++fr)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const float sc = acc[fr][r];
-                    if (!(sc < ts)) {
-                        const uint64_t li = w0 + fr * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
-                        if (qok && (full || li < a.n) && make_key(ord_f32(sc), (uint32_t)(li * a.row_step)) >= tau)
-                            pass |= 1u << (fr * 16 + r);
-                    }
-                }
-            if (__ballot(pass != 0)) {
-                const uint32_t mine = __popc(pass);
-                const uint32_t other = __shfl_xor(mine, 32);
-                uint32_t base = 0;
-                if (h == 0 && mine + other) base = atomicAdd(&a.cnt[qq], mine + other);
-                base = __shfl(base, c);
-                if (pass) {
-                    uint64_t pos = (uint64_t)base + (h ? other : 0u);
-#pragma unroll
-                    for (int fr = 0; fr < 2; ++fr)
-#pragma unroll
-                        for (int r = 0; r < 16; ++r)
-                            if (pass & (1u << (fr * 16 + r))) {
-                                const uint64_t li = w0 + fr * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
-                                if (pos < a.cap) out[pos] = make_key(ord_f32(acc[fr][r]), (uint32_t)(li * a.row_step));
-                                ++pos;
-                            }
-                }
-            }
-        }
-        if (!more) break;
-        ap[0] = np[0];
-        ap[1] = np[1];
-        tile = ntile;
-    }
-}
-
 // One workgroup per query.  The kk-th best key is found by binning the
 // keys over their actual range (2048 bins of a power-of-two width, so keys
 // concentrated in a few score octaves still spread over many bins) and
@@ -1608,49 +1367,6 @@ __global__ __launch_bounds__(RR_THREADS) void mq_rerank(MqRerankArgs a) {
 }
 
 namespace {
-
-// One wave per row: f64 sum of squares in element order, rounded to f32.
-__global__ __launch_bounds__(256) void row_sqnorms(const float *rows, uint64_t n, uint32_t dim, float *rsq,
-                                                   uint32_t *max_bits) {
-    const int lane = threadIdx.x & 63;
-    const uint64_t nw = (uint64_t)gridDim.x * 4;
-    uint32_t mx = 0;
-    for (uint64_t r = (uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6); r < n; r += nw) {
-        const float *x = rows + r * dim;
-        double s = 0.0;
-        for (uint32_t i = lane; i < dim; i += 64) s = fma((double)x[i], (double)x[i], s);
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) s += __shfl_xor(s, o);
-        if (lane == 0) {
-            rsq[r] = (float)s;
-            // the bound uses a value no smaller than any row's: round up
-            const float up = next_up((float)s);
-            const uint32_t b = __float_as_uint(up);
-            mx = b > mx ? b : mx;
-        }
-    }
-    if (lane == 0 && mx) atomicMax(max_bits, mx);
-}
-
-// One wave per query: |q|^2 and the slack 2E of the exact fp32 batch.
-__global__ __launch_bounds__(64) void mq_f32_qconst(const float *q, uint32_t dim, const uint32_t *max_bits, int l2,
-                                                    float *qsq, float *slack) {
-    const int lane = threadIdx.x;
-    const float *x = q + (uint64_t)blockIdx.x * dim;
-    double s = 0.0;
-    for (uint32_t i = lane; i < dim; i += 64) s = fma((double)x[i], (double)x[i], s);
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) s += __shfl_xor(s, o);
-    if (lane == 0) {
-        const double u = 0x1p-24;
-        const double xn = sqrt((double)__uint_as_float(*max_bits)) * (1.0 + 0x1p-20);
-        const double qn = sqrt(s) * (1.0 + 0x1p-20);
-        const double e = l2 ? 4.0 * (dim + 4) * u * (xn + qn) * (xn + qn) : 3.0 * (dim + 2) * u * xn * qn;
-        qsq[blockIdx.x] = (float)s;
-        // 2E plus room for the subnormal products a matrix core may flush
-        slack[blockIdx.x] = (float)((2.0 * e + dim * 0x1p-126) * (1.0 + 0x1p-10));
-    }
-}
 
 // One wave per row: |c|_2 of the int8 codes, rounded up to f32 (the exact
 // sum of squares from v_dot4 of each word with itself, below 2^24; f64
@@ -2414,22 +2130,6 @@ hipError_t launch_mq1_scan(const Mq1Args &a, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_row_sqnorms(const float *rows, uint64_t n, uint32_t dim, float *rsq, uint32_t *max_bits,
-                              hipStream_t s) {
-    if (n == 0) return hipSuccess;
-    uint64_t blocks = (n + 3) / 4;
-    if (blocks > 65536) blocks = 65536;
-    hipLaunchKernelGGL(row_sqnorms, dim3((uint32_t)blocks), dim3(256), 0, s, rows, n, dim, rsq, max_bits);
-    return hipGetLastError();
-}
-
-hipError_t launch_mq_f32_qconst(const float *q, uint32_t nq, uint32_t dim, const uint32_t *max_bits, int l2,
-                                float *qsq, float *slack, hipStream_t s) {
-    if (nq == 0) return hipSuccess;
-    hipLaunchKernelGGL(mq_f32_qconst, dim3(nq), dim3(64), 0, s, q, dim, max_bits, l2, qsq, slack);
-    return hipGetLastError();
-}
-
 hipError_t launch_mq_scan(const MqArgs &a, hipStream_t s) {
     if (a.n == 0 || a.nq == 0) return hipSuccess;
     const uint32_t steps = a.units >> 1;
@@ -2455,37 +2155,6 @@ hipError_t launch_mq_scan(const MqArgs &a, hipStream_t s) {
     default: return hipErrorInvalidValue;
     }
 #undef BV_MQ_CASE
-    return hipGetLastError();
-}
-
-bool mq_f32_supported(uint32_t dim) {
-    switch (dim) {
-    case 32: case 64: case 96: case 128: case 192: case 256: case 384: case 512: case 768: case 1024: return true;
-    default: return false;
-    }
-}
-
-hipError_t launch_mq_scan_f32(const MqArgs &a, hipStream_t s) {
-    if (a.n == 0 || a.nq == 0) return hipSuccess;
-    if (!mq_f32_supported(a.W) || a.units * 8 != a.W || a.qblocks == 0 || a.groups == 0 ||
-        (uint64_t)a.qblocks * MQ_QB < a.nq)
-        return hipErrorInvalidValue;
-    const uint64_t blocks = 8ull * a.groups * a.qblocks;
-    if (blocks > 0x7fffffffull) return hipErrorInvalidValue;
-    const dim3 g((uint32_t)blocks), wg(MQ_WAVES * 64);
-    switch (a.units) {
-    case 4: hipLaunchKernelGGL(mq_scan_f32<4>, g, wg, 0, s, a); break;
-    case 8: hipLaunchKernelGGL(mq_scan_f32<8>, g, wg, 0, s, a); break;
-    case 12: hipLaunchKernelGGL(mq_scan_f32<12>, g, wg, 0, s, a); break;
-    case 16: hipLaunchKernelGGL(mq_scan_f32<16>, g, wg, 0, s, a); break;
-    case 24: hipLaunchKernelGGL(mq_scan_f32<24>, g, wg, 0, s, a); break;
-    case 32: hipLaunchKernelGGL(mq_scan_f32<32>, g, wg, 0, s, a); break;
-    case 48: hipLaunchKernelGGL(mq_scan_f32<48>, g, wg, 0, s, a); break;
-    case 64: hipLaunchKernelGGL(mq_scan_f32<64>, g, wg, 0, s, a); break;
-    case 96: hipLaunchKernelGGL(mq_scan_f32<96>, g, wg, 0, s, a); break;
-    case 128: hipLaunchKernelGGL(mq_scan_f32<128>, g, wg, 0, s, a); break;
-    default: return hipErrorInvalidValue;
-    }
     return hipGetLastError();
 }
 

@@ -1,0 +1,82 @@
+"""GPU tests of the bf16 prefilter of fp32 query batches: batches return the
+rows and score bits of single queries at every edge of its tiles (32 rows, 128
+dimensions, 16-byte pieces, 256 or 128 queries), and rows and queries that its
+bounds say nothing about are kept."""
+import numpy as np
+import pytest
+
+from tests.helpers import need_gpu, say
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    need_gpu()
+    from browservec_amd import DeviceContext
+
+    c = DeviceContext(0)
+    yield c
+    c.destroy()
+
+
+def same_as_singles(idx, qs, k, which):
+    batch = idx.query_batch(qs, len(qs), k)
+    for i in which:
+        one = idx.query(qs[i], k)
+        assert [h.row for h in batch[i]] == [h.row for h in one], i
+        a = np.float32([h.score for h in batch[i]]).view(np.uint32)
+        assert np.array_equal(a, np.float32([h.score for h in one]).view(np.uint32)), i
+
+
+@pytest.mark.parametrize("metric,dim,n,nq", [
+    ("cosine", 5, 1_000_000, 300), ("l2", 31, 200_001, 257), ("cosine", 127, 60_000, 300),
+    ("l2", 129, 60_033, 300), ("dot", 300, 40_000, 256), ("cosine", 383, 16_385, 300),
+    ("l2", 514, 20_000, 300), ("cosine", 767, 20_001, 260), ("l2", 768, 20_031, 300),
+    ("dot", 769, 20_000, 129), ("cosine", 1001, 20_000, 300), ("l2", 1024, 16_400, 130),
+])
+def test_batches_equal_singles(ctx, metric, dim, n, nq):
+    from browservec_amd import FlatIndex
+
+    say("bf16 prefilter", metric, dim, n, nq)
+    rng = np.random.default_rng(dim)
+    data = rng.standard_normal((n, dim), dtype=np.float32)
+    data *= rng.uniform(0.5, 2.0, (n, 1)).astype(np.float32)
+    idx = FlatIndex(ctx, dim, metric)
+    idx.append(data[: n // 3], n // 3)
+    idx.append(data[n // 3:], n - n // 3)
+    qs = (data[rng.integers(0, n, nq)] + 0.3 * rng.standard_normal((nq, dim))).astype(np.float32)
+    same_as_singles(idx, qs, 10, (0, 31, 32, 127, 128, nq // 2, nq - 1))
+    idx.destroy()
+
+
+@pytest.mark.parametrize("metric", ["dot", "l2"])
+def test_rows_and_queries_without_bounds(ctx, metric):
+    """Rows and queries whose squares or products leave the range of f32, that
+    are not finite, zero or subnormal; 1001 dimensions, so that a row's last
+    piece also holds elements of the next row."""
+    from browservec_amd import FlatIndex
+
+    dim, n, nq = 1001, 17_000, 140
+    say("bf16 prefilter out of range", metric)
+    rng = np.random.default_rng(9)
+    data = rng.standard_normal((n, dim), dtype=np.float32)
+    data[5] = 0
+    data[6] *= np.float32(1e-42)
+    data[7] *= np.float32(1e-20)
+    data[100, 3] = np.inf
+    data[101, 0] = -np.inf
+    data[8000, 1000] = np.float32(3e38)
+    data[9000, 0] = np.nan
+    data[16_999, 7] = np.float32(2e19)
+    idx = FlatIndex(ctx, dim, metric)
+    idx.append(data, n)
+    qs = rng.standard_normal((nq, dim), dtype=np.float32)
+    qs[1] = 0
+    qs[2] *= np.float32(1e-42)
+    qs[3] *= np.float32(1e-20)
+    qs[4, 9] = np.float32(3e38)
+    qs[5, 0] = np.inf
+    qs[6] *= np.float32(1e18)
+    same_as_singles(idx, qs, 10, range(8))
+    idx.destroy()
