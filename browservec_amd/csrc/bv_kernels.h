@@ -574,7 +574,7 @@ hipError_t launch_ivf_pairs(const uint32_t *probes, uint32_t nq, uint32_t nprobe
 hipError_t launch_ivf_pair_scatter(const uint32_t *probes, const uint32_t *base, uint32_t npairs, uint32_t nprobe,
                                    const uint32_t *pair_off, uint32_t *fill, uint32_t *pair_q, uint32_t *pair_base,
                                    hipStream_t s);
-// chunks[c]: list c's work items (8 of its queries each).
+// chunks[c]: list c's work items (16 of its queries each).
 hipError_t launch_ivf_chunk_counts(const uint32_t *pair_count, uint32_t nlist, uint32_t *chunks, hipStream_t s);
 // Every probed list's rows scored once per work item (chunk_off: exclusive
 // scan of chunks): the single-query scan's key at cand[q * cap + base + i].

@@ -1681,7 +1681,8 @@ __global__ __launch_bounds__(256) void ivf_pair_scatter(const uint32_t *probes, 
 // queries probing it, the single-query scan's key (the three levels' exact
 // int32 dots, combined in f64) written at the row's candidate position of
 // each query.
-constexpr int IVF_QC = 8;
+constexpr int IVF_QG = 8;            // queries whose three levels fill one 32-column operand
+constexpr int IVF_QC = 2 * IVF_QG;
 // chunks[c] = the list's work items (IVF_QC queries each).
 __global__ __launch_bounds__(256) void ivf_chunk_counts(const uint32_t *pair_count, uint32_t nlist, uint32_t *chunks) {
     const uint32_t c = blockIdx.x * 256 + threadIdx.x;
@@ -1691,15 +1692,28 @@ __global__ __launch_bounds__(256) void ivf_chunk_counts(const uint32_t *pair_cou
 // One workgroup per work item: a list and up to IVF_QC of the queries
 // probing it (chunk_off = exclusive scan of the lists' item counts), so a
 // list probed by many queries spreads over many workgroups.  The work runs
-// on v_mfma_i32_32x32x32_i8: IVF_LM_WAVES waves per workgroup,
-// each taking 32-row tiles of the list.  B holds 24 columns, level l of
-// query k at column 8l + k (columns 24-31 and missing queries are zero),
+// on v_mfma_i32_32x32x32_i8: IVF_LM_WAVES waves per workgroup, each taking
+// 32-row tiles of the list.  B holds 24 columns, level l of query k of a group
+// of eight at column 8l + k (columns 24-31 and missing queries are zero),
 // staged in LDS by 16-byte unit so lane (c, h) reads column c at unit
 // 2 * step + h; A is row c of the tile at the same unit (int4 rows unpacked
-// to n ^ 8 bytes).  The int32 dots are exact; the three level dots of a
-// (row, query) meet in a per-wave LDS tile and q_key combines them in f64,
-// giving the single-query scan's key.
-constexpr uint32_t IVF_LM_WAVES = 4;  // eight measured slower for int8 rows (1.58 ms against 1.35 ms at 4M x 768)
+// to n ^ 8 bytes), read once for both groups.  The int32 dots are exact; the
+// three level dots of a (row, query) meet in a per-wave LDS tile and q_key
+// combines them in f64, giving the single-query scan's key.
+//
+// Rows come through LDS in chunks of 256 bytes a row, in a ring of its own
+// for each wave (no barrier), four chunks in flight (128 KB per CU): a load
+// instruction takes whole 256-byte pieces of four rows, pieces of 16 bytes
+// stored at piece ^ row.  The operands of the queries stay in registers, and
+// the row ids and scales of up to IVF_LM_IDS rows are staged first, so that
+// nothing else waits on memory in between.
+// Bound by the gather of rows (1 KB each, in the order of the lists, out of
+// the order of the index): 4M x 768, 1,024 queries, 32 of 4,096 lists, 4.1 GB
+// of rows read: 920 us, 4.5 TB/s.  With the rows straight into registers for
+// eight queries at a time it took 1,150 us, for sixteen 1,078, with two
+// chunks in flight and the queries' operands in LDS 975.
+constexpr uint32_t IVF_LM_WAVES = 4;
+constexpr uint32_t IVF_LM_IDS = 1024;
 template <int UNITS, int BITS>
 __global__ __launch_bounds__(IVF_LM_WAVES * 64) void ivf_list_mfma(const uint32_t *codes, const float *scales, float scale_mul,
                                                      const uint32_t *list_off, const uint32_t *list_rows,
@@ -1708,20 +1722,31 @@ __global__ __launch_bounds__(IVF_LM_WAVES * 64) void ivf_list_mfma(const uint32_
                                                      const uint32_t *pair_q, const uint32_t *pair_base,
                                                      const unsigned char *qlev, uint64_t qstride, uint64_t *cand,
                                                      uint64_t cap) {
-    static_assert(IVF_QC == 8 && UNITS % 2 == 0, "24 columns: three levels of eight queries");
-    constexpr int S = UNITS / 2;                 // K steps of 32 codes
-    constexpr uint32_t W = UNITS * BITS / 2;     // words per row
-    __shared__ v4i bq[S][2][32];
+    static_assert(IVF_QG == 8 && UNITS % 2 == 0, "24 columns: three levels of eight queries");
+    constexpr int S = UNITS / 2;                  // K steps of 32 codes
+    constexpr uint32_t RB = UNITS * BITS * 2;     // bytes per row
+    constexpr uint32_t CB = RB < 256 ? RB : 256;  // bytes of a row per chunk
+    constexpr uint32_t UC = CB / 16;              // 16-byte pieces
+    constexpr int NC = RB / CB, SC = S / NC;      // chunks per row, K steps per chunk
+    constexpr int PW = UC > 2 ? UC / 2 : 1;       // loads per chunk
+    constexpr uint32_t SLOT = 32 * CB < 1024 ? 1024 : 32 * CB;
+    constexpr uint32_t RD = 4;                    // ring of chunks
+    __shared__ __align__(1024) unsigned char ring[IVF_LM_WAVES][RD][SLOT];
     __shared__ int32_t stg[IVF_LM_WAVES][32][25];  // per wave: 32 rows x 24 columns (+1)
+    __shared__ uint32_t ids[IVF_LM_IDS];
+    __shared__ float scs[IVF_LM_IDS];
     __shared__ double qs[IVF_QC][3];
     __shared__ int32_t qc[IVF_QC][3];
     __shared__ uint32_t qid[IVF_QC], qbase[IVF_QC];
-    const uint32_t item = blockIdx.x, tid = threadIdx.x;
-    uint32_t lo = 0, hi = nlist;  // the list: the last c with chunk_off[c] <= item
+    const uint32_t item = blockIdx.x, tid = threadIdx.x, lane = tid & 63, c = lane & 31, h = lane >> 5;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // the list: the last c with chunk_off[c] <= item, 64 probes at a time
+    uint32_t lo = 0, hi = nlist;
     while (hi - lo > 1) {
-        const uint32_t mid = (lo + hi) / 2;
-        if (chunk_off[mid] <= item) lo = mid;
-        else hi = mid;
+        const uint32_t step = (hi - lo + 63) / 64, at = lo + lane * step;
+        const uint64_t le = __ballot(at < hi && chunk_off[at < hi ? at : lo] <= item);
+        lo += le ? (__popcll(le) - 1) * step : 0;  // (the offsets do not decrease)
+        hi = lo + step < hi ? lo + step : hi;
     }
     const uint32_t li = lo;
     const uint32_t np = pair_count[li], p0 = pair_off[li];
@@ -1729,68 +1754,121 @@ __global__ __launch_bounds__(IVF_LM_WAVES * 64) void ivf_list_mfma(const uint32_
     const uint32_t r0 = list_off[li], nrows = list_off[li + 1] - r0;
     if (chunk_off[li] > item || pc >= np || nrows == 0) return;  // past the last item
     const uint32_t m = np - pc < (uint32_t)IVF_QC ? np - pc : (uint32_t)IVF_QC;
-    for (uint32_t i = tid; i < (uint32_t)UNITS * 32; i += IVF_LM_WAVES * 64) {
-        const uint32_t u = i / 32, col = i % 32, k = col % 8, l = col / 8;
-        v4i v{};
-        if (l < 3 && k < m) v = ((const v4i *)(qlev + (uint64_t)pair_q[p0 + pc + k] * qstride))[3 * u + l];
-        bq[u / 2][u % 2][col] = v;
+    const bool two = m > (uint32_t)IVF_QG;
+    if (tid < (uint32_t)IVF_QC) {
+        const uint32_t at = p0 + pc + (tid < m ? tid : 0);
+        qid[tid] = pair_q[at];
+        qbase[tid] = pair_base[at];
+    }
+    __syncthreads();
+    // the queries' levels as B operands, in registers (lanes of columns 24-31
+    // and of missing queries hold another's: their results are dropped)
+    v4i B[2][S];
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+        if (g && !two) break;
+        const uint32_t col = c < 24 ? c : c - 8, l = col / 8, k = g * IVF_QG + col % 8;
+        const v4i *src = (const v4i *)(qlev + (uint64_t)qid[k] * qstride) + l + 3 * h;
+#pragma unroll
+        for (int st = 0; st < S; ++st) B[g][st] = src[6 * st];
     }
     if (tid < m) {
-        const uint32_t q = pair_q[p0 + pc + tid];
-        const QLevelTail *t = (const QLevelTail *)(qlev + (uint64_t)q * qstride + (uint64_t)UNITS * 48);
+        const QLevelTail *t = (const QLevelTail *)(qlev + (uint64_t)qid[tid] * qstride + (uint64_t)UNITS * 48);
         for (int l = 0; l < 3; ++l) {
             qs[tid][l] = t->s[l];
             qc[tid][l] = BITS == 4 ? 8 * t->sum[l] : 0;
         }
-        qid[tid] = q;
-        qbase[tid] = pair_base[p0 + pc + tid];
     }
-    __syncthreads();
-    const uint32_t wave = tid >> 6, lane = tid & 63, c = lane & 31, h = lane >> 5;
-    const uint32_t tiles = (nrows + 31) / 32;
-    for (uint32_t t = wave; t < tiles; t += IVF_LM_WAVES) {
-        const uint32_t ri = t * 32 + c;
-        const uint64_t row = list_rows[r0 + (ri < nrows ? ri : nrows - 1)];  // past the end: a valid row, dropped
-        v4i A[S];
-        if constexpr (BITS == 8) {
-            // every load of the tile is issued before the first MFMA (left to
-            // itself the compiler places each load next to its MFMA and the
-            // wave waits on memory once per K step)
+    const uint32_t ring0 = lds_addr(&ring[wave][0][0]);
+    // where piece p of row r lies in its row (the rows that share banks differ)
+    auto swz = [](uint32_t r) { return r / (16 / UC) % UC; };
+    for (uint32_t b0 = 0; b0 < nrows; b0 += IVF_LM_IDS) {
+        const uint32_t bn = nrows - b0 < IVF_LM_IDS ? nrows - b0 : IVF_LM_IDS;
+        __syncthreads();  // (the last block's ids are no longer read)
+        {
+            constexpr int NI = IVF_LM_IDS / (IVF_LM_WAVES * 64);
+            uint32_t rw[NI];
+            float sc[NI];
 #pragma unroll
-            for (int st = 0; st < S; ++st) A[st] = ((const v4i *)(codes + row * W))[2 * st + h];
-            __builtin_amdgcn_sched_barrier(0);
-        } else {
-            uint2 raw[S];
+            for (int j = 0; j < NI; ++j) {
+                const uint32_t i = tid + j * (IVF_LM_WAVES * 64);
+                rw[j] = list_rows[r0 + b0 + (i < bn ? i : bn - 1)];
+            }
 #pragma unroll
-            for (int st = 0; st < S; ++st) raw[st] = ((const uint2 *)(codes + row * W))[2 * st + h];
-            __builtin_amdgcn_sched_barrier(0);
+            for (int j = 0; j < NI; ++j) sc[j] = scales[rw[j]];
 #pragma unroll
-            for (int st = 0; st < S; ++st) A[st] = unpack_q4(raw[st]);
-        }
-        v16i acc = v16i{};
-#pragma unroll
-        for (int st = 0; st < S; ++st) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[st], bq[st][h][c], acc, 0, 0, 0);
-        if (c < 24) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) stg[wave][8 * (r >> 2) + 4 * h + (r & 3)][c] = acc[r];
-        }
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t p = lane + 64 * j, rr = p % 32, k = p / 32;
-            const uint32_t i = t * 32 + rr;
-            if (k < m && i < nrows) {
-                const uint32_t rw = list_rows[r0 + i];
-                const float sc = scales[rw] * scale_mul;
-                cand[(uint64_t)qid[k] * cap + qbase[k] + i] =
-                    q_key(qs[k][0], qs[k][1], qs[k][2], dq<BITS>(stg[wave][rr][k], qc[k][0]),
-                          dq<BITS>(stg[wave][rr][8 + k], qc[k][1]), dq<BITS>(stg[wave][rr][16 + k], qc[k][2]), sc,
-                          rw);
+            for (int j = 0; j < NI; ++j) {
+                ids[tid + j * (IVF_LM_WAVES * 64)] = rw[j];
+                scs[tid + j * (IVF_LM_WAVES * 64)] = sc[j] * scale_mul;
             }
         }
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __syncthreads();
+        const uint32_t tiles = (bn + 31) / 32, mine = wave < tiles ? (tiles - wave + IVF_LM_WAVES - 1) / IVF_LM_WAVES : 0;
+        const uint32_t total = mine * NC;
+        auto load = [&](uint32_t g) {
+            const uint32_t t = wave + g / NC * IVF_LM_WAVES, ck = g % NC;
+#pragma unroll
+            for (int j = 0; j < PW; ++j) {
+                const uint32_t r = (j * (64 / UC) + lane / UC) % 32, p = (lane % UC) ^ swz(r);
+                const uint32_t i = t * 32 + r;
+                const uint32_t rw = ids[i];  // (past the end: the last row, whose results are dropped)
+                lds_dma16((const char *)codes + (uint64_t)rw * RB + ck * CB + p * 16, ring0 + g % RD * SLOT + j * 1024);
+            }
+        };
+        for (uint32_t g = 0; g < RD && g < total; ++g) load(g);
+        uint32_t g = 0;
+        for (uint32_t k0 = 0; k0 < mine; ++k0) {
+            v16i acc[2] = {v16i{}, v16i{}};
+#pragma unroll
+            for (int ck = 0; ck < NC; ++ck, ++g) {
+                const uint32_t after = total - 1 - g;
+                if (after >= RD - 1) __builtin_amdgcn_s_waitcnt(vmcnt_imm((RD - 1) * PW));
+                else if (after == 2) __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 * PW));
+                else if (after == 1) __builtin_amdgcn_s_waitcnt(vmcnt_imm(PW));
+                else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+                asm volatile("" ::: "memory");
+                const unsigned char *row = ring[wave][g % RD] + c * CB;
+                v4i A[SC];
+#pragma unroll
+                for (int st = 0; st < SC; ++st) {
+                    if constexpr (BITS == 8) A[st] = *(const v4i *)(row + (((2 * st + h) ^ swz(c)) << 4));
+                    else A[st] = unpack_q4(*(const uint2 *)(row + ((st ^ swz(c)) << 4) + h * 8));
+                }
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                if (g + RD < total) load(g + RD);  // (into the slot just read)
+#pragma unroll
+                for (int st = 0; st < SC; ++st)
+                    acc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[st], B[0][ck * SC + st], acc[0], 0, 0, 0);
+                if (two) {
+#pragma unroll
+                    for (int st = 0; st < SC; ++st)
+                        acc[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[st], B[1][ck * SC + st], acc[1], 0, 0, 0);
+                }
+            }
+            const uint32_t t = wave + k0 * IVF_LM_WAVES;
+#pragma unroll
+            for (int gr = 0; gr < 2; ++gr) {
+                if (gr && !two) break;
+                if (c < 24) {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) stg[wave][8 * (r >> 2) + 4 * h + (r & 3)][c] = acc[gr][r];
+                }
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const uint32_t p = lane + 64 * j, rr = p % 32, k8 = p / 32, k = gr * IVF_QG + k8;
+                    const uint32_t i = t * 32 + rr;
+                    if (k < m && i < bn)
+                        cand[(uint64_t)qid[k] * cap + qbase[k] + b0 + i] =
+                            q_key(qs[k][0], qs[k][1], qs[k][2], dq<BITS>(stg[wave][rr][k8], qc[k][0]),
+                                  dq<BITS>(stg[wave][rr][8 + k8], qc[k][1]), dq<BITS>(stg[wave][rr][16 + k8], qc[k][2]),
+                                  scs[i], ids[i]);
+                }
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            }
+        }
     }
 }
 }  // namespace
