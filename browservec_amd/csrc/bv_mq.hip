@@ -1151,6 +1151,11 @@ constexpr int SEL_THREADS = 1024;
 constexpr int SEL_BINS = 2048;
 constexpr int SEL_CAP = 4096;
 constexpr int SEL_KPT = 16;  // keys per thread held in registers (lists up to 16,384 keys)
+// A longer list is first cut down: the bin of its kk-th best key among 16,384
+// of its keys, evenly spread, bounds the kk-th best of all from below, and one
+// pass (eight loads a thread in flight) gathers the keys at or above it.  When
+// they fit SEL_CAP they are the list from there on.  31,000 keys for each of
+// 1,024 queries: 211 us with three passes over memory, one load at a time, 140.
 
 __global__ __launch_bounds__(SEL_THREADS) void mq_select(MqSelArgs a) {
     // (a pad word per 32 bins: the scan's lanes start 32 bins apart)
@@ -1172,13 +1177,13 @@ __global__ __launch_bounds__(SEL_THREADS) void mq_select(MqSelArgs a) {
         }
         return;
     }
-    const uint32_t n = (uint64_t)total < a.cap ? total : (uint32_t)a.cap;
+    uint32_t n = (uint64_t)total < a.cap ? total : (uint32_t)a.cap;
     const uint64_t *keys = a.cand + (uint64_t)q * a.cap;
     const uint32_t kk = a.kk < n ? a.kk : n;
     const bool sorted = a.merged != nullptr || a.out_rows != nullptr;
     // lists of at most SEL_KPT keys per thread are read once into registers
     // and every pass below runs over those; longer lists re-read memory
-    const bool cached = n <= (uint32_t)(SEL_THREADS * SEL_KPT);
+    bool cached = n <= (uint32_t)(SEL_THREADS * SEL_KPT);
     uint64_t kr[SEL_KPT];
     if (cached) {
 #pragma unroll
@@ -1186,6 +1191,10 @@ __global__ __launch_bounds__(SEL_THREADS) void mq_select(MqSelArgs a) {
             const uint32_t i = tid + (uint32_t)j * SEL_THREADS;
             kr[j] = i < n ? keys[i] : 0ull;
         }
+    } else {
+#pragma unroll
+        for (int j = 0; j < SEL_KPT; ++j)
+            kr[j] = keys[(uint64_t)(tid + (uint32_t)j * SEL_THREADS) * n / (SEL_THREADS * SEL_KPT)];
     }
     // f(key) for every key of the list
     auto each = [&](auto f) {
@@ -1200,9 +1209,10 @@ __global__ __launch_bounds__(SEL_THREADS) void mq_select(MqSelArgs a) {
     auto hbin = [](uint32_t b) { return b + (b >> 5); };
     uint32_t lim = 256;
     while (lim < 2 * kk && lim < (uint32_t)SEL_CAP) lim <<= 1;
-    uint64_t G = 0;  // keys >= G are gathered
-    uint64_t Gend = ~0ull;  // the last key of the kk-th's bin
-    if (n > kk) {
+    // narrows to the bin of the best-first rank `rank` key of each()'s keys
+    // (more than rank of them), until done(keys at or above its lower edge,
+    // keys in it): [G, Gend]
+    auto narrow = [&](auto each, uint32_t rank, auto done, uint64_t &G, uint64_t &Gend) {
         uint64_t lo = ~0ull, hi = 0;
         each([&](uint64_t k) {
             lo = k < lo ? k : lo;
@@ -1225,7 +1235,7 @@ __global__ __launch_bounds__(SEL_THREADS) void mq_select(MqSelArgs a) {
             lo = red[0][w] < lo ? red[0][w] : lo;
             hi = red[1][w] > hi ? red[1][w] : hi;
         }
-        uint32_t above = 0, rem = kk;  // keys above [lo, hi]; rank of the kk-th within [lo, hi]
+        uint32_t above = 0, rem = rank;  // keys above [lo, hi]; rank of the kk-th within [lo, hi]
         for (;;) {
             const uint64_t span = hi - lo;
             const int shift = (span >> 11) ? 64 - __clzll((long long)(span >> 11)) : 0;  // (span >> shift) < 2048
@@ -1268,13 +1278,54 @@ __global__ __launch_bounds__(SEL_THREADS) void mq_select(MqSelArgs a) {
             G = lo + ((uint64_t)bin << shift);
             const uint64_t w = (1ull << shift) - 1;  // the bin's last key, without wrapping past 2^64
             Gend = hi - G > w ? G + w : hi;
-            if ((sorted ? above + excl + cb <= lim : cb <= 1) || shift == 0) break;
+            if (done(above + excl + cb, cb) || shift == 0) break;
             above += excl;
             rem -= excl;
             lo = G;
             hi = Gend;
         }
+    };
+    uint64_t G = 0;         // keys >= G are gathered
+    uint64_t Gend = ~0ull;  // the last key of the kk-th's bin
+    if (!cached && kk < (uint32_t)(SEL_THREADS * SEL_KPT)) {
+        narrow(
+            [&](auto f) {
+#pragma unroll
+                for (int j = 0; j < SEL_KPT; ++j) f(kr[j]);
+            },
+            kk, [&](uint32_t upto, uint32_t) { return upto <= kk + kk / 4 + 32; }, G, Gend);
+        if (tid == 0) s_cnt = 0;
+        __syncthreads();
+        for (uint32_t i0 = tid; i0 < n; i0 += 8 * SEL_THREADS) {
+            uint64_t k[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const uint32_t i = i0 + (uint32_t)j * SEL_THREADS;
+                k[j] = i < n ? keys[i] : 0ull;
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if (k[j] >= G && k[j] != 0) {
+                    const uint32_t p = atomicAdd(&s_cnt, 1u);
+                    if (p < (uint32_t)SEL_CAP) sel[p] = k[j];
+                }
+        }
+        __syncthreads();
+        const uint32_t got = s_cnt;
+        if (got > kk && got <= (uint32_t)SEL_CAP) {  // (else the whole list, from memory)
+#pragma unroll
+            for (int j = 0; j < SEL_CAP / SEL_THREADS; ++j) {
+                const uint32_t i = tid + (uint32_t)j * SEL_THREADS;
+                kr[j] = i < got ? sel[i] : 0ull;
+            }
+            n = got;
+            cached = true;
+        }
+        G = 0;
+        Gend = ~0ull;
+        __syncthreads();  // (sel and s_cnt are written again below)
     }
+    if (n > kk) narrow(each, kk, [&](uint32_t upto, uint32_t in) { return sorted ? upto <= lim : in <= 1; }, G, Gend);
     if (!sorted) {
         // the bound alone: the kk-th key is the one key in [G, Gend]
         if (tid == 0) s_cnt = 0;
