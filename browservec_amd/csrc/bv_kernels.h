@@ -418,9 +418,10 @@ hipError_t launch_mqf_prep(const float *q, uint32_t nq, uint32_t dim, const uint
                            unsigned char *qbf, MqfQuery *qk, uint32_t *cnt, uint32_t cnt_value, hipStream_t s);
 hipError_t launch_mqf_scan(const MqfArgs &a, hipStream_t s);
 // Per query: the best kk keys of cand[q][0, min(cnt[q], cap)).  Outputs are
-// optional: tau = the kk-th best key (0 when there are kk or fewer), the
-// selected keys (merged, merged_n), overflow = cnt[q] > cap, and the selected
-// keys ranked into (rows, scores, n) for k_out results.
+// optional: tau = the kk-th best key, or when no keys are selected a bound a
+// little below it (0 when there are kk or fewer), the selected keys (merged,
+// merged_n), overflow = cnt[q] > cap, and the selected keys ranked into (rows,
+// scores, n) for k_out results.
 struct MqSelArgs {
     const uint64_t *cand;
     const uint32_t *cnt;

@@ -305,7 +305,7 @@ int bv_index_export_probe_scores(bv_index *idx, const float *queries, uint32_t n
 /* HNSWGpuSearcher (src/index/hnswGpu.ts:28-244): the host's HNSW build keeps
  * the graph; this object holds the corpus rows and the flat layer-0
  * adjacency on the device and beam-searches query batches
- * (src/engine/wgsl/graphSearch.ts:62-259), one wave per query.  degree is
+ * (src/engine/wgsl/graphSearch.ts:62-259), one workgroup per query.  degree is
  * the adjacency's fixed out-degree (2M), at most 64; metric BV_METRIC_* (the
  * rows and queries arrive prepared, as for an index). */
 int bv_graph_create(bv_device *dev, uint32_t dim, uint32_t metric, uint32_t degree, bv_graph **out);
