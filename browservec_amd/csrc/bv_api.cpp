@@ -3703,14 +3703,11 @@ extern "C" int bv_graph_search(bv_graph *g, const float *queries, uint32_t nq, u
     rc = graph_run(g, queries, nq, seeds, ns, efA, efA, kk, k, false);
     if (rc) return rc;
     HIPX(g->dev, hipStreamSynchronize(g->stream), "graph search");
-    // (a query's hits past its count are left as the caller had them)
     const size_t rb = HostIo::pad((size_t)nq * k * 4);
     const char *out = (const char *)g->io.out.p;
+    std::memcpy(rows, out, (size_t)nq * k * 4);
+    std::memcpy(scores, out + rb, (size_t)nq * k * 4);
     std::memcpy(n_out, out + 2 * rb, (size_t)nq * 4);
-    for (uint32_t i = 0; i < nq; i++) {
-        std::memcpy(rows + (size_t)i * k, out + (size_t)i * k * 4, (size_t)n_out[i] * 4);
-        std::memcpy(scores + (size_t)i * k, out + rb + (size_t)i * k * 4, (size_t)n_out[i] * 4);
-    }
     return BV_OK;
 }
 

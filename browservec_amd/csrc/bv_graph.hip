@@ -406,7 +406,12 @@ __global__ __launch_bounds__(GS_WG) void graph_beam(GraphArgs a) {
             a.out_scores[(uint64_t)q * a.out_stride + r] = sc;
         }
     }
-    if (tid == 0) a.out_n[q] = (uint32_t)nlive < a.k ? (uint32_t)nlive : a.k;
+    const uint32_t ko = (uint32_t)nlive < a.k ? (uint32_t)nlive : a.k;
+    for (uint32_t r = ko + tid; r < a.out_stride; r += GS_WG) {  // (no hit: zeros)
+        a.out_rows[(uint64_t)q * a.out_stride + r] = 0u;
+        a.out_scores[(uint64_t)q * a.out_stride + r] = 0.0f;
+    }
+    if (tid == 0) a.out_n[q] = ko;
 }
 
 }  // namespace
