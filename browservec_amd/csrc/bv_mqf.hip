@@ -24,7 +24,7 @@
 // stored at piece ^ row, which spreads the rows of a matrix operand over the
 // banks.
 // 1M x 768, 256 queries: the pass over seven eighths of the rows takes 555 us
-// (4.8 TB/s; 3.07 GB cost 430 us a pass as a plain stream), 817 us the call;
+// (4.8 TB/s; 3.07 GB cost 430 us a pass as a plain stream), 759 us the call;
 // the exact fp32 products it replaces (v_mfma_f32_32x32x2f32, every row once
 // per 32 queries) took 3,401 us.  Up to 64 queries the stream bounds it (674
 // us a call); at 256 the matrix cores are busy a quarter of the time and the
