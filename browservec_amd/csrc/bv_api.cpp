@@ -2434,7 +2434,9 @@ static int run_slots(bv_index *idx, const float *d_q, uint32_t nq, uint32_t kpri
     uint32_t nsub = 1;
     while (nsub < 8 && rw / (nsub * 2) >= 2 * step) nsub *= 2;
     const uint64_t per = (uint64_t)nslots * rw;
-    const uint32_t chunk = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(nq, (256ull << 20) / (per * 4)));
+    // (a launch takes up to SLOTS_MAX_NQ queries: its grid's second dimension)
+    const uint32_t chunk = (uint32_t)std::max<uint64_t>(
+        1, std::min<uint64_t>(std::min(nq, SLOTS_MAX_NQ), (256ull << 20) / (per * 4)));
     HIPX(idx->dev, idx->sl_ord.ensure((size_t)chunk * per * 4, 0, s), "scratch");
     HIPX(idx->dev, idx->sl_best.ensure((size_t)chunk * nslots * 8, 0, s), "scratch");
     HIPX(idx->dev, idx->sl_part.ensure((size_t)chunk * nslots * nsub * 4, 0, s), "scratch");

@@ -120,6 +120,7 @@ struct ScanArgs {
 // The scan of short scans and small query batches (bv_slots.h): every row's
 // order word and every slot's best key, for pick_topk.
 constexpr uint32_t SLOTS_MAX = 16384;  // slots per query (pick_topk holds their best keys in registers)
+constexpr uint32_t SLOTS_MAX_NQ = 65535;  // queries per launch (the grid's second dimension)
 struct SlotArgs {
     const void *codes;        // row-major rows, row_bytes each
     uint64_t row_bytes;

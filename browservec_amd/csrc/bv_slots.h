@@ -191,7 +191,7 @@ template <int C, int LPR, int UPL> hipError_t slots_go(const SlotArgs &a, hipStr
     using SH = ScanShape<C, LPR, UPL>;
     // slots of whole steps, parts of whole step pairs; row positions in 32 bits
     if (a.rw == 0 || a.rw % SH::RPS || a.nsub == 0 || a.rw % a.nsub || (a.nsub > 1 && a.rw / a.nsub % (2 * SH::RPS)) ||
-        a.nslots == 0 || a.nq == 0 || a.nq > 65535 ||
+        a.nslots == 0 || a.nq == 0 || a.nq > SLOTS_MAX_NQ ||
         (uint64_t)a.nslots * a.rw >= (1ull << 31) || (uint64_t)a.nslots * a.rw < a.n)
         return hipErrorInvalidValue;
     const uint32_t gx = (a.nslots + SH::WAVES - 1) / SH::WAVES;

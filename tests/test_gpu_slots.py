@@ -144,3 +144,28 @@ def test_listed_rows_equal_dot_row(ctx, metric, dim, n_list, k):
     assert [h.row for h in hits] == lst[order].tolist()
     assert np.array_equal(np.array([h.score for h in hits], np.float32).view(np.uint32), s[order].view(np.uint32))
     idx.destroy()
+
+
+def test_more_queries_than_a_launch_takes(ctx):
+    """70,000 queries over 300 rows in one call: a launch takes up to 65,535,
+    and the rest get one of their own."""
+    import torch
+
+    n, dim, nq, k = 300, 16, 70_000, 3
+    say("slots", nq, "queries")
+    idx, x, _ = make(ctx, "cosine", dim, n, 11)
+    q = torch.randn(nq, dim, generator=torch.Generator(device="cuda").manual_seed(12), device="cuda")
+    out = []
+    for width in (nq, 2500):
+        rows = torch.full((nq, k), -1, dtype=torch.int32, device="cuda")
+        scores = torch.zeros(nq, k, device="cuda")
+        cnt = torch.zeros(nq, dtype=torch.int32, device="cuda")
+        torch.cuda.synchronize()
+        for i in range(0, nq, width):
+            idx.search_device(q[i:].data_ptr(), width, 0, k, rows[i:].data_ptr(), scores[i:].data_ptr(),
+                              cnt[i:].data_ptr())
+        idx.sync()
+        out.append([rows.cpu().numpy(), scores.cpu().numpy().view(np.uint32), cnt.cpu().numpy()])
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+    idx.destroy()
