@@ -1752,6 +1752,24 @@ static int finish_batched_indexed(bv_index *idx, const float *d_q, uint32_t nq, 
     return BV_OK;
 }
 
+// Rows an fp32 batch keeps per query at most.
+static uint64_t mqf_cap(const bv_index *idx, uint32_t kprime) {
+    const uint64_t cap = std::max<uint64_t>(MQ_SAMPLE, 4ull * kprime * ((idx->rows + MQ_SAMPLE - 1) / MQ_SAMPLE));
+    return std::min<uint64_t>(cap, idx->rows);
+}
+
+// Queries per pass of an fp32 batch: up to 1,024, and what 2 GiB of scratch
+// hold, whole blocks where it is more than one.  A query takes 16 bytes per
+// row it can keep and 12 per bucket entry: 0.65 MB at k 10 over 1M rows
+// (1,024 queries at a time), 7 MB at k 1000 (256), where 1,024 took 7 GB.
+static uint32_t mqf_queries(const bv_index *idx, uint32_t kprime) {
+    const uint64_t cap = mqf_cap(idx, kprime), wgs = 256;
+    const uint64_t per = 16 * cap + 12 * std::max<uint64_t>(128 * wgs, cap + 16 * wgs);
+    const uint32_t m = (uint32_t)std::min<uint64_t>(1024, std::max<uint64_t>(1, (2ull << 30) / per));
+    const uint32_t block = mqf_block(idx->dim);
+    return m > block ? m / block * block : m;
+}
+
 // fp32 batches, exactly equal to single queries: the bf16 prefilter
 // (mqf_scan) bounds every row's score, and the passes are those of
 // run_batched_q8 below: a dense pass over MQ_SAMPLE strided rows gives each
@@ -1763,8 +1781,7 @@ static int run_batched_f32(bv_index *idx, const float *d_q, uint32_t nq, uint32_
                            uint32_t *d_rows, float *d_scores, uint32_t *d_n) {
     const uint64_t N = idx->rows, S = MQ_SAMPLE;  // N > S (mq_eligible)
     const uint32_t dim = idx->dim;
-    uint64_t cap = std::max<uint64_t>(S, 4ull * kprime * ((N + S - 1) / S));
-    cap = std::min<uint64_t>(cap, N);
+    const uint64_t cap = mqf_cap(idx, kprime);
     hipStream_t s = idx->stream;
     const uint32_t qblocks = (nq + mqf_block(dim) - 1) / mqf_block(dim);
     const int cus = idx->dev->prop.multiProcessorCount > 0 ? idx->dev->prop.multiProcessorCount : 256;
@@ -2131,10 +2148,10 @@ static int run_batched_q8(bv_index *idx, const float *d_q, uint32_t nq, uint32_t
 static int run_batched(bv_index *idx, const float *d_q, uint32_t nq, uint32_t kprime, uint32_t k_out, bool rerank,
                        uint32_t *d_rows, float *d_scores, uint32_t *d_n) {
     if (!idx->quant) {
-        // (in calls of at most 1,024 queries, whose scratch is 0.65 MB a query)
+        const uint32_t chunk = mqf_queries(idx, kprime);
         uint64_t scanned = 0;
-        for (uint32_t q0 = 0; q0 < nq; q0 += 1024) {
-            const int rc = run_batched_f32(idx, d_q + (size_t)q0 * idx->dim, std::min(1024u, nq - q0), kprime, k_out,
+        for (uint32_t q0 = 0; q0 < nq; q0 += chunk) {
+            const int rc = run_batched_f32(idx, d_q + (size_t)q0 * idx->dim, std::min(chunk, nq - q0), kprime, k_out,
                                            d_rows + (size_t)q0 * k_out, d_scores + (size_t)q0 * k_out, d_n + q0);
             if (rc) return rc;
             scanned += idx->last_scanned;
@@ -2512,9 +2529,9 @@ static int run_pipeline(bv_index *idx, const float *d_q, uint32_t nq, uint32_t k
 }
 
 // Queries per device call for query batches: the matrix-core path takes
-// large batches (its scratch is about 32 * kprime * N / MQ_SAMPLE bytes per
-// query; run_slots bounds its own); the fused scan's scratch is sized per
-// query in flight.
+// large batches (its scratch is about 112 * kprime * N / MQ_SAMPLE bytes per
+// query, of fp32 rows in passes of its own; run_slots bounds its own); the
+// fused scan's scratch is sized per query in flight.
 static uint32_t batch_chunk(const bv_index *idx, uint32_t nq) {
     return mq_eligible(idx, nq, nullptr) || (nq > 1 && slots_route(idx, nq, 1, idx->quant, false)) ? 1024u : 64u;
 }

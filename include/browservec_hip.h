@@ -214,8 +214,8 @@ int bv_index_search(bv_index *idx, const float *queries, uint32_t nq, uint32_t f
 /* Same as bv_index_search with every pointer in device memory; enqueued on
  * the index's stream and returns without waiting, except for batches of 8 or
  * more queries on a flat index, which may run on the matrix cores and then
- * wait once (fp32 rows: once per 1,024 queries; a count per query is read
- * back). */
+ * wait once (fp32 rows: once per 1,024 queries, or fewer at a time where k
+ * and the row count are large; a count per query is read back). */
 int bv_index_search_device(bv_index *idx, const float *d_queries, uint32_t nq, uint32_t fetch, uint32_t k,
                            uint32_t *d_rows, float *d_scores, uint32_t *d_n_out);
 

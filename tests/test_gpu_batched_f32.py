@@ -80,3 +80,36 @@ def test_rows_and_queries_without_bounds(ctx, metric):
     qs[6] *= np.float32(1e18)
     same_as_singles(idx, qs, 10, range(8))
     idx.destroy()
+
+
+def test_large_k_batches_bound_their_scratch(ctx):
+    """1,024 queries at k 1000 over 1M rows keep up to 250,000 rows each: the
+    batch runs in passes whose scratch stays near 2 GiB (7 GB in one), and
+    every pass answers as single queries do."""
+    import torch
+
+    from browservec_amd import FlatIndex
+
+    dim, n, nq, k = 8, 1_000_000, 1024, 1000
+    say("bf16 prefilter scratch", nq, k)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn(n, dim, generator=g, device="cuda")
+    q = torch.randn(nq, dim, generator=g, device="cuda")
+    torch.cuda.synchronize()
+    idx = FlatIndex(ctx, dim, "l2")
+    idx.append_device(x.data_ptr(), n)
+    rows = torch.zeros(nq, k, dtype=torch.int32, device="cuda")
+    scores = torch.zeros(nq, k, device="cuda")
+    cnt = torch.zeros(nq, dtype=torch.int32, device="cuda")
+    idx.sync()
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    idx.search_device(q.data_ptr(), nq, 0, k, rows.data_ptr(), scores.data_ptr(), cnt.data_ptr())
+    idx.sync()
+    assert free - torch.cuda.mem_get_info()[0] < 4 << 30
+    for i in (0, 255, 256, 700, nq - 1):
+        r, s, c = idx.search(q[i:i + 1].cpu().numpy(), 0, k)
+        assert c[0] == cnt[i].item() == k
+        assert np.array_equal(r[0], rows[i].cpu().numpy().view(np.uint32)), i
+        assert np.array_equal(s[0].view(np.uint32), scores[i].cpu().numpy().view(np.uint32)), i
+    idx.destroy()
