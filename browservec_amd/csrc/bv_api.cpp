@@ -211,6 +211,7 @@ struct bv_index {
     DevBuf mq_cand, mq_cnt, mq_tau, mq_tau2, mq_flag;  // batched matrix-core scans
     DevBuf rsq, bf16_ratio;                   // flat fp32: squared row norms; the largest relative bf16 rounding of a row (float bits)
     DevBuf mq_qbf, mq_qk, mq_rows;            // fp32 batches: bf16 queries, constants of their bounds; surviving rows
+    DevBuf mq_sk, mq_su, mq_sn;               // fp32 batches: spill lists (lower keys, upper bounds, lengths)
     DevBuf cnorm, mq_rq, mq_up, mq_kept;       // flat int8 level-one batches: row code norms, query bounds, upper bounds, kept counts
     DevBuf mq_bk, mq_bu, mq_bc;               // level-one batches: per-workgroup buckets (lower keys, upper bounds, lengths)
     DevBuf sel_keys, sel_sorted, sel_tmp;     // selection by sort: keys, sorted keys, hipCUB scratch
@@ -1758,14 +1759,14 @@ static uint64_t mqf_cap(const bv_index *idx, uint32_t kprime) {
     return std::min<uint64_t>(cap, idx->rows);
 }
 
-// Queries per pass of an fp32 batch: up to 1,024, and what 2 GiB of scratch
-// hold, whole blocks where it is more than one.  A query takes 16 bytes per
-// row it can keep and 12 per bucket entry: 0.65 MB at k 10 over 1M rows
-// (1,024 queries at a time), 7 MB at k 1000 (256), where 1,024 took 7 GB.
+// Queries per pass of an fp32 batch: up to 1,024, and what 3 GiB of scratch
+// hold, whole blocks where it is more than one.  A query takes 28 bytes per
+// row it can keep and 12 per bucket entry: 0.85 MB at k 10 over 1M rows
+// (1,024 queries at a time), 10 MB at k 1000 (256).
 static uint32_t mqf_queries(const bv_index *idx, uint32_t kprime) {
     const uint64_t cap = mqf_cap(idx, kprime), wgs = 256;
-    const uint64_t per = 16 * cap + 12 * std::max<uint64_t>(128 * wgs, cap + 16 * wgs);
-    const uint32_t m = (uint32_t)std::min<uint64_t>(1024, std::max<uint64_t>(1, (2ull << 30) / per));
+    const uint64_t per = 28 * cap + 12 * std::max<uint64_t>(128 * wgs, cap + 16 * wgs);
+    const uint32_t m = (uint32_t)std::min<uint64_t>(1024, std::max<uint64_t>(1, (3ull << 30) / per));
     const uint32_t block = mqf_block(idx->dim);
     return m > block ? m / block * block : m;
 }
@@ -1799,6 +1800,9 @@ static int run_batched_f32(bv_index *idx, const float *d_q, uint32_t nq, uint32_
     HIPX(idx->dev, idx->mq_tau.ensure((size_t)nq * 8, 0, s), "scratch");
     HIPX(idx->dev, idx->mq_qbf.ensure((size_t)nq * qstride, 0, s), "scratch");
     HIPX(idx->dev, idx->mq_qk.ensure((size_t)nq * sizeof(MqfQuery), 0, s), "scratch");
+    HIPX(idx->dev, idx->mq_sk.ensure((size_t)nq * cap * 8, 0, s), "scratch");
+    HIPX(idx->dev, idx->mq_su.ensure((size_t)nq * cap * 4, 0, s), "scratch");
+    HIPX(idx->dev, idx->mq_sn.ensure((size_t)nq * 4, 0, s), "scratch");
     HIPX(idx->dev, idx->h_cnt.ensure((size_t)nq * 8), "pinned buffer");
 
     timing_begin(idx);
@@ -1812,9 +1816,13 @@ static int run_batched_f32(bv_index *idx, const float *d_q, uint32_t nq, uint32_
     m.qblocks = qblocks;
     m.nwg = nwg;
     m.capw = capw;
+    m.spill_k = idx->mq_sk.as<uint64_t>();
+    m.spill_u = idx->mq_su.as<uint32_t>();
+    m.spill_n = idx->mq_sn.as<uint32_t>();
+    m.spill_cap = (uint32_t)cap;
     HIPX(idx->dev,
          launch_mqf_prep(d_q, nq, dim, idx->bf16_ratio.as<uint32_t>(), m.l2 != 0, idx->mq_qbf.as<unsigned char>(),
-                         idx->mq_qk.as<MqfQuery>(), idx->mq_cnt.as<uint32_t>(), (uint32_t)S, s),
+                         idx->mq_qk.as<MqfQuery>(), idx->mq_cnt.as<uint32_t>(), (uint32_t)S, m.spill_n, s),
          "query bound kernel");
     // sample pass: the lower-bound key of every logical row i < S
     m.rows = idx->raw.as<float>();
@@ -1850,7 +1858,7 @@ static int run_batched_f32(bv_index *idx, const float *d_q, uint32_t nq, uint32_
         HIPX(idx->dev,
              launch_mq1_compact(idx->mq_bk.as<uint64_t>(), idx->mq_bu.as<uint32_t>(), idx->mq_bc.as<uint32_t>(), nwg,
                                 capw, cap, idx->mq_cand.as<uint64_t>(), idx->mq_up.as<uint32_t>(),
-                                idx->mq_cnt.as<uint32_t>(), part > 0, nq, s),
+                                idx->mq_cnt.as<uint32_t>(), part > 0, nq, s, m.spill_k, m.spill_u, m.spill_n, m.spill_cap),
              "batched compact kernel");
         HIPX(idx->dev, launch_mq_select(sa, nq, s), "batched select kernel");
     }

@@ -410,13 +410,18 @@ struct MqfArgs {
     uint32_t *cnt;
     uint64_t cap;
     uint32_t capw;
+    uint64_t *spill_k;        // [nq][spill_cap] entries (lower key, upper bound) that a tile's staging does not hold
+    uint32_t *spill_u;
+    uint32_t *spill_n;        // [nq] how many (past spill_cap: some are missing)
+    uint32_t spill_cap;
 };
 bool mqf_supported(uint32_t dim);
 uint32_t mqf_block(uint32_t dim);    // queries per workgroup
 uint64_t mqf_qstride(uint32_t dim);
-// Queries to bf16 and their constants; cnt (if given) is filled with cnt_value.
+// Queries to bf16 and their constants; cnt is filled with cnt_value, spill_n with 0.
 hipError_t launch_mqf_prep(const float *q, uint32_t nq, uint32_t dim, const uint32_t *ratio_bits, bool l2,
-                           unsigned char *qbf, MqfQuery *qk, uint32_t *cnt, uint32_t cnt_value, hipStream_t s);
+                           unsigned char *qbf, MqfQuery *qk, uint32_t *cnt, uint32_t cnt_value, uint32_t *spill_n,
+                           hipStream_t s);
 hipError_t launch_mqf_scan(const MqfArgs &a, hipStream_t s);
 // Per query: the best kk keys of cand[q][0, min(cnt[q], cap)).  Outputs are
 // optional: tau = the kk-th best key, or when no keys are selected a bound a
@@ -497,10 +502,12 @@ hipError_t launch_ham_exact(const uint32_t *codes, uint32_t W, const uint32_t *q
                             uint64_t cap, uint64_t *keys, uint32_t nq, hipStream_t s);
 // Per query: its buckets joined into lk / uo [nq][cap] (after the list's
 // cnt[q] entries when append is set) and the length in cnt[q] (0xffffffff
-// when a bucket overflowed or the total exceeds cap).
+// when a bucket overflowed or the total exceeds cap).  spill_k (or null): the
+// entries of its spill list join them, and spill_n[q] is 0 again.
 hipError_t launch_mq1_compact(const uint64_t *bk, const uint32_t *bu, const uint32_t *bc, uint32_t nwg,
                               uint32_t capw, uint64_t cap, uint64_t *lk, uint32_t *uo, uint32_t *cnt, bool append,
-                              uint32_t nq, hipStream_t s);
+                              uint32_t nq, hipStream_t s, const uint64_t *spill_k = nullptr,
+                              const uint32_t *spill_u = nullptr, uint32_t *spill_n = nullptr, uint32_t spill_cap = 0);
 // Per query: the rows among cand[q][0, min(cnt[q], cap)) whose upper bound
 // (make_key(up[q][i], row)) reaches tau[q], into rows[q][...], their number
 // in kept[q].

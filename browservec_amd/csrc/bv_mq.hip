@@ -1083,7 +1083,8 @@ __global__ __launch_bounds__(MQ_WAVES * 64) void mq1_scan_bits(Mq1Args a) {
 // than cap entries gets length 0xffffffff (it falls back).
 __global__ __launch_bounds__(1024) void mq1_compact(const uint64_t *bk, const uint32_t *bu, const uint32_t *bc,
                                                      uint32_t nwg, uint32_t capw, uint64_t cap, uint64_t *lk,
-                                                     uint32_t *uo, uint32_t *cnt, int append) {
+                                                     uint32_t *uo, uint32_t *cnt, int append, const uint64_t *spill_k,
+                                                     const uint32_t *spill_u, uint32_t *spill_n, uint32_t spill_cap) {
     __shared__ uint32_t off[1025];
     __shared__ uint32_t wsum[16];
     __shared__ uint32_t bad;
@@ -1091,8 +1092,10 @@ __global__ __launch_bounds__(1024) void mq1_compact(const uint64_t *bk, const ui
     const int lane = tid & 63, wave = tid >> 6;
     const uint32_t base = append ? cnt[q] : 0u;  // entries already in the list
     if ((uint64_t)base > cap) return;             // already overflowed
-    if (tid == 0) bad = 0;
+    const uint32_t ns = spill_k ? spill_n[q] : 0u;
+    if (tid == 0) bad = ns > spill_cap;
     __syncthreads();
+    if (tid == 0 && spill_k) spill_n[q] = 0;
     // bucket lengths (one thread per bucket; nwg <= 1024) and their exclusive
     // prefix: within each wave, then across the waves
     uint32_t c = 0;
@@ -1120,7 +1123,7 @@ __global__ __launch_bounds__(1024) void mq1_compact(const uint64_t *bk, const ui
         off[nwg] = t;
     }
     __syncthreads();
-    const uint32_t total = base + off[nwg];
+    const uint64_t total = (uint64_t)base + off[nwg] + ns;
     if (bad || total > cap) {
         if (tid == 0) cnt[q] = 0xffffffffu;
         return;
@@ -1134,7 +1137,11 @@ __global__ __launch_bounds__(1024) void mq1_compact(const uint64_t *bk, const ui
             uo[dst + i] = bu[src + i];
         }
     }
-    if (tid == 0) cnt[q] = total;
+    for (uint32_t i = tid; i < ns; i += 1024) {
+        lk[(uint64_t)q * cap + base + off[nwg] + i] = spill_k[(uint64_t)q * spill_cap + i];
+        uo[(uint64_t)q * cap + base + off[nwg] + i] = spill_u[(uint64_t)q * spill_cap + i];
+    }
+    if (tid == 0) cnt[q] = (uint32_t)total;
 }
 
 // One workgroup per query.  The kk-th best key is found by binning the
@@ -2062,11 +2069,12 @@ hipError_t launch_ham_exact(const uint32_t *codes, uint32_t W, const uint32_t *q
 
 hipError_t launch_mq1_compact(const uint64_t *bk, const uint32_t *bu, const uint32_t *bc, uint32_t nwg,
                               uint32_t capw, uint64_t cap, uint64_t *lk, uint32_t *uo, uint32_t *cnt, bool append,
-                              uint32_t nq, hipStream_t s) {
+                              uint32_t nq, hipStream_t s, const uint64_t *spill_k, const uint32_t *spill_u,
+                              uint32_t *spill_n, uint32_t spill_cap) {
     if (nq == 0) return hipSuccess;
-    if (nwg == 0 || nwg > 1024) return hipErrorInvalidValue;
+    if (nwg == 0 || nwg > 1024 || (spill_k && (!spill_u || !spill_n))) return hipErrorInvalidValue;
     hipLaunchKernelGGL(mq1_compact, dim3(nq), dim3(1024), 0, s, bk, bu, bc, nwg, capw, cap, lk, uo, cnt,
-                       append ? 1 : 0);
+                       append ? 1 : 0, spill_k, spill_u, spill_n, spill_cap);
     return hipGetLastError();
 }
 

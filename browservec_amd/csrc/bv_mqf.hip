@@ -56,7 +56,6 @@ struct MqfStage {
     uint32_t uo[2][8][MQF_STAGE];  // order words of the upper bounds
     uint16_t lo[2][8][64];         // first entry of each lane
     uint16_t ln[2][8][64];         // entries of each lane
-    uint8_t qovf[256];             // a query's entries did not all fit
 };
 
 __device__ __forceinline__ float mqf_upper(float s, float e) { return fmaf(fabsf(s), 0x1p-20f, s + e); }
@@ -85,7 +84,7 @@ __device__ __forceinline__ void mqf_flush(const MqfArgs &a, uint32_t qb, uint32_
     const uint32_t off1 = st.lo[fb][w][c + 32], n1 = st.ln[fb][w][c + 32];
     for (uint32_t j = 0; j < n0 + n1; ++j) {
         const uint32_t i = j < n0 ? off0 + j : off1 + (j - n0);
-        if (i >= MQF_STAGE) continue;  // not staged (the query is marked)
+        if (i >= MQF_STAGE) continue;  // (in the query's spill list)
         if (len < a.capw) {
             a.cand[bucket + len] = st.lk[fb][w][i];
             a.up_out[bucket + len] = st.uo[fb][w][i];
@@ -126,7 +125,6 @@ __global__ __launch_bounds__(WAVES * 64) void mqf_scan(MqfArgs a) {
     const uint64_t ntiles = (a.n + MQF_ROWS - 1) / MQF_ROWS;
     const bool loader = wave < LOADERS;
     for (uint32_t i = threadIdx.x; i < 2 * 8 * 64; i += WAVES * 64) st.ln[i / 512][(i / 64) % 8][i % 64] = 0;
-    for (uint32_t i = threadIdx.x; i < 256; i += WAVES * 64) st.qovf[i] = 0;
     uint32_t blen = 0;
     bool bovf = false;
     const uint32_t mine = wg < ntiles ? (uint32_t)((ntiles - wg + a.nwg - 1) / a.nwg) : 0;  // tiles wg, wg + nwg, ..
@@ -353,11 +351,12 @@ __global__ __launch_bounds__(WAVES * 64) void mqf_scan(MqfArgs a) {
             st.ln[sb][wave][lane] = (uint16_t)cnt;
             if (__builtin_amdgcn_readlane((int)incl, 63)) {
                 uint32_t pos = incl - cnt;
+                // what the staging buffer does not hold (whole tiles pass where
+                // a topic's rows lie next to each other and its queries too)
+                // goes to the query's spill list
+                uint32_t at = 0;
+                if (incl > MQF_STAGE && cnt) at = atomicAdd(&a.spill_n[q], incl - MQF_STAGE < cnt ? incl - MQF_STAGE : cnt);
                 for (uint32_t m = p; m; m &= m - 1, ++pos) {
-                    if (pos >= MQF_STAGE) {
-                        st.qovf[qlocal] = 1;  // the query's list can no longer be complete: it falls back
-                        break;
-                    }
                     const uint32_t bit = __builtin_ctz(m);
                     float s = 0.0f, e = 0.0f;
 #pragma unroll
@@ -365,8 +364,18 @@ __global__ __launch_bounds__(WAVES * 64) void mqf_scan(MqfArgs a) {
                         if ((uint32_t)r == bit) s = acc[r], e = ev[r];
                     const float lo = mqf_lower(s, e), up = mqf_upper(s, e);
                     const uint32_t row = (uint32_t)(a.row_base + (t0 + (uint32_t)row_of((int)bit)) * a.row_step);
-                    st.lk[sb][wave][pos] = make_key(lo == lo ? ord_f32(lo) : 0u, row);
-                    st.uo[sb][wave][pos] = up == up ? ord_f32(up) : 0xffffffffu;
+                    const uint64_t lk = make_key(lo == lo ? ord_f32(lo) : 0u, row);
+                    const uint32_t uo = up == up ? ord_f32(up) : 0xffffffffu;
+                    if (pos < MQF_STAGE) {
+                        st.lk[sb][wave][pos] = lk;
+                        st.uo[sb][wave][pos] = uo;
+                    } else {
+                        if (at < a.spill_cap) {  // (a count past it tells mq1_compact)
+                            a.spill_k[(uint64_t)q * a.spill_cap + at] = lk;
+                            a.spill_u[(uint64_t)q * a.spill_cap + at] = uo;
+                        }
+                        ++at;
+                    }
                 }
             }
         }
@@ -376,7 +385,7 @@ __global__ __launch_bounds__(WAVES * 64) void mqf_scan(MqfArgs a) {
         if (!loader) {
             if (mine) mqf_flush<QB>(a, qb, wg, st, (int)((mine - 1) & 1), wave - LOADERS, lane, blen, bovf);
             const uint32_t ql = (uint32_t)(wave - LOADERS) * 64 + lane, qq = qb * QB + ql;
-            if (qq < a.nq) a.cnt[(uint64_t)qq * a.nwg + wg] = bovf || st.qovf[ql] ? 0xffffffffu : blen;
+            if (qq < a.nq) a.cnt[(uint64_t)qq * a.nwg + wg] = bovf ? 0xffffffffu : blen;
         }
     }
 }
@@ -385,7 +394,7 @@ __global__ __launch_bounds__(WAVES * 64) void mqf_scan(MqfArgs a) {
 // constants of its bounds.  ratio: the largest |x - bf16(x)| / |x| of a row.
 __global__ __launch_bounds__(64) void mqf_prep(const float *q, uint32_t dim, const uint32_t *ratio_bits, int l2,
                                                unsigned char *qbf, uint64_t qstride, MqfQuery *qk, uint32_t *cnt,
-                                               uint32_t cnt_value) {
+                                               uint32_t cnt_value, uint32_t *spill_n) {
     const int lane = threadIdx.x;
     const float *x = q + (uint64_t)blockIdx.x * dim;
     __bf16 *out = (__bf16 *)(qbf + (uint64_t)blockIdx.x * qstride);
@@ -427,7 +436,8 @@ __global__ __launch_bounds__(64) void mqf_prep(const float *q, uint32_t dim, con
     if (!(qn < 0x1p60)) k.alpha = __builtin_inff();  // (products or sums could leave the range of f32)
     k.qsq = (float)s;
     qk[blockIdx.x] = k;
-    if (cnt) cnt[blockIdx.x] = cnt_value;
+    cnt[blockIdx.x] = cnt_value;
+    spill_n[blockIdx.x] = 0;
 }
 
 // One wave per row: f64 sum of squares rounded to f32, and the largest ratio
@@ -499,11 +509,12 @@ uint32_t mqf_block(uint32_t dim) { return dim <= 768 ? 256u : 128u; }
 uint64_t mqf_qstride(uint32_t dim) { return (uint64_t)((dim + MQF_DIMS - 1) / MQF_DIMS) * MQF_DIMS * 2; }
 
 hipError_t launch_mqf_prep(const float *q, uint32_t nq, uint32_t dim, const uint32_t *ratio_bits, bool l2,
-                           unsigned char *qbf, MqfQuery *qk, uint32_t *cnt, uint32_t cnt_value, hipStream_t s) {
+                           unsigned char *qbf, MqfQuery *qk, uint32_t *cnt, uint32_t cnt_value, uint32_t *spill_n,
+                           hipStream_t s) {
     if (nq == 0) return hipSuccess;
     if (!mqf_supported(dim)) return hipErrorInvalidValue;
     hipLaunchKernelGGL(mqf_prep, dim3(nq), dim3(64), 0, s, q, dim, ratio_bits, l2 ? 1 : 0, qbf, mqf_qstride(dim), qk,
-                       cnt, cnt_value);
+                       cnt, cnt_value, spill_n);
     return hipGetLastError();
 }
 
@@ -520,7 +531,7 @@ template <int CH, int WAVES> static hipError_t mqf_go(const MqfArgs &a, hipStrea
 hipError_t launch_mqf_scan(const MqfArgs &a, hipStream_t s) {
     if (a.n == 0 || a.nq == 0) return hipSuccess;
     if (a.n > (1ull << 32) || !mqf_supported(a.dim) || !a.cand || !a.rsq || a.qstride != mqf_qstride(a.dim) ||
-        (a.tau && (!a.up_out || !a.cnt || a.capw == 0)))
+        (a.tau && (!a.up_out || !a.cnt || a.capw == 0 || !a.spill_k || !a.spill_u || !a.spill_n)))
         return hipErrorInvalidValue;
     switch ((a.dim + MQF_DIMS - 1) / MQF_DIMS) {
     case 1: return mqf_go<1, 8>(a, s);
