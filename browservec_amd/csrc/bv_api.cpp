@@ -211,7 +211,6 @@ struct bv_index {
     DevBuf mq_cand, mq_cnt, mq_tau, mq_tau2, mq_flag;  // batched matrix-core scans
     DevBuf rsq, bf16_ratio;                   // flat fp32: squared row norms; the largest relative bf16 rounding of a row (float bits)
     DevBuf mq_qbf, mq_qk, mq_rows;            // fp32 batches: bf16 queries, constants of their bounds; surviving rows
-    DevBuf mq_sk, mq_su, mq_sn;               // fp32 batches: spill lists (lower keys, upper bounds, lengths)
     DevBuf cnorm, mq_rq, mq_up, mq_kept;       // flat int8 level-one batches: row code norms, query bounds, upper bounds, kept counts
     DevBuf mq_bk, mq_bu, mq_bc;               // level-one batches: per-workgroup buckets (lower keys, upper bounds, lengths)
     DevBuf sel_keys, sel_sorted, sel_tmp;     // selection by sort: keys, sorted keys, hipCUB scratch
@@ -1789,21 +1788,23 @@ static int run_batched_f32(bv_index *idx, const float *d_q, uint32_t nq, uint32_
     const uint32_t nwg = std::min<uint32_t>(1024, std::max<uint32_t>(8, (uint32_t)cus / qblocks & ~7u));
     const uint32_t capw = (uint32_t)((std::max<uint64_t>(128, (cap + nwg - 1) / nwg) + 15) & ~15ull);
     const uint64_t qstride = mqf_qstride(dim);
+    const size_t nbk = (size_t)nq * nwg * capw;  // bucket entries; the spill lists follow
     HIPX(idx->dev, idx->mq_cand.ensure((size_t)nq * std::max<uint64_t>(cap, S) * 8, 0, s), "scratch");
     HIPX(idx->dev, idx->mq_up.ensure((size_t)nq * cap * 4, 0, s), "scratch");
-    HIPX(idx->dev, idx->mq_bk.ensure((size_t)nq * nwg * capw * 8, 0, s), "scratch");
-    HIPX(idx->dev, idx->mq_bu.ensure((size_t)nq * nwg * capw * 4, 0, s), "scratch");
-    HIPX(idx->dev, idx->mq_bc.ensure((size_t)nq * nwg * 4, 0, s), "scratch");
+    HIPX(idx->dev, idx->mq_bk.ensure((nbk + (size_t)nq * cap) * 8, 0, s), "scratch");
+    HIPX(idx->dev, idx->mq_bu.ensure((nbk + (size_t)nq * cap) * 4, 0, s), "scratch");
+    HIPX(idx->dev, idx->mq_bc.ensure((size_t)nq * (nwg + 1) * 4, 0, s), "scratch");
     HIPX(idx->dev, idx->mq_rows.ensure((size_t)nq * cap * 4, 0, s), "scratch");
     HIPX(idx->dev, idx->mq_cnt.ensure((size_t)nq * 4, 0, s), "scratch");
     HIPX(idx->dev, idx->mq_kept.ensure((size_t)nq * 4, 0, s), "scratch");
     HIPX(idx->dev, idx->mq_tau.ensure((size_t)nq * 8, 0, s), "scratch");
     HIPX(idx->dev, idx->mq_qbf.ensure((size_t)nq * qstride, 0, s), "scratch");
     HIPX(idx->dev, idx->mq_qk.ensure((size_t)nq * sizeof(MqfQuery), 0, s), "scratch");
-    HIPX(idx->dev, idx->mq_sk.ensure((size_t)nq * cap * 8, 0, s), "scratch");
-    HIPX(idx->dev, idx->mq_su.ensure((size_t)nq * cap * 4, 0, s), "scratch");
-    HIPX(idx->dev, idx->mq_sn.ensure((size_t)nq * 4, 0, s), "scratch");
     HIPX(idx->dev, idx->h_cnt.ensure((size_t)nq * 8), "pinned buffer");
+
+    const uint64_t *spill_k = idx->mq_bk.as<uint64_t>() + nbk;
+    const uint32_t *spill_u = idx->mq_bu.as<uint32_t>() + nbk;
+    uint32_t *spill_n = idx->mq_bc.as<uint32_t>() + (size_t)nq * nwg;
 
     timing_begin(idx);
     MqfArgs m{};
@@ -1816,13 +1817,9 @@ static int run_batched_f32(bv_index *idx, const float *d_q, uint32_t nq, uint32_
     m.qblocks = qblocks;
     m.nwg = nwg;
     m.capw = capw;
-    m.spill_k = idx->mq_sk.as<uint64_t>();
-    m.spill_u = idx->mq_su.as<uint32_t>();
-    m.spill_n = idx->mq_sn.as<uint32_t>();
-    m.spill_cap = (uint32_t)cap;
     HIPX(idx->dev,
          launch_mqf_prep(d_q, nq, dim, idx->bf16_ratio.as<uint32_t>(), m.l2 != 0, idx->mq_qbf.as<unsigned char>(),
-                         idx->mq_qk.as<MqfQuery>(), idx->mq_cnt.as<uint32_t>(), (uint32_t)S, m.spill_n, s),
+                         idx->mq_qk.as<MqfQuery>(), idx->mq_cnt.as<uint32_t>(), (uint32_t)S, spill_n, s),
          "query bound kernel");
     // sample pass: the lower-bound key of every logical row i < S
     m.rows = idx->raw.as<float>();
@@ -1858,7 +1855,7 @@ static int run_batched_f32(bv_index *idx, const float *d_q, uint32_t nq, uint32_
         HIPX(idx->dev,
              launch_mq1_compact(idx->mq_bk.as<uint64_t>(), idx->mq_bu.as<uint32_t>(), idx->mq_bc.as<uint32_t>(), nwg,
                                 capw, cap, idx->mq_cand.as<uint64_t>(), idx->mq_up.as<uint32_t>(),
-                                idx->mq_cnt.as<uint32_t>(), part > 0, nq, s, m.spill_k, m.spill_u, m.spill_n, m.spill_cap),
+                                idx->mq_cnt.as<uint32_t>(), part > 0, nq, s, spill_k, spill_u, spill_n, (uint32_t)cap),
              "batched compact kernel");
         HIPX(idx->dev, launch_mq_select(sa, nq, s), "batched select kernel");
     }

@@ -404,16 +404,15 @@ struct MqfArgs {
     uint32_t nq;
     uint32_t qblocks;         // ceil(nq / mqf_block(dim))
     uint32_t nwg;             // workgroups per query block (a multiple of 8)
-    const uint64_t *tau;      // null: dense pass; else [nq] bound keys; outputs as in Mq1Args
+    // null: dense pass; else [nq] bound keys; outputs as in Mq1Args, and behind
+    // the buckets (in cand and up_out; counts behind theirs in cnt) a spill list
+    // of cap entries per query: what a tile's staging does not hold
+    const uint64_t *tau;
     uint64_t *cand;
     uint32_t *up_out;
     uint32_t *cnt;
     uint64_t cap;
     uint32_t capw;
-    uint64_t *spill_k;        // [nq][spill_cap] entries (lower key, upper bound) that a tile's staging does not hold
-    uint32_t *spill_u;
-    uint32_t *spill_n;        // [nq] how many (past spill_cap: some are missing)
-    uint32_t spill_cap;
 };
 bool mqf_supported(uint32_t dim);
 uint32_t mqf_block(uint32_t dim);    // queries per workgroup

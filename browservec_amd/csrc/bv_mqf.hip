@@ -350,31 +350,29 @@ __global__ __launch_bounds__(WAVES * 64) void mqf_scan(MqfArgs a) {
             st.lo[sb][wave][lane] = (uint16_t)(incl - cnt);
             st.ln[sb][wave][lane] = (uint16_t)cnt;
             if (__builtin_amdgcn_readlane((int)incl, 63)) {
-                uint32_t pos = incl - cnt;
-                // what the staging buffer does not hold (whole tiles pass where
-                // a topic's rows lie next to each other and its queries too)
-                // goes to the query's spill list
-                uint32_t at = 0;
-                if (incl > MQF_STAGE && cnt) at = atomicAdd(&a.spill_n[q], incl - MQF_STAGE < cnt ? incl - MQF_STAGE : cnt);
-                for (uint32_t m = p; m; m &= m - 1, ++pos) {
-                    const uint32_t bit = __builtin_ctz(m);
+                uint32_t pos = incl - cnt, m = p;
+                auto entry = [&](uint32_t bit, uint64_t &lk, uint32_t &uo) {
                     float s = 0.0f, e = 0.0f;
 #pragma unroll
                     for (int r = 0; r < 16; ++r)
                         if ((uint32_t)r == bit) s = acc[r], e = ev[r];
                     const float lo = mqf_lower(s, e), up = mqf_upper(s, e);
                     const uint32_t row = (uint32_t)(a.row_base + (t0 + (uint32_t)row_of((int)bit)) * a.row_step);
-                    const uint64_t lk = make_key(lo == lo ? ord_f32(lo) : 0u, row);
-                    const uint32_t uo = up == up ? ord_f32(up) : 0xffffffffu;
-                    if (pos < MQF_STAGE) {
-                        st.lk[sb][wave][pos] = lk;
-                        st.uo[sb][wave][pos] = uo;
-                    } else {
-                        if (at < a.spill_cap) {  // (a count past it tells mq1_compact)
-                            a.spill_k[(uint64_t)q * a.spill_cap + at] = lk;
-                            a.spill_u[(uint64_t)q * a.spill_cap + at] = uo;
-                        }
-                        ++at;
+                    lk = make_key(lo == lo ? ord_f32(lo) : 0u, row);
+                    uo = up == up ? ord_f32(up) : 0xffffffffu;
+                };
+                for (; m && pos < MQF_STAGE; m &= m - 1, ++pos) entry(__builtin_ctz(m), st.lk[sb][wave][pos], st.uo[sb][wave][pos]);
+                // what the staging buffer does not hold (whole tiles pass where
+                // a topic's rows lie next to each other and its queries too)
+                // goes to the query's spill list, behind the buckets
+                if (__builtin_expect(__ballot(m != 0) != 0, 0)) {
+                    const uint64_t nb = (uint64_t)a.nq * a.nwg;
+                    uint64_t at = 0;
+                    if (m) at = atomicAdd(&a.cnt[nb + q], (uint32_t)__popc(m));
+                    for (; m; m &= m - 1, ++at) {
+                        if (at >= a.cap) break;  // (a count past it tells mq1_compact)
+                        const uint64_t i = nb * a.capw + (uint64_t)q * a.cap + at;
+                        entry(__builtin_ctz(m), a.cand[i], a.up_out[i]);
                     }
                 }
             }
@@ -531,7 +529,7 @@ template <int CH, int WAVES> static hipError_t mqf_go(const MqfArgs &a, hipStrea
 hipError_t launch_mqf_scan(const MqfArgs &a, hipStream_t s) {
     if (a.n == 0 || a.nq == 0) return hipSuccess;
     if (a.n > (1ull << 32) || !mqf_supported(a.dim) || !a.cand || !a.rsq || a.qstride != mqf_qstride(a.dim) ||
-        (a.tau && (!a.up_out || !a.cnt || a.capw == 0 || !a.spill_k || !a.spill_u || !a.spill_n)))
+        (a.tau && (!a.up_out || !a.cnt || a.capw == 0)))
         return hipErrorInvalidValue;
     switch ((a.dim + MQF_DIMS - 1) / MQF_DIMS) {
     case 1: return mqf_go<1, 8>(a, s);
