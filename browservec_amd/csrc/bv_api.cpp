@@ -179,6 +179,11 @@ struct HostIo {
     hipError_t send(hipStream_t s) { return launch_copy_in(dev.p, in.p, used, s); }
 };
 
+// Queries of a batch that are run again, and their results.
+struct Rerun {
+    DevBuf q, rows, scores, n;
+};
+
 // ------------------------------------------------------------------ index
 // query streams a caller may keep single queries in flight on
 // (bv_index_set_query_streams)
@@ -209,8 +214,10 @@ struct bv_index {
     DevBuf out_rows, out_scores, out_n;
     DevBuf cand, cand_n, dense;
     DevBuf mq_cand, mq_cnt, mq_tau, mq_tau2, mq_flag;  // batched matrix-core scans
-    DevBuf rsq, bf16_ratio;                   // flat fp32: squared row norms; the largest relative bf16 rounding of a row (float bits)
+    DevBuf rsq, row_max;                      // flat fp32: squared row norms; the largest relative bf16 rounding and squared norm of a row (float bits)
     DevBuf mq_qbf, mq_qk, mq_rows;            // fp32 batches: bf16 queries, constants of their bounds; surviving rows
+    DevBuf mq_qsq, mq_slack;                  // ... and of the pass of fp32 products: squared query norms, slacks
+    Rerun rerun[2];                           // queries of a batch that are run again
     DevBuf cnorm, mq_rq, mq_up, mq_kept;       // flat int8 level-one batches: row code norms, query bounds, upper bounds, kept counts
     DevBuf mq_bk, mq_bu, mq_bc;               // level-one batches: per-workgroup buckets (lower keys, upper bounds, lengths)
     DevBuf sel_keys, sel_sorted, sel_tmp;     // selection by sort: keys, sorted keys, hipCUB scratch
@@ -455,8 +462,8 @@ extern "C" int bv_index_create(bv_device *dev, const bv_index_desc *desc, bv_ind
     if (e == hipSuccess) e = hipEventCreateWithFlags(&x->ev0, hipEventDisableSystemFence);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&x->ev1, hipEventDisableSystemFence);
     if (e == hipSuccess && !quant && !x->ivf) {
-        e = x->bf16_ratio.ensure(256, 0, x->stream, false);
-        if (e == hipSuccess) e = hipMemset(x->bf16_ratio.p, 0, 256);
+        e = x->row_max.ensure(256, 0, x->stream, false);
+        if (e == hipSuccess) e = hipMemset(x->row_max.p, 0, 256);
     }
     if (e == hipSuccess && quant) {
         std::vector<float> s;
@@ -843,7 +850,7 @@ static int append_common(bv_index *idx, const float *data, bool device_src, uint
         if (norms)
             HIPX(idx->dev,
                  launch_row_sqnorms(idx->raw.as<float>() + r0 * idx->dim, m, idx->dim, idx->rsq.as<float>() + r0,
-                                    idx->bf16_ratio.as<uint32_t>(), idx->stream),
+                                    idx->row_max.as<uint32_t>(), idx->stream),
                  "norm kernel");
         if (idx->quant) {
             EncodeArgs e{};
@@ -1572,7 +1579,7 @@ static int run_fused(bv_index *idx, const float *d_q, uint32_t nq, uint32_t kpri
 // best kprime per query go to the exact re-rank or straight to the output.
 // Keys are the single-query scan's keys, so results equal the same queries
 // run one at a time.  A query whose appended keys overflow their buffer (a
-// bound left loose by the sample) is re-run through the fused scan.
+// bound left loose by the sample) is run again (rerun_overflowed).
 constexpr uint32_t MQ_MIN_Q = 8;  // smallest batch for the matrix-core path (it waits once; fewer queries never do)
 
 static bool mq_eligible(const bv_index *idx, uint32_t nq, const uint32_t *d_mask) {
@@ -1621,8 +1628,8 @@ static uint32_t mq_groups(const bv_index *idx, uint32_t qblocks) {
 // keys with the single-query arithmetic (three exact level dots, f64
 // combine), and the best kprime of them are selected and re-ranked as a
 // single query's are.
-// A query whose kept rows overflow their buffer runs the fused scan over
-// every row.
+// A query whose kept rows overflow their buffer is run again
+// (rerun_overflowed).
 // The codes the first-level pass reads: the index's int8 codes, or for a
 // Hamming index the +1 / -1 expansion of its 1-bit codes (unit scales), whose
 // int8 dots are the Hamming similarities.
@@ -1706,9 +1713,13 @@ static int prepare_pm(bv_index *idx, const float *d_q, uint32_t nq, const unsign
 // apart; a query whose joined list overflowed, mq_cnt[q] > cap, kept none):
 // the fused scan in indexed mode over the kept rows computes their
 // single-query keys, selects and re-ranks, so every query returns what it
-// returns alone.  Overflowed queries are re-run alone over every row.
+// returns alone.  Overflowed queries are run again (rerun_overflowed).
+static int rerun_overflowed(bv_index *idx, const float *d_q, const std::vector<uint32_t> &over, uint32_t kprime,
+                            uint32_t k_out, bool rerank, bool products, uint32_t *d_rows, float *d_scores,
+                            uint32_t *d_n);
 static int finish_batched_indexed(bv_index *idx, const float *d_q, uint32_t nq, uint32_t kprime, uint32_t k_out,
-                                  bool rerank, uint64_t cap, uint32_t *d_rows, float *d_scores, uint32_t *d_n) {
+                                  bool rerank, uint64_t cap, bool products, uint32_t *d_rows, float *d_scores,
+                                  uint32_t *d_n) {
     hipStream_t s = idx->stream;
     uint32_t *h = (uint32_t *)idx->h_cnt.p;  // [nq] kept, then [nq] joined counts
     HIPX(idx->dev, hipMemcpyAsync(h, idx->mq_kept.p, (size_t)nq * 4, hipMemcpyDeviceToHost, s), "count download");
@@ -1743,13 +1754,10 @@ static int finish_batched_indexed(bv_index *idx, const float *d_q, uint32_t nq, 
     uint64_t scanned = (idx->rows + MQ_SAMPLE) * nq;
     for (uint32_t i = 0; i < nq; i++) scanned += std::min<uint64_t>(kept[i], cap);
     idx->last_scanned = scanned;
-    for (uint32_t i = 0; i < nq; i++) {
-        if (joined[i] <= cap) continue;
-        rc = run_fused(idx, d_q + (size_t)i * idx->dim, 1, kprime, k_out, rerank, nullptr, 0,
-                       d_rows + (size_t)i * k_out, d_scores + (size_t)i * k_out, d_n + i);
-        if (rc) return rc;
-    }
-    return BV_OK;
+    std::vector<uint32_t> over;
+    for (uint32_t i = 0; i < nq; i++)
+        if (joined[i] > cap) over.push_back(i);
+    return rerun_overflowed(idx, d_q, over, kprime, k_out, rerank, products, d_rows, d_scores, d_n);
 }
 
 // Rows an fp32 batch keeps per query at most.
@@ -1818,7 +1826,7 @@ static int run_batched_f32(bv_index *idx, const float *d_q, uint32_t nq, uint32_
     m.nwg = nwg;
     m.capw = capw;
     HIPX(idx->dev,
-         launch_mqf_prep(d_q, nq, dim, idx->bf16_ratio.as<uint32_t>(), m.l2 != 0, idx->mq_qbf.as<unsigned char>(),
+         launch_mqf_prep(d_q, nq, dim, idx->row_max.as<uint32_t>(), m.l2 != 0, idx->mq_qbf.as<unsigned char>(),
                          idx->mq_qk.as<MqfQuery>(), idx->mq_cnt.as<uint32_t>(), (uint32_t)S, spill_n, s),
          "query bound kernel");
     // sample pass: the lower-bound key of every logical row i < S
@@ -1863,7 +1871,7 @@ static int run_batched_f32(bv_index *idx, const float *d_q, uint32_t nq, uint32_
          launch_mq1_keep(idx->mq_cand.as<uint64_t>(), idx->mq_up.as<uint32_t>(), idx->mq_cnt.as<uint32_t>(), cap,
                          idx->mq_tau.as<uint64_t>(), idx->mq_rows.as<uint32_t>(), idx->mq_kept.as<uint32_t>(), nq, s),
          "batched keep kernel");
-    return finish_batched_indexed(idx, d_q, nq, kprime, k_out, false, cap, d_rows, d_scores, d_n);
+    return finish_batched_indexed(idx, d_q, nq, kprime, k_out, false, cap, true, d_rows, d_scores, d_n);
 }
 
 static int run_batched_q8(bv_index *idx, const float *d_q, uint32_t nq, uint32_t kprime, uint32_t k_out,
@@ -2084,7 +2092,7 @@ static int run_batched_q8(bv_index *idx, const float *d_q, uint32_t nq, uint32_t
                          idx->mq_kept.as<uint32_t>(), nq, s),
          "batched keep kernel");
     if (asym1 && idx->codec != C_Q1P)
-        return finish_batched_indexed(idx, d_q, nq, kprime, k_out, rerank, cap, d_rows, d_scores, d_n);
+        return finish_batched_indexed(idx, d_q, nq, kprime, k_out, rerank, cap, false, d_rows, d_scores, d_n);
     // exact keys of those rows, the best kprime of them, and the re-rank
     if (asym1) {
         qa.rows = idx->mq_rows.as<uint32_t>();
@@ -2138,16 +2146,10 @@ static int run_batched_q8(bv_index *idx, const float *d_q, uint32_t nq, uint32_t
     HIPX(idx->dev, hipStreamSynchronize(s), "batched scan");
     const uint32_t *cnt = (const uint32_t *)idx->h_cnt.p;
     idx->last_scanned = (N + S) * nq;
-    // queries whose kept rows overflowed their buffer: the fused scan over every row
     std::vector<uint32_t> over;
     for (uint32_t i = 0; i < nq; i++)
         if (cnt[i] > cap) over.push_back(i);
-    for (uint32_t i : over) {
-        rc = run_fused(idx, d_q + (size_t)i * idx->dim, 1, kprime, k_out, rerank, nullptr, 0,
-                       d_rows + (size_t)i * k_out, d_scores + (size_t)i * k_out, d_n + i);
-        if (rc) return rc;
-    }
-    return BV_OK;
+    return rerun_overflowed(idx, d_q, over, kprime, k_out, rerank, false, d_rows, d_scores, d_n);
 }
 
 static int run_batched(bv_index *idx, const float *d_q, uint32_t nq, uint32_t kprime, uint32_t k_out, bool rerank,
@@ -2253,19 +2255,16 @@ static int run_batched(bv_index *idx, const float *d_q, uint32_t nq, uint32_t kp
     }
     timing_end(idx);
     idx->last_scanned = (N + (one_pass ? 0 : S)) * nq;
-    // queries whose appended keys overflowed: the fused scan, one at a time
+    // queries whose appended keys overflowed
     HIPX(idx->dev, idx->h_flag.ensure((size_t)nq * 4), "pinned buffer");
     HIPX(idx->dev, hipMemcpyAsync(idx->h_flag.p, idx->mq_flag.p, (size_t)nq * 4, hipMemcpyDeviceToHost, idx->stream),
          "flag download");
     HIPX(idx->dev, hipStreamSynchronize(idx->stream), "batched scan");
     const uint32_t *flags = (const uint32_t *)idx->h_flag.p;
-    for (uint32_t i = 0; i < nq; i++) {
-        if (!flags[i]) continue;
-        rc = run_fused(idx, d_q + (size_t)i * idx->dim, 1, kprime, k_out, rerank, nullptr, 0,
-                       d_rows + (size_t)i * k_out, d_scores + (size_t)i * k_out, d_n + i);
-        if (rc) return rc;
-    }
-    return BV_OK;
+    std::vector<uint32_t> over;
+    for (uint32_t i = 0; i < nq; i++)
+        if (flags[i]) over.push_back(i);
+    return rerun_overflowed(idx, d_q, over, kprime, k_out, rerank, false, d_rows, d_scores, d_n);
 }
 
 // The device pipeline shared by every query entry point.
@@ -2415,9 +2414,12 @@ static int run_ivf_batched(bv_index *idx, const float *d_q, uint32_t nq, uint32_
 //   fp32 batches cost 0.62 us per million elements on top: 100,000 x 384
 //     crosses at 20 (16 queries 129 / 161, 32 183 / 165), 20,000 x 384 at 75
 //     (64 queries 119 / 132).
+static bool slots_fit(const bv_index *idx, bool rerank) {
+    return !idx->ivf && idx->rows > 0 && idx->rows < (1ull << 30) &&
+           pick_supported(idx->codec, idx->P, rerank ? idx->dim : 0);
+}
 static bool slots_route(const bv_index *idx, uint32_t nq, uint32_t kprime, bool rerank, bool batchable) {
-    if (idx->ivf || idx->rows == 0 || idx->rows >= (1ull << 30)) return false;
-    if (!pick_supported(idx->codec, idx->P, rerank ? idx->dim : 0)) return false;
+    if (!slots_fit(idx, rerank)) return false;
     if (nq == 1) return !(idx->codec == C_Q8 && idx->rows * idx->row_bytes >= (512ull << 20) && kprime <= 256);
     if (!batchable) return true;
     double per;  // us per million (row, unit)
@@ -2506,6 +2508,131 @@ static int run_slots(bv_index *idx, const float *d_q, uint32_t nq, uint32_t kpri
     }
     timing_end(idx);
     idx->last_scanned = idx->rows * nq;
+    return BV_OK;
+}
+
+// fp32 queries that overflowed under the bf16 bounds, with fp32 products
+// (mqx_scan): a dense pass over the sample, the rows that reach its bound
+// minus the rounding of the sums, their exact scores.
+static int run_products_f32(bv_index *idx, const float *d_q, uint32_t nq, uint32_t kprime, uint32_t k_out,
+                            uint32_t *d_rows, float *d_scores, uint32_t *d_n) {
+    const uint64_t N = idx->rows, S = MQ_SAMPLE, cap = mqf_cap(idx, kprime);
+    hipStream_t s = idx->stream;
+    HIPX(idx->dev, idx->mq_cand.ensure((size_t)nq * S * 8, 0, s), "scratch");
+    HIPX(idx->dev, idx->mq_rows.ensure((size_t)nq * cap * 4, 0, s), "scratch");
+    HIPX(idx->dev, idx->mq_cnt.ensure((size_t)nq * 4, 0, s), "scratch");
+    HIPX(idx->dev, idx->mq_kept.ensure((size_t)nq * 4, 0, s), "scratch");
+    HIPX(idx->dev, idx->mq_tau.ensure((size_t)nq * 8, 0, s), "scratch");
+    HIPX(idx->dev, idx->mq_qsq.ensure((size_t)nq * 4, 0, s), "scratch");
+    HIPX(idx->dev, idx->mq_slack.ensure((size_t)nq * 4, 0, s), "scratch");
+    HIPX(idx->dev, idx->h_cnt.ensure((size_t)nq * 8), "pinned buffer");
+
+    timing_begin(idx);
+    MqxArgs m{};
+    m.rows = idx->raw.as<float>();
+    m.rsq = idx->rsq.as<float>();
+    m.dim = idx->dim;
+    m.l2 = idx->d.metric == BV_METRIC_L2;
+    m.q = d_q;
+    m.qsq = idx->mq_qsq.as<float>();
+    m.slack = idx->mq_slack.as<float>();
+    m.nq = nq;
+    m.qblocks = (nq + MQ_QB - 1) / MQ_QB;
+    m.groups = mq_groups(idx, m.qblocks);
+    HIPX(idx->dev,
+         launch_mqx_qconst(d_q, nq, idx->dim, idx->row_max.as<uint32_t>() + 1, m.l2 != 0, idx->mq_qsq.as<float>(),
+                           idx->mq_slack.as<float>(), s),
+         "query norm kernel");
+    m.n = S;
+    m.row_step = N / S;
+    m.cand = idx->mq_cand.as<uint64_t>();
+    m.cap = S;
+    HIPX(idx->dev, launch_mqx_scan(m, s), "batched scan kernel");
+    HIPX(idx->dev, hipMemsetD32Async((hipDeviceptr_t)idx->mq_cnt.p, (int)S, nq, s), "scratch");
+    MqSelArgs sa{};
+    sa.cand = m.cand;
+    sa.cnt = idx->mq_cnt.as<uint32_t>();
+    sa.cap = S;
+    sa.kk = kprime;
+    sa.tau = idx->mq_tau.as<uint64_t>();
+    HIPX(idx->dev, launch_mq_select(sa, nq, s), "batched select kernel");
+    HIPX(idx->dev, hipMemsetAsync(idx->mq_cnt.p, 0, (size_t)nq * 4, s), "scratch");
+    m.n = N;
+    m.row_step = 1;
+    m.tau = idx->mq_tau.as<uint64_t>();
+    m.rows_out = idx->mq_rows.as<uint32_t>();
+    m.cnt = idx->mq_cnt.as<uint32_t>();
+    m.cap = cap;
+    HIPX(idx->dev, launch_mqx_scan(m, s), "batched scan kernel");
+    HIPX(idx->dev, hipMemcpyAsync(idx->mq_kept.p, idx->mq_cnt.p, (size_t)nq * 4, hipMemcpyDeviceToDevice, s), "counts");
+    return finish_batched_indexed(idx, d_q, nq, kprime, k_out, false, cap, false, d_rows, d_scores, d_n);
+}
+
+// The queries of a batch whose kept rows overflowed their lists, all together:
+// first (products) with fp32 products, which may tell apart what bf16 ones do
+// not, then by slot scans, which read the rows once for up to four queries
+// (the fused scan where they do not take the index).
+static int rerun_overflowed(bv_index *idx, const float *d_q, const std::vector<uint32_t> &over, uint32_t kprime,
+                            uint32_t k_out, bool rerank, bool products, uint32_t *d_rows, float *d_scores,
+                            uint32_t *d_n) {
+    if (over.empty()) return BV_OK;
+    const uint64_t before = idx->last_scanned;
+    const uint32_t m = (uint32_t)over.size(), dim = idx->dim;
+    hipStream_t s = idx->stream;
+    const float *q = d_q + (size_t)over[0] * dim;
+    uint32_t *rows = d_rows + (size_t)over[0] * k_out, *n = d_n + over[0];
+    float *scores = d_scores + (size_t)over[0] * k_out;
+    // queries that do not lie next to each other are gathered (the pass of
+    // products may leave some for slot scans: buffers for each)
+    Rerun &b = idx->rerun[products ? 0 : 1];
+    std::vector<std::pair<uint32_t, uint32_t>> runs;  // position in over, length
+    for (uint32_t i = 0; i < m; ++i) {
+        if (i && over[i] == over[i - 1] + 1) runs.back().second++;
+        else runs.push_back({i, 1});
+    }
+    const bool gather = runs.size() > 1;
+    if (gather) {
+        HIPX(idx->dev, b.q.ensure((size_t)m * dim * 4, 0, s), "scratch");
+        HIPX(idx->dev, b.rows.ensure((size_t)m * k_out * 4, 0, s), "scratch");
+        HIPX(idx->dev, b.scores.ensure((size_t)m * k_out * 4, 0, s), "scratch");
+        HIPX(idx->dev, b.n.ensure((size_t)m * 4, 0, s), "scratch");
+        for (const auto &r : runs)
+            HIPX(idx->dev,
+                 hipMemcpyAsync(b.q.as<float>() + (size_t)r.first * dim, d_q + (size_t)over[r.first] * dim,
+                                (size_t)r.second * dim * 4, hipMemcpyDeviceToDevice, s),
+                 "query gather");
+        q = b.q.as<float>();
+        rows = b.rows.as<uint32_t>();
+        scores = b.scores.as<float>();
+        n = b.n.as<uint32_t>();
+    }
+    int rc = BV_OK;
+    if (products && m >= MQ_MIN_Q && mqx_supported(dim)) {
+        rc = run_products_f32(idx, q, m, kprime, k_out, rows, scores, n);
+    } else if (slots_fit(idx, rerank)) {
+        rc = run_slots(idx, q, m, kprime, k_out, rerank, nullptr, 0, rows, scores, n);
+    } else {
+        for (uint32_t i = 0; i < m && !rc; i += 64)
+            rc = run_fused(idx, q + (size_t)i * dim, std::min(64u, m - i), kprime, k_out, rerank, nullptr, 0,
+                           rows + (size_t)i * k_out, scores + (size_t)i * k_out, n + i);
+        idx->last_scanned = idx->rows * m;
+    }
+    if (rc) return rc;
+    idx->last_scanned += before;
+    if (gather)
+        for (const auto &r : runs) {
+            const size_t to = over[r.first], from = r.first;
+            HIPX(idx->dev,
+                 hipMemcpyAsync(d_rows + to * k_out, rows + from * k_out, (size_t)r.second * k_out * 4,
+                                hipMemcpyDefault, s),
+                 "result scatter");
+            HIPX(idx->dev,
+                 hipMemcpyAsync(d_scores + to * k_out, scores + from * k_out, (size_t)r.second * k_out * 4,
+                                hipMemcpyDefault, s),
+                 "result scatter");
+            HIPX(idx->dev, hipMemcpyAsync(d_n + to, n + from, (size_t)r.second * 4, hipMemcpyDefault, s),
+                 "result scatter");
+        }
     return BV_OK;
 }
 
@@ -3501,7 +3628,7 @@ extern "C" int bv_index_load_section(bv_index *idx, const float *data, uint64_t 
     }
     if (norms)
         HIPX(idx->dev, launch_row_sqnorms(idx->raw.as<float>(), count, idx->dim, idx->rsq.as<float>(),
-                                          idx->bf16_ratio.as<uint32_t>(), s),
+                                          idx->row_max.as<uint32_t>(), s),
              "norm kernel");
     if (code_norms)
         HIPX(idx->dev, launch_row_code_norms(idx->codes.as<uint32_t>(), count, idx->words_per_row,

@@ -380,9 +380,10 @@ struct MqArgs {
     uint64_t cap;
 };
 // Per-row squared norms of fp32 rows (f64 sums rounded to f32) and, raised in
-// *ratio_bits, the largest |x - bf16(x)| / |x| of the rows (float bits, rounded
-// up; the ratios are >= 0, so the bits order like the values).
-hipError_t launch_row_sqnorms(const float *rows, uint64_t n, uint32_t dim, float *rsq, uint32_t *ratio_bits,
+// max_bits, the largest |x - bf16(x)| / |x| (max_bits[0]) and squared norm
+// (max_bits[1]) of the rows (float bits, rounded up; both are >= 0, so the bits
+// order like the values).
+hipError_t launch_row_sqnorms(const float *rows, uint64_t n, uint32_t dim, float *rsq, uint32_t *max_bits,
                               hipStream_t s);
 // The bf16 prefilter of fp32 batches (mqf_scan): bounds s +- E of every row's
 // score, E = alpha |x| + beta + gamma |x|^2 per query.
@@ -422,6 +423,32 @@ hipError_t launch_mqf_prep(const float *q, uint32_t nq, uint32_t dim, const uint
                            unsigned char *qbf, MqfQuery *qk, uint32_t *cnt, uint32_t cnt_value, uint32_t *spill_n,
                            hipStream_t s);
 hipError_t launch_mqf_scan(const MqfArgs &a, hipStream_t s);
+// The fp32-product prefilter of queries that overflow under the bf16 bounds
+// (mqx_scan), for the dimensions mqx_supported accepts.
+struct MqxArgs {
+    const float *rows;        // logical row i at rows + i * row_step * dim
+    const float *rsq;         // ... its squared norm at rsq[i * row_step]
+    uint32_t dim;
+    int l2;
+    uint64_t n;               // logical rows in this pass
+    uint64_t row_step;
+    const float *q;           // nq x dim queries
+    const float *qsq;         // [nq] squared norms and slacks (launch_mqx_qconst)
+    const float *slack;
+    uint32_t nq;
+    uint32_t qblocks;         // ceil(nq / MQ_QB)
+    uint32_t groups;          // workgroups per (XCD, query block)
+    const uint64_t *tau;      // null: dense pass into cand [nq][cap] (cap >= n); else [nq] bound keys
+    uint64_t *cand;
+    uint32_t *rows_out;       // [nq][cap] ids of the kept rows
+    uint32_t *cnt;            // [nq] how many (past cap: some are missing)
+    uint64_t cap;
+};
+bool mqx_supported(uint32_t dim);
+// max_bits: float bits of the largest squared row norm.
+hipError_t launch_mqx_qconst(const float *q, uint32_t nq, uint32_t dim, const uint32_t *max_bits, bool l2, float *qsq,
+                             float *slack, hipStream_t s);
+hipError_t launch_mqx_scan(const MqxArgs &a, hipStream_t s);
 // Per query: the best kk keys of cand[q][0, min(cnt[q], cap)).  Outputs are
 // optional: tau = the kk-th best key, or when no keys are selected a bound a
 // little below it (0 when there are kk or fewer), the selected keys (merged,

@@ -51,6 +51,15 @@ constexpr uint32_t MQF_CHUNK = MQF_ROWS * MQF_DIMS * 4; // bytes
 constexpr uint32_t MQF_TILE = MQF_CHUNK / 2;            // the same as bf16
 constexpr uint32_t MQF_STAGE = 120;                     // entries per wave per staging buffer
 
+// The next float below x.
+__device__ __forceinline__ float mqx_below(float x) {
+    if (x != x) return x;  // (keeps every row)
+    const uint32_t b = __float_as_uint(x);
+    if ((b & 0x7fffffffu) == 0) return __uint_as_float(0x80000001u);
+    if (b == 0xff800000u) return x;
+    return __uint_as_float((b & 0x80000000u) ? b + 1 : b - 1);
+}
+
 struct MqfStage {
     uint64_t lk[2][8][MQF_STAGE];  // lower-bound keys, in lane order
     uint32_t uo[2][8][MQF_STAGE];  // order words of the upper bounds
@@ -374,6 +383,10 @@ __global__ __launch_bounds__(WAVES * 64) void mqf_scan(MqfArgs a) {
                         const uint64_t i = nb * a.capw + (uint64_t)q * a.cap + at;
                         entry(__builtin_ctz(m), a.cand[i], a.up_out[i]);
                     }
+                    // (the query is run again whatever else is kept of it: from
+                    // here on nothing.  Where every row passes for 64 queries,
+                    // 1M x 768, a call took 4.4 ms with all of them spilled)
+                    if (at >= a.cap) stau[qlocal] = __builtin_inff();
                 }
             }
         }
@@ -438,19 +451,224 @@ __global__ __launch_bounds__(64) void mqf_prep(const float *q, uint32_t dim, con
     spill_n[blockIdx.x] = 0;
 }
 
-// One wave per row: f64 sum of squares rounded to f32, and the largest ratio
-// |x - bf16(x)| / |x| (float bits, rounded up, at most 2^-8: a larger ratio
-// comes from subnormal elements, which the bounds' absolute terms cover).
+// ------------------------------------------------------- fp32 products ----
+// The same prefilter with fp32 products (v_mfma_f32_32x32x2f32), for queries
+// whose kept rows overflowed under the bf16 bounds: where the rows have a
+// large part in common (a mean ten times the spread), 2 x 0.0035 |x| |q| keeps
+// every row, and the rounding of the f32 sums, which is all that separates
+// these scores from the single-query scan's, still tells them apart.
+// 1M x 768, 256 queries: 3.4 ms, against 34 for slot scans of the rows and 125
+// for one fused scan per query.
+//
+// The block's 32 queries stay in LDS, each wave streams 64 rows.  Lane l =
+// 32h + c supplies, over the four matrix steps of chunk t, elements 8t + 4h ..
+// 8t + 4h + 3 of row c (A) and of query c (B), one 16-byte load each, so both
+// operands pair the same elements.  A score differs from the single-query
+// scan's by at most E = slack / 2 (mqx_qconst).
+//
+// Passes: dense (tau null: every key of logical row i at cand[q][i]), and the
+// ids of the rows whose score reaches tau's score minus slack[q].  That keeps
+// every row the exact scan can rank: a row in the exact top-kk has a
+// single-query score >= the kk-th best single-query score >= tau's score - E,
+// hence a score here >= tau's score - 2E.
+template <int CHUNKS>
+__global__ __launch_bounds__(MQ_WAVES * 64) void mqx_scan(MqxArgs a) {
+    constexpr int G = CHUNKS < 4 ? CHUNKS : 4;
+    __shared__ float4 qlds[CHUNKS][64];
+    __shared__ float qts[MQ_QB];
+    __shared__ float qn2[MQ_QB];
+    __shared__ float rn2[MQ_WAVES][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int h = lane >> 5, c = lane & 31;
+    const uint32_t b = blockIdx.x, xcd = b & 7u, slot = b >> 3;
+    const uint32_t qb = slot % a.qblocks, grp = slot / a.qblocks;
+    const uint64_t tstride = 8ull * a.groups;
+    uint64_t tile = xcd + 8ull * grp;
+    if (tile * MQ_ROWS >= a.n) return;
+    {
+        uint32_t q = qb * MQ_QB + c;
+        if (q >= a.nq) q = a.nq - 1;
+        const float *src = a.q + (uint64_t)q * a.dim;
+        for (int t = wave; t < CHUNKS; t += MQ_WAVES)
+            __builtin_amdgcn_global_load_lds((glb_void *)(src + 8 * t + 4 * h), (lds_void *)&qlds[t][0], 16, 0, 0);
+    }
+    if (threadIdx.x < MQ_QB) {
+        uint32_t q = qb * MQ_QB + threadIdx.x;
+        if (q >= a.nq) q = a.nq - 1;
+        const uint64_t t = a.tau ? a.tau[q] : 0ull;
+        // tau's score minus the slack, rounded down
+        qts[threadIdx.x] = t ? mqx_below((float)((double)f32_from_ord((uint32_t)(t >> 32)) - (double)a.slack[q]))
+                             : -__builtin_inff();
+        qn2[threadIdx.x] = a.l2 ? a.qsq[q] : 0.0f;
+    }
+    auto row_sq = [&](uint64_t t) {
+        uint64_t li = t * MQ_ROWS + (uint64_t)wave * 64 + lane;
+        if (li >= a.n) li = a.n - 1;
+        return a.rsq[li * a.row_step];
+    };
+    float rsq_next = a.l2 ? row_sq(tile) : 0.0f;
+    auto row_ptrs = [&](uint64_t t, const float4 *(&ap)[2]) {
+        const uint64_t w0 = t * MQ_ROWS + (uint64_t)wave * 64;
+#pragma unroll
+        for (int fr = 0; fr < 2; ++fr) {
+            uint64_t li = w0 + fr * 32 + c;
+            if (li >= a.n) li = a.n - 1;  // rows past the end load a valid row; their results are dropped
+            ap[fr] = (const float4 *)(a.rows + li * a.row_step * a.dim + 4 * h);
+        }
+    };
+    const float4 *ap[2];
+    row_ptrs(tile, ap);
+    float4 ring[2][G][2];
+#pragma unroll
+    for (int j = 0; j < G; ++j)
+#pragma unroll
+        for (int fr = 0; fr < 2; ++fr) ring[0][j][fr] = ap[fr][2 * j];
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+
+    const uint32_t q = qb * MQ_QB + c;
+    const bool qok = q < a.nq;
+    const uint32_t qq = qok ? q : a.nq - 1;
+    for (;;) {
+        const uint64_t ntile = tile + tstride;
+        const bool more = ntile * MQ_ROWS < a.n;
+        const float4 *np[2];
+        row_ptrs(more ? ntile : tile, np);
+        v16f acc[2] = {v16f{}, v16f{}};
+#pragma unroll
+        for (int t = 0; t < CHUNKS; ++t) {
+            const int gp = (t / G) & 1, j = t % G;
+            if (j == 0) {
+                const int nt = t + G;
+#pragma unroll
+                for (int jj = 0; jj < G; ++jj)
+#pragma unroll
+                    for (int fr = 0; fr < 2; ++fr) {
+                        if (nt < CHUNKS) ring[gp ^ 1][jj][fr] = ap[fr][2 * (nt + jj)];
+                        else if (more) ring[gp ^ 1][jj][fr] = np[fr][2 * (nt - CHUNKS + jj)];
+                    }
+            }
+            const float4 B = qlds[t][lane];
+            const float bv[4] = {B.x, B.y, B.z, B.w};
+#pragma unroll
+            for (int fr = 0; fr < 2; ++fr) {
+                const float4 A = ring[gp][j][fr];
+                const float av[4] = {A.x, A.y, A.z, A.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[fr] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[e], bv[e], acc[fr], 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr ((CHUNKS / G) & 1) {
+#pragma unroll
+            for (int j = 0; j < G; ++j)
+#pragma unroll
+                for (int fr = 0; fr < 2; ++fr) ring[0][j][fr] = ring[1][j][fr];
+        }
+        // l2: the score from the dot and the squared norms (this wave's 64
+        // rows' norms through wave-private LDS)
+        if (a.l2) {
+            rn2[wave][lane] = rsq_next;
+            if (more) rsq_next = row_sq(ntile);
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            const float qs2 = qn2[c];
+#pragma unroll
+            for (int fr = 0; fr < 2; ++fr)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const float x2 = rn2[wave][fr * 32 + 8 * (r >> 2) + 4 * h + (r & 3)];
+                    acc[fr][r] = 2.0f * acc[fr][r] - x2 - qs2;
+                }
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        }
+        const uint64_t w0 = tile * MQ_ROWS + (uint64_t)wave * 64;
+        const bool full = w0 + 64 <= a.n;
+        if (!a.tau) {
+            uint64_t *out = a.cand + (uint64_t)qq * a.cap;
+#pragma unroll
+            for (int fr = 0; fr < 2; ++fr)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const uint64_t li = w0 + fr * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
+                    if (qok && (full || li < a.n)) out[li] = make_key(ord_f32(acc[fr][r]), (uint32_t)(li * a.row_step));
+                }
+        } else {
+            const float ts = qts[c];
+            uint32_t pass = 0;
+#pragma unroll
+            for (int fr = 0; fr < 2; ++fr)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const uint64_t li = w0 + fr * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
+                    // a NaN score passes: the exact scan ranks it as it ranks any key
+                    if (qok && (full || li < a.n) && !(acc[fr][r] < ts)) pass |= 1u << (fr * 16 + r);
+                }
+            if (__ballot(pass != 0)) {
+                const uint32_t mine = __popc(pass);
+                const uint32_t other = __shfl_xor(mine, 32);
+                uint32_t base = 0;
+                if (h == 0 && mine + other) base = atomicAdd(&a.cnt[qq], mine + other);
+                base = __shfl(base, c);
+                if (pass) {
+                    uint32_t *ro = a.rows_out + (uint64_t)qq * a.cap;
+                    uint64_t pos = (uint64_t)base + (h ? other : 0u);
+#pragma unroll
+                    for (int fr = 0; fr < 2; ++fr)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r)
+                            if (pass & (1u << (fr * 16 + r))) {
+                                const uint64_t li = w0 + fr * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
+                                if (pos < a.cap) ro[pos] = (uint32_t)(li * a.row_step);
+                                ++pos;
+                            }
+                }
+            }
+        }
+        if (!more) break;
+        ap[0] = np[0];
+        ap[1] = np[1];
+        tile = ntile;
+    }
+}
+
+// One wave per query: |q|^2 and the slack 2E.  u = 2^-24: E is 3 (dim + 2) u
+// |x|max |q| for dot products, 4 (dim + 4) u (|x|max + |q|)^2 under l2, and
+// room for the subnormal products a matrix core may flush.
+__global__ __launch_bounds__(64) void mqx_qconst(const float *q, uint32_t dim, const uint32_t *max_bits, int l2,
+                                                 float *qsq, float *slack) {
+    const int lane = threadIdx.x;
+    const float *x = q + (uint64_t)blockIdx.x * dim;
+    double s = 0.0;
+    for (uint32_t i = lane; i < dim; i += 64) s = fma((double)x[i], (double)x[i], s);
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) s += __shfl_xor(s, o);
+    if (lane == 0) {
+        const double u = 0x1p-24;
+        const double xn = sqrt((double)__uint_as_float(*max_bits)) * (1.0 + 0x1p-20);
+        const double qn = sqrt(s) * (1.0 + 0x1p-20);
+        const double e = l2 ? 4.0 * (dim + 4) * u * (xn + qn) * (xn + qn) : 3.0 * (dim + 2) * u * xn * qn;
+        qsq[blockIdx.x] = (float)s;
+        slack[blockIdx.x] = (float)((2.0 * e + dim * 0x1p-126) * (1.0 + 0x1p-10));
+    }
+}
+
+// One wave per row: f64 sum of squares rounded to f32, and over the rows the
+// largest ratio |x - bf16(x)| / |x| (float bits, rounded up, at most 2^-8: a
+// larger ratio comes from subnormal elements, which the bounds' absolute terms
+// cover) in max_bits[0] and the largest sum (rounded up) in max_bits[1].
 // Rows of zeros have none, and rows out of range have no bounds at all
 // (mqf_norm).
 // 1M x 768: 0.59 ms (5.2 TB/s); with an atomic per wave instead of one per
 // workgroup of many rows 3.0 ms.
 __global__ __launch_bounds__(256) void row_sqnorms(const float *rows, uint64_t n, uint32_t dim, float *rsq,
-                                                   uint32_t *ratio_bits) {
+                                                   uint32_t *max_bits) {
     const int lane = threadIdx.x & 63;
     const uint64_t nw = (uint64_t)gridDim.x * 4;
-    __shared__ uint32_t wmx[4];
+    __shared__ uint32_t wmx[4], wsq[4];
     double mx = 0.0;  // largest squared ratio
+    uint32_t sq = 0;  // largest sum's bits (the next float up: it may have been rounded down)
     for (uint64_t r = (uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6); r < n; r += nw) {
         const float *x = rows + r * dim;
         double s = 0.0, res = 0.0;
@@ -475,30 +693,37 @@ __global__ __launch_bounds__(256) void row_sqnorms(const float *rows, uint64_t n
         }
         if (lane == 0) {
             rsq[r] = (float)s;
+            const uint32_t b = __float_as_uint((float)s);
+            sq = max(sq, b < 0x7f800000u ? b + 1 : b);  // (inf and NaN stay)
             const double ratio = s > 0.0 && s < 0x1p122 ? res / s : 0.0;
             mx = ratio > mx ? ratio : mx;
         }
     }
     if (lane == 0) {
         const double ratio = sqrt(mx) * (1.0 + 0x1p-20);
+        wsq[threadIdx.x >> 6] = sq;
         wmx[threadIdx.x >> 6] = __float_as_uint(ratio < 0x1p-8 ? (float)ratio : 0x1p-8f);
     }
     __syncthreads();
-    if (threadIdx.x == 0) {  // (one atomic per workgroup: they serialize)
-        uint32_t b = wmx[0];
-        for (int i = 1; i < 4; ++i) b = wmx[i] > b ? wmx[i] : b;
-        if (b) atomicMax(ratio_bits, b);
+    if (threadIdx.x == 0) {  // (two atomics per workgroup: they serialize)
+        uint32_t b = wmx[0], m = wsq[0];
+        for (int i = 1; i < 4; ++i) {
+            b = wmx[i] > b ? wmx[i] : b;
+            m = wsq[i] > m ? wsq[i] : m;
+        }
+        if (b) atomicMax(max_bits, b);
+        if (m) atomicMax(max_bits + 1, m);
     }
 }
 
 }  // namespace
 
-hipError_t launch_row_sqnorms(const float *rows, uint64_t n, uint32_t dim, float *rsq, uint32_t *ratio_bits,
+hipError_t launch_row_sqnorms(const float *rows, uint64_t n, uint32_t dim, float *rsq, uint32_t *max_bits,
                               hipStream_t s) {
     if (n == 0) return hipSuccess;
     uint64_t blocks = (n + 3) / 4;
     if (blocks > 2048) blocks = 2048;  // eight workgroups per CU
-    hipLaunchKernelGGL(row_sqnorms, dim3((uint32_t)blocks), dim3(256), 0, s, rows, n, dim, rsq, ratio_bits);
+    hipLaunchKernelGGL(row_sqnorms, dim3((uint32_t)blocks), dim3(256), 0, s, rows, n, dim, rsq, max_bits);
     return hipGetLastError();
 }
 
@@ -542,6 +767,44 @@ hipError_t launch_mqf_scan(const MqfArgs &a, hipStream_t s) {
     case 8: return mqf_go<8, 4>(a, s);
     default: return hipErrorInvalidValue;
     }
+}
+
+bool mqx_supported(uint32_t dim) {
+    switch (dim) {
+    case 32: case 64: case 96: case 128: case 192: case 256: case 384: case 512: case 768: case 1024: return true;
+    default: return false;
+    }
+}
+
+hipError_t launch_mqx_qconst(const float *q, uint32_t nq, uint32_t dim, const uint32_t *max_bits, bool l2, float *qsq,
+                             float *slack, hipStream_t s) {
+    if (nq == 0) return hipSuccess;
+    hipLaunchKernelGGL(mqx_qconst, dim3(nq), dim3(64), 0, s, q, dim, max_bits, l2 ? 1 : 0, qsq, slack);
+    return hipGetLastError();
+}
+
+hipError_t launch_mqx_scan(const MqxArgs &a, hipStream_t s) {
+    if (a.n == 0 || a.nq == 0) return hipSuccess;
+    if (!mqx_supported(a.dim) || a.qblocks == 0 || a.groups == 0 || (uint64_t)a.qblocks * MQ_QB < a.nq || !a.rsq ||
+        !a.qsq || (a.tau ? !a.rows_out || !a.cnt || !a.slack : !a.cand || a.cap < a.n))
+        return hipErrorInvalidValue;
+    const uint64_t blocks = 8ull * a.groups * a.qblocks;
+    if (blocks > 0x7fffffffull) return hipErrorInvalidValue;
+    const dim3 g((uint32_t)blocks), wg(MQ_WAVES * 64);
+    switch (a.dim) {
+    case 32: hipLaunchKernelGGL(mqx_scan<4>, g, wg, 0, s, a); break;
+    case 64: hipLaunchKernelGGL(mqx_scan<8>, g, wg, 0, s, a); break;
+    case 96: hipLaunchKernelGGL(mqx_scan<12>, g, wg, 0, s, a); break;
+    case 128: hipLaunchKernelGGL(mqx_scan<16>, g, wg, 0, s, a); break;
+    case 192: hipLaunchKernelGGL(mqx_scan<24>, g, wg, 0, s, a); break;
+    case 256: hipLaunchKernelGGL(mqx_scan<32>, g, wg, 0, s, a); break;
+    case 384: hipLaunchKernelGGL(mqx_scan<48>, g, wg, 0, s, a); break;
+    case 512: hipLaunchKernelGGL(mqx_scan<64>, g, wg, 0, s, a); break;
+    case 768: hipLaunchKernelGGL(mqx_scan<96>, g, wg, 0, s, a); break;
+    case 1024: hipLaunchKernelGGL(mqx_scan<128>, g, wg, 0, s, a); break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
 }
 
 }  // namespace bvk

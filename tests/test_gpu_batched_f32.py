@@ -168,3 +168,70 @@ def test_neighbouring_rows_of_a_corpus_in_topic_order(ctx, metric, dim, n, size,
     scanned = equals_fused(idx, x[s:s + nq].contiguous(), nq, 10)
     assert (n + SAMPLE) * nq < scanned < (n + SAMPLE) * nq + nq * 2 * size + 8 * n
     idx.destroy()
+
+
+@pytest.mark.parametrize("metric,dim,products", [("dot", 768, True), ("l2", 128, True), ("dot", 100, False)])
+def test_rows_with_a_large_part_in_common(ctx, metric, dim, products):
+    """A common mean keeps every row under the bf16 bounds: the batch is run
+    again with fp32 products where the dimension has them, else by slot scans,
+    and answers as single queries do."""
+    import torch
+
+    from browservec_amd import FlatIndex
+
+    n, nq = 60_000, 300
+    say("common mean", metric, dim)
+    g = torch.Generator(device="cuda").manual_seed(dim)
+    mean = 100 if metric == "dot" else 10
+    x = torch.randn(n, dim, generator=g, device="cuda") / dim ** 0.5
+    x += mean * torch.nn.functional.normalize(torch.randn(dim, generator=g, device="cuda"), dim=0)
+    q = x[torch.randint(0, n, (nq,), generator=g, device="cuda")]
+    q = (q + 0.1 * torch.randn(nq, dim, generator=g, device="cuda") / dim ** 0.5).contiguous()
+    torch.cuda.synchronize()
+    idx = FlatIndex(ctx, dim, metric)
+    idx.append_device(x.data_ptr(), n)
+    scanned = equals_fused(idx, q, nq, 10)
+    first = (n + SAMPLE) * nq
+    if products:  # (and few rows kept)
+        assert 2 * first < scanned < 2 * first + nq * 4000
+    else:
+        assert scanned == first + n * nq
+    idx.destroy()
+
+
+def test_only_overflowed_queries_are_run_again(ctx):
+    """Three kinds of queries in turn: close to the first are rows 1e-6 apart
+    (their lists overflow under either bound: slot scans), to the second rows
+    1e-3 apart (fp32 products tell them apart), and the third need no second
+    pass."""
+    import torch
+
+    from browservec_amd import FlatIndex
+
+    dim, n, nq = 64, 80_000, 150
+    say("overflow of some")
+    g = torch.Generator(device="cuda").manual_seed(8)
+
+    def rand(*shape):
+        return torch.randn(*shape, generator=g, device="cuda")
+
+    u, v = torch.linalg.qr(rand(dim, 2)).Q.T
+    i = torch.arange(n, device="cuda")
+    x = torch.nn.functional.normalize(rand(n, dim), dim=1)
+    near_u = (i % 8 == 0) | (i % 4 == 1)  # (the sample takes every fourth row)
+    near_v = i % 4 >= 2
+    x[near_u] = u * (1 + 1e-3 * rand(int(near_u.sum()), 1)) + 1e-3 * rand(int(near_u.sum()), dim) / 8
+    x[near_v] = v + 1e-6 * rand(int(near_v.sum()), dim) / 8
+    q = rand(nq, dim)
+    q -= torch.outer(q @ u, u) + torch.outer(q @ v, v)
+    q = torch.nn.functional.normalize(q, dim=1)
+    q[0::3] = v + 0.01 * rand(50, dim) / 8
+    q[1::3] = u + 0.01 * rand(50, dim) / 8
+    q = q.contiguous()
+    torch.cuda.synchronize()
+    idx = FlatIndex(ctx, dim, "dot")
+    idx.append_device(x.contiguous().data_ptr(), n)
+    scanned = equals_fused(idx, q, nq, 10)
+    least = (n + SAMPLE) * nq + (n + SAMPLE) * 100 + n * 50
+    assert least < scanned < least + 50 * SAMPLE * 2 + nq * 4000
+    idx.destroy()
