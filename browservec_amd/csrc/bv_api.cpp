@@ -2396,16 +2396,29 @@ static int run_ivf_batched(bv_index *idx, const float *d_q, uint32_t nq, uint32_
 
 // ------------------------------------------------------------- slot scans
 // Small batches and short scans: scan_slots (the rows read once for up to
-// four queries) and pick_topk (one workgroup per query).
+// four queries) and pick_topk (one workgroup per query, or a few).
+static bool slots_fit(const bv_index *idx, bool rerank) {
+    return !idx->ivf && idx->rows > 0 && idx->rows < (1ull << 30) &&
+           pick_supported(idx->codec, idx->P, rerank ? idx->dim : 0);
+}
+
 // Which calls take them.  Measured on one MI355X, us a call alone (slot scan
 // against the other path):
 //   against one fused scan per query (2 to 7 queries, or no batch path):
-//     every size and codec, 1M x 768 int8 4 queries 286 / 702, 1-bit 219 /
-//     8,234, 100,000 x 384 int4 fetch 160 one query 57 / 1,108, 100,000 x 300
-//     fp32 256 queries 1,660 / 8,360;
-//   single queries likewise, but for the int8 scan from half a GB on, which
-//     the fused scan's one launch serves in 192 us against 212 (1M x 768;
-//     500,000 rows: 132 / 130);
+//     every size and codec, 1M x 768 int8 4 queries 233 / 702, 1-bit 219 /
+//     8,234, 4M x 1024 int4 724 / 1,414, 100,000 x 384 int4 fetch 160 one query
+//     57 / 1,108, 100,000 x 300 fp32 256 queries 1,660 / 8,360;
+//   single queries likewise, but for 8- and 4-bit scans of which the rows fill
+//     the device long enough for the fused scan's bound to form (a larger fetch
+//     takes longer) and its selection to hide behind them: int8 600,000 x 768
+//     fetch 100 150 / 139, 320 158 / 155, 1M 215 / 197, fetch 512 227 / 251,
+//     4M 680 / 672, fetch 1000 727 / 937 (500,000 129 / 131); int8 symmetric 1M
+//     211 / 196, 500,000 132 / 136; int4 4M x 1024 fetch 160 407 / 374, 512
+//     424 / 403, 1000 452 / 618, 2M 226 / 219, 1M 139 / 143;
+//   1-bit and Hamming scans stay: 4M x 1024 194 / 195 and 156 / 147 at fetch
+//     200, but Hamming 149 / 194 at 100 and 162 / 233 at 320, 1-bit 10M x 256
+//     266 / 279, and with other indexes queried in turn 123 / 148 and 105 / 120;
+//     fp32 ones too (1M x 768 496 / 497, 1M x 300 219 / 249);
 //   against the batched passes: those cost about 140 us of launches and
 //     0.24 us per million codes whatever the batch, a slot scan 45 us and a
 //     time per query, row and 16-byte unit set by its dot products (below):
@@ -2414,13 +2427,15 @@ static int run_ivf_batched(bv_index *idx, const float *d_q, uint32_t nq, uint32_
 //   fp32 batches cost 0.62 us per million elements on top: 100,000 x 384
 //     crosses at 20 (16 queries 129 / 161, 32 183 / 165), 20,000 x 384 at 75
 //     (64 queries 119 / 132).
-static bool slots_fit(const bv_index *idx, bool rerank) {
-    return !idx->ivf && idx->rows > 0 && idx->rows < (1ull << 30) &&
-           pick_supported(idx->codec, idx->P, rerank ? idx->dim : 0);
-}
 static bool slots_route(const bv_index *idx, uint32_t nq, uint32_t kprime, bool rerank, bool batchable) {
     if (!slots_fit(idx, rerank)) return false;
-    if (nq == 1) return !(idx->codec == C_Q8 && idx->rows * idx->row_bytes >= (512ull << 20) && kprime <= 256);
+    if (nq == 1) {
+        const uint64_t bytes = idx->rows * idx->row_bytes;
+        const uint64_t least = idx->codec == C_Q8 || idx->codec == C_I8S ? 512ull << 20
+                               : idx->codec == C_Q4                     ? 1ull << 30
+                                                                        : ~0ull;
+        return bytes < least || kprime > std::min<uint64_t>(512, bytes >> 22);
+    }
     if (!batchable) return true;
     double per;  // us per million (row, unit)
     switch (idx->codec) {
@@ -2440,6 +2455,16 @@ static bool slots_route(const bv_index *idx, uint32_t nq, uint32_t kprime, bool 
     return slots < batch;
 }
 
+// The re-ranks' counters, zero when a kernel starts (it leaves them so).
+static int rerank_tickets(bv_index *idx, uint32_t nq) {
+    const size_t old = idx->rr_tickets.cap;
+    HIPX(idx->dev, idx->rr_tickets.ensure((size_t)nq * 4, 0, idx->stream), "scratch");
+    if (idx->rr_tickets.cap != old)
+        HIPX(idx->dev, launch_zero(idx->rr_tickets.p, idx->rr_tickets.cap, idx->stream), "scratch");
+    return BV_OK;
+}
+
+constexpr uint32_t PICK_SPLIT = 8;
 static int run_slots(bv_index *idx, const float *d_q, uint32_t nq, uint32_t kprime, uint32_t k_out, bool rerank,
                      const uint32_t *d_mask, uint64_t mask_bits, uint32_t *d_rows, float *d_scores, uint32_t *d_n) {
     hipStream_t s = idx->stream;
@@ -2489,6 +2514,20 @@ static int run_slots(bv_index *idx, const float *d_q, uint32_t nq, uint32_t kpri
     p.is_int = idx->codec == C_HAM || idx->codec == C_I8S;
     p.kk = kprime;
     p.k_out = k_out;
+    // Few queries leave the selection's workgroups alone on their CUs: where the
+    // re-rank has much to read (200 rows x 1,024 took 20 us of a call), several
+    // workgroups share it; each selects for itself, which costs nothing while
+    // the CUs are free.  4M x 1024 1-bit, us a call alone, one workgroup, four,
+    // eight: fetch 200 201 / 193 / 188, 1000 358 / 306 / 298, Hamming 163 / 156 /
+    // 155; 250,000 x 768 int8 fetch 100 92 / 88 / 88, fetch 40 no difference.
+    p.split = rerank && nq < MQ_MIN_Q && (uint64_t)kprime * idx->dim >= 65536 ? PICK_SPLIT : 1;
+    if (p.split > 1) {
+        HIPX(idx->dev, idx->rr_keys.ensure((size_t)chunk * kprime * 8, 0, s), "scratch");
+        rc = rerank_tickets(idx, chunk);
+        if (rc) return rc;
+        p.rr_keys = idx->rr_keys.as<uint64_t>();
+        p.tickets = idx->rr_tickets.as<uint32_t>();
+    }
     timing_begin(idx);
     for (uint32_t q0 = 0; q0 < nq; q0 += chunk) {
         a.nq = std::min(chunk, nq - q0);
@@ -2965,12 +3004,8 @@ extern "C" int bv_index_rerank(bv_index *idx, const float *q, const uint32_t *ca
     const uint32_t *d_cand_n = (const uint32_t *)idx->io.put(&n_cand, 4);
     HIPX(idx->dev, idx->io.send(idx->stream), "upload");
     HIPX(idx->dev, idx->rr_keys.ensure((size_t)n_cand * 8, 0, idx->stream), "scratch");
-    {
-        const size_t old = idx->rr_tickets.cap;
-        HIPX(idx->dev, idx->rr_tickets.ensure(4, 0, idx->stream), "scratch");
-        if (idx->rr_tickets.cap != old)
-            HIPX(idx->dev, hipMemsetAsync(idx->rr_tickets.p, 0, idx->rr_tickets.cap, idx->stream), "scratch");
-    }
+    rc = rerank_tickets(idx, 1);
+    if (rc) return rc;
     const size_t rb = HostIo::pad((size_t)kk * 4);
     HIPX(idx->dev, idx->io.out.ensure(2 * rb + 4), "pinned buffer");
     char *out = (char *)idx->io.out.p;
@@ -3036,6 +3071,7 @@ static int exact_list_topk(bv_index *idx, const float *d_q, const uint32_t *d_li
         o_n[1] = 0;  // set when a listed row is out of range
         p.kk = kk;
         p.k_out = kk;
+        p.split = 1;
         p.out_rows = (uint32_t *)out;
         p.out_scores = (float *)(out + rb);
         p.out_n = o_n;

@@ -163,6 +163,9 @@ struct PickArgs {
     uint32_t *out_rows;       // [nq][k_out]
     float *out_scores;
     uint32_t *out_n;
+    uint32_t split;           // workgroups that share a query's re-rank (1: the next two are not used)
+    uint64_t *rr_keys;        // [nq][kk] their exact keys
+    uint32_t *tickets;        // [nq] zero (and left so)
 };
 // Store.dotRow / Store.l2Row of the rows cand[0, n) (a.codes the fp32 rows of
 // a.padded_dim floats; slots of a multiple of 16 rows, one part each) against

@@ -307,11 +307,25 @@ template <int LPR> __global__ __launch_bounds__(PICK_THREADS) void pick_topk(Pic
 
     // ---- the exact re-rank, and the results ----
     if (a.rr_src) {
-        for (uint32_t c0 = (uint32_t)wave * 16; c0 < m; c0 += PICK_WAVES * 16) {
+        const uint32_t ns = gridDim.y;
+        uint64_t *rr = ns > 1 ? a.rr_keys + (uint64_t)q * kk : nullptr;
+        for (uint32_t c0 = ((uint32_t)wave * ns + blockIdx.y) * 16; c0 < m; c0 += PICK_WAVES * ns * 16) {
             const uint32_t ci = c0 + (uint32_t)(lane >> 2);
             const uint32_t row = key_row(L.keys[ci < m ? ci : c0]);
             const uint64_t ek = exact_keys16(a.rr_src, a.rr_dim, rq, pick_smem, row, L.tiles + wave * EXACT_TILE, lane);
-            if ((lane & 3) == 0 && ci < m) L.keys[ci] = ek;  // (each entry read and written by its own lanes)
+            if ((lane & 3) == 0 && ci < m) {
+                if (rr) store_shared(&rr[ci], ek);
+                else L.keys[ci] = ek;  // (each entry read and written by its own lanes)
+            }
+        }
+        if (rr) {  // the last workgroup ranks all of them
+            wait_stores_done();
+            __syncthreads();
+            if (tid == 0) L.sum = atomicAdd(&a.tickets[q], 1u) == ns - 1;
+            __syncthreads();
+            if (!L.sum) return;
+            if (tid == 0) a.tickets[q] = 0;
+            for (uint32_t i = tid; i < m; i += PICK_THREADS) L.keys[i] = load_shared(&rr[i]);
         }
         __syncthreads();
         uint32_t npow = 2;
@@ -391,7 +405,8 @@ hipError_t launch_pick_topk(const PickArgs &a, hipStream_t s) {
     size_t lds = a.rr_src ? 16 * (size_t)exact_q_stride(a.rr_dim) : 0;
     if (a.q1p) lds += q1p_lut_bytes(a.s.padded_dim);
     if (lds + sizeof(PickLds) > 160 * 1024) return hipErrorInvalidValue;
-    const dim3 g(a.s.nq), wg(PICK_THREADS);
+    if (a.split == 0 || (a.split > 1 && (!a.rr_src || !a.rr_keys || !a.tickets))) return hipErrorInvalidValue;
+    const dim3 g(a.s.nq, a.split), wg(PICK_THREADS);
     if (!a.q1p) hipLaunchKernelGGL((pick_topk<0>), g, wg, lds, s, a);
     else {
         Layout L;

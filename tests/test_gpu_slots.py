@@ -169,3 +169,43 @@ def test_more_queries_than_a_launch_takes(ctx):
     for a, b in zip(*out):
         assert np.array_equal(a, b)
     idx.destroy()
+
+
+@pytest.mark.parametrize("kind,n,dim,fetch", [("8", 600_000, 1024, 100), ("8int8sym", 600_000, 1024, 100),
+                                              ("4", 2_100_000, 1024, 160), ("8", 600_000, 1024, 300)])
+def test_single_queries_over_large_codes(ctx, kind, n, dim, fetch):
+    """Single queries on either side of the sizes at which the fused scan takes
+    them, against the slot scan of two queries at once."""
+    import torch
+
+    say("large single", kind, n, fetch)
+    idx, x, q = make(ctx, kind, dim, n, 5)
+    del x
+    out = []
+    for width in (1, 2):
+        rows = torch.full((4, 10), -1, dtype=torch.int32, device="cuda")
+        scores = torch.zeros(4, 10, device="cuda")
+        cnt = torch.zeros(4, dtype=torch.int32, device="cuda")
+        torch.cuda.synchronize()
+        for i in range(0, 4, width):
+            idx.search_device(q[i:].data_ptr(), width, fetch, 10, rows[i:].data_ptr(), scores[i:].data_ptr(),
+                              cnt[i:].data_ptr())
+        idx.sync()
+        out.append([rows.cpu().numpy(), scores.cpu().numpy().view(np.uint32), cnt.cpu().numpy()])
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+    idx.destroy()
+    torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("kind,dim,n,nq,fetch,k", [("8", 1000, 3000, 1, 66, 10), ("4", 1024, 5000, 7, 1024, 1024),
+                                                   ("1", 768, 40_000, 2, 96, 96), ("1hamming", 1024, 100, 3, 100, 5),
+                                                   ("8int8sym", 2048, 9000, 2, 33, 33)])
+def test_shared_rerank_equals_the_fused_scan(ctx, kind, dim, n, nq, fetch, k):
+    """A re-rank that several workgroups share (65,536 elements and more, up to
+    seven queries), fewer sixteens of rows than workgroups among them."""
+    say("shared re-rank", kind, dim, n, nq, fetch, k)
+    idx, x, q = make(ctx, kind, dim, n, dim + n)
+    both_equal(idx, q[:nq].contiguous(), nq, fetch, k)
+    both_equal(idx, q[8:8 + nq].contiguous(), nq, fetch, k)  # (the counters are as they were)
+    idx.destroy()
