@@ -41,6 +41,7 @@ struct bv_device {
     bool lost = false;
     bool inject_append_oom = false;  // bv_debug_inject: fail the next append's allocation
     bool inject_append_late = false; // bv_debug_inject: fail the next append after its rows are encoded
+    bool inject_slots_oom = false;   // bv_debug_inject: fail the next slot scan's allocation
     void *scratch = nullptr;         // this GPU's copy of the no-allocation scratch array
 };
 
@@ -329,6 +330,7 @@ extern "C" int bv_debug_inject(bv_device *dev, int what) {
     case BV_INJECT_LOST: dev->lost = true; return BV_OK;
     case BV_INJECT_APPEND_OOM: dev->inject_append_oom = true; return BV_OK;
     case BV_INJECT_APPEND_LATE: dev->inject_append_late = true; return BV_OK;
+    case BV_INJECT_SLOTS_OOM: dev->inject_slots_oom = true; return BV_OK;
     default: return fail(BV_E_INVALID, "unknown injection %d", what);
     }
 }
@@ -2486,6 +2488,10 @@ static int run_slots(bv_index *idx, const float *d_q, uint32_t nq, uint32_t kpri
     // (a launch takes up to SLOTS_MAX_NQ queries: its grid's second dimension)
     const uint32_t chunk = (uint32_t)std::max<uint64_t>(
         1, std::min<uint64_t>(std::min(nq, SLOTS_MAX_NQ), (256ull << 20) / (per * 4)));
+    if (idx->dev->inject_slots_oom) {
+        idx->dev->inject_slots_oom = false;
+        return fail(BV_E_OOM, "slot scan: injected out of device memory");
+    }
     HIPX(idx->dev, idx->sl_ord.ensure((size_t)chunk * per * 4, 0, s), "scratch");
     HIPX(idx->dev, idx->sl_best.ensure((size_t)chunk * nslots * 8, 0, s), "scratch");
     HIPX(idx->dev, idx->sl_part.ensure((size_t)chunk * nslots * nsub * 4, 0, s), "scratch");
@@ -2651,6 +2657,11 @@ static int rerun_overflowed(bv_index *idx, const float *d_q, const std::vector<u
     } else if (slots_fit(idx, rerank)) {
         rc = run_slots(idx, q, m, kprime, k_out, rerank, nullptr, 0, rows, scores, n);
     } else {
+        rc = BV_E_OOM;
+    }
+    if (rc == BV_E_OOM) {  // (no slot scan, or no room for one)
+        (void)hipGetLastError();
+        rc = BV_OK;
         for (uint32_t i = 0; i < m && !rc; i += 64)
             rc = run_fused(idx, q + (size_t)i * dim, std::min(64u, m - i), kprime, k_out, rerank, nullptr, 0,
                            rows + (size_t)i * k_out, scores + (size_t)i * k_out, n + i);
@@ -2689,7 +2700,11 @@ static int run_pipeline(bv_index *idx, const float *d_q, uint32_t nq, uint32_t k
     if (!streams && slots_route(idx, nq, kprime, rerank, mq_eligible(idx, nq, d_mask))) {
         int rc = lanes_join(idx);
         if (rc) return rc;
-        return run_slots(idx, d_q, nq, kprime, k_out, rerank, d_mask, mask_bits, d_rows, d_scores, d_n);
+        rc = run_slots(idx, d_q, nq, kprime, k_out, rerank, d_mask, mask_bits, d_rows, d_scores, d_n);
+        // (the order words, 4 bytes a row and query, may not fit a device that
+        // the rows fill: the other paths need less)
+        if (rc != BV_E_OOM) return rc;
+        (void)hipGetLastError();
     }
     if (mq_eligible(idx, nq, d_mask)) {
         int rc = lanes_join(idx);  // the batch path shares the index stream's scratch and outputs

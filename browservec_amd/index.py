@@ -64,10 +64,11 @@ class DeviceContext:
 
     def debug_inject(self, what: str) -> None:
         """Force the device-lost state ('lost'), a failed allocation on the
-        next append ('append_oom') or a failure of the next append after its
-        rows are encoded ('append_late') from the host; no device work is made
-        to fail."""
-        L.check(self.lib.bv_debug_inject(self.handle, {"lost": 1, "append_oom": 2, "append_late": 3}[what]))
+        next append ('append_oom') or slot scan ('slots_oom') or a failure of
+        the next append after its rows are encoded ('append_late') from the
+        host; no device work is made to fail."""
+        flags = {"lost": 1, "append_oom": 2, "append_late": 3, "slots_oom": 4}
+        L.check(self.lib.bv_debug_inject(self.handle, flags[what]))
 
     def destroy(self) -> None:
         if self.handle:

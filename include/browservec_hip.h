@@ -138,6 +138,7 @@ int bv_device_is_lost(const bv_device *dev, int *lost);
 #define BV_INJECT_APPEND_OOM 2 /* the next append fails as if a device allocation failed; the index is unchanged */
 #define BV_INJECT_APPEND_LATE 3 /* the next append fails after its rows are uploaded and encoded, before its
                                  * reservoir sample and lists are committed; the index is unchanged */
+#define BV_INJECT_SLOTS_OOM 4 /* the next slot scan's scratch does not fit: the query takes another path */
 int bv_debug_inject(bv_device *dev, int what);
 /* Device name, compute-unit count and HBM size. */
 int bv_device_info(const bv_device *dev, char *name, uint32_t name_len, uint32_t *cu_count, uint64_t *hbm_bytes);

@@ -171,6 +171,22 @@ def test_more_queries_than_a_launch_takes(ctx):
     idx.destroy()
 
 
+@pytest.mark.parametrize("kind,dim,n,nq,fetch", [("8", 768, 20_000, 1, 60), ("1hamming", 256, 30_000, 5, 100),
+                                                 ("4", 384, 20_000, 10, 40), ("cosine", 100, 25_000, 3, 0)])
+def test_no_room_for_order_words(ctx, kind, dim, n, nq, fetch):
+    """Where a slot scan's scratch does not fit, the query takes the path it
+    would take without one and answers the same."""
+    say("slots out of memory", kind, nq)
+    idx, x, q = make(ctx, kind, dim, n, 21)
+    qh = q[:nq].cpu().numpy()
+    want = idx.search(qh, fetch, 10)
+    ctx.debug_inject("slots_oom")
+    got = idx.search(qh, fetch, 10)
+    for a, b in zip(want, got):
+        assert np.array_equal(np.asarray(a).view(np.uint32), np.asarray(b).view(np.uint32))
+    idx.destroy()
+
+
 @pytest.mark.parametrize("kind,n,dim,fetch", [("8", 600_000, 1024, 100), ("8int8sym", 600_000, 1024, 100),
                                               ("4", 2_100_000, 1024, 160), ("8", 600_000, 1024, 300)])
 def test_single_queries_over_large_codes(ctx, kind, n, dim, fetch):
