@@ -13,6 +13,7 @@
 #include <cstddef>
 #include <cstdio>
 #include <cstring>
+#include <initializer_list>
 #include <mutex>
 #include <thread>
 #include <string>
@@ -139,8 +140,10 @@ struct HostBuf {
 // buffer and brought to the device by one small kernel; the last kernels of
 // the call write their results to pinned memory (coherent, so they are in
 // place when the stream is).  A pageable copy each way cost 8-12 us a piece:
-// 3,000 listed rows took 116 us a call, 36 of them kernels.  The buffers are
-// free again when the call has waited for its stream.
+// 3,000 listed rows took 116 us a call, 36 of them kernels (42 now).  The buffers are
+// free again when the call has waited for its stream.  Inputs above
+// 8 MB are copied from where they are: the pinned memory that stays with an
+// index or a graph is bounded.
 struct PinnedBuf {
     void *p = nullptr;
     size_t cap = 0;
@@ -160,24 +163,42 @@ struct PinnedBuf {
     }
 };
 struct HostIo {
+    static constexpr size_t PINNED_MAX = 8 << 20;
     PinnedBuf in, out;
     DevBuf dev;
-    size_t used = 0;
+    size_t used = 0, large = 0;  // the next pinned input's place, the next larger one's
+    hipStream_t stream = nullptr;
+    hipError_t err = hipSuccess;
     static size_t pad(size_t bytes) { return (bytes + 255) & ~size_t(255); }
-    // room for a call's inputs: the padded sizes' sum
-    hipError_t begin(size_t bytes, hipStream_t s) {
+    // room for a call's inputs
+    hipError_t begin(std::initializer_list<size_t> sizes, hipStream_t s) {
+        size_t small = 0, total = 0;
+        for (const size_t b : sizes) {
+            total += pad(b);
+            if (b <= PINNED_MAX) small += pad(b);
+        }
         used = 0;
-        const hipError_t e = in.ensure(bytes);
-        return e == hipSuccess ? dev.ensure(bytes, 0, s) : e;
+        large = small;
+        stream = s;
+        err = in.ensure(small);
+        if (err == hipSuccess) err = dev.ensure(total, 0, s);
+        return err;
     }
     // the input's place on the device, valid after send()
     void *put(const void *src, size_t bytes) {
-        std::memcpy((char *)in.p + used, src, bytes);
+        if (bytes > PINNED_MAX) {
+            void *d = (char *)dev.p + large;
+            large += pad(bytes);
+            const hipError_t e = hipMemcpyAsync(d, src, bytes, hipMemcpyHostToDevice, stream);
+            if (err == hipSuccess) err = e;
+            return d;
+        }
+        if (bytes) std::memcpy((char *)in.p + used, src, bytes);
         void *d = (char *)dev.p + used;
         used += pad(bytes);
         return d;
     }
-    hipError_t send(hipStream_t s) { return launch_copy_in(dev.p, in.p, used, s); }
+    hipError_t send() { return err != hipSuccess ? err : launch_copy_in(dev.p, in.p, used, stream); }
 };
 
 // Queries of a batch that are run again, and their results.
@@ -2737,14 +2758,14 @@ static int host_query(bv_index *idx, const float *q, uint32_t nq, uint32_t kprim
     hipStream_t st = idx->stream;
     const size_t qbytes = (size_t)nq * idx->dim * 4, mbytes = mask ? mask_words * 4 : 0;
     const size_t rbytes = HostIo::pad((size_t)nq * k_out * 4);
-    HIPX(idx->dev, idx->io.begin(HostIo::pad(qbytes) + HostIo::pad(mbytes), st), "query buffer");
+    HIPX(idx->dev, idx->io.begin({qbytes, mbytes}, st), "query buffer");
     HIPX(idx->dev, idx->io.out.ensure(2 * rbytes + (size_t)nq * 4), "pinned buffer");
     uint32_t *o_rows = (uint32_t *)idx->io.out.p, *o_n = (uint32_t *)((char *)idx->io.out.p + 2 * rbytes);
     float *o_scores = (float *)((char *)idx->io.out.p + rbytes);
     const float *d_q = (const float *)idx->io.put(q, qbytes);
     const uint32_t *d_mask = mask ? (const uint32_t *)idx->io.put(mask, mbytes) : nullptr;
     HIPX(idx->dev, hipEventRecord(idx->ev0, st), "event");
-    HIPX(idx->dev, idx->io.send(st), "query upload");
+    HIPX(idx->dev, idx->io.send(), "query upload");
     rc = run_pipeline(idx, d_q, nq, kprime, k_out, rerank, d_mask, mask ? mask_words * 32 : 0, o_rows, o_scores, o_n);
     if (rc) {
         (void)hipStreamSynchronize(st);  // (launched kernels may still read the buffers)
@@ -3012,12 +3033,11 @@ extern "C" int bv_index_rerank(bv_index *idx, const float *q, const uint32_t *ca
         return BV_OK;
     }
     const size_t qb = (size_t)idx->dim * 4;
-    HIPX(idx->dev, idx->io.begin(HostIo::pad(qb) + HostIo::pad((size_t)n_cand * 4) + HostIo::pad(4), idx->stream),
-         "query buffer");
+    HIPX(idx->dev, idx->io.begin({qb, (size_t)n_cand * 4, 4}, idx->stream), "query buffer");
     const float *d_q = (const float *)idx->io.put(q, qb);
     const uint32_t *d_cand = (const uint32_t *)idx->io.put(cand, (size_t)n_cand * 4);
     const uint32_t *d_cand_n = (const uint32_t *)idx->io.put(&n_cand, 4);
-    HIPX(idx->dev, idx->io.send(idx->stream), "upload");
+    HIPX(idx->dev, idx->io.send(), "upload");
     HIPX(idx->dev, idx->rr_keys.ensure((size_t)n_cand * 8, 0, idx->stream), "scratch");
     rc = rerank_tickets(idx, 1);
     if (rc) return rc;
@@ -3133,10 +3153,10 @@ extern "C" int bv_index_query_rows(bv_index *idx, const float *q, const uint32_t
         return BV_OK;
     }
     const size_t qb = (size_t)idx->dim * 4;
-    HIPX(idx->dev, idx->io.begin(HostIo::pad(qb) + HostIo::pad(n_list * 4), idx->stream), "query buffer");
+    HIPX(idx->dev, idx->io.begin({qb, n_list * 4}, idx->stream), "query buffer");
     const float *d_q = (const float *)idx->io.put(q, qb);
     const uint32_t *d_list = (const uint32_t *)idx->io.put(list, n_list * 4);
-    HIPX(idx->dev, idx->io.send(idx->stream), "upload");
+    HIPX(idx->dev, idx->io.send(), "upload");
     return exact_list_topk(idx, d_q, d_list, n_list, k, rows, scores, n_out);
 }
 
@@ -3156,10 +3176,10 @@ extern "C" int bv_index_query_rows_masked(bv_index *idx, const float *q, const u
     }
     hipStream_t s = idx->stream;
     const size_t qb = (size_t)idx->dim * 4;
-    HIPX(idx->dev, idx->io.begin(HostIo::pad(qb) + HostIo::pad(words * 4), s), "query buffer");
+    HIPX(idx->dev, idx->io.begin({qb, words * 4}, s), "query buffer");
     const float *d_q = (const float *)idx->io.put(q, qb);
     const uint32_t *d_mask = (const uint32_t *)idx->io.put(mask_words, words * 4);
-    HIPX(idx->dev, idx->io.send(s), "upload");
+    HIPX(idx->dev, idx->io.send(), "upload");
     HIPX(idx->dev, idx->sel_popc.ensure(words * 4, 0, s), "scratch");
     HIPX(idx->dev, idx->sel_off.ensure(words * 4, 0, s), "scratch");
     HIPX(idx->dev, idx->sel_misc.ensure(8, 0, s), "scratch");
@@ -3777,10 +3797,10 @@ int graph_run(bv_graph *g, const float *queries, uint32_t nq, const uint32_t *en
               uint32_t ef_active, uint32_t iter_cap, uint32_t k, uint32_t stride, bool beams) {
     hipStream_t s = g->stream;
     const size_t qb = (size_t)nq * g->dim * 4, eb = (size_t)n_entries * 4;
-    HIPX(g->dev, g->io.begin(HostIo::pad(qb) + HostIo::pad(eb), s), "query buffer");
+    HIPX(g->dev, g->io.begin({qb, eb}, s), "query buffer");
     const float *d_q = (const float *)g->io.put(queries, qb);
     const uint32_t *d_e = (const uint32_t *)g->io.put(entries, eb);
-    HIPX(g->dev, g->io.send(s), "upload");
+    HIPX(g->dev, g->io.send(), "upload");
     GraphArgs a{};
     a.corpus = g->corpus.as<float>();
     a.dim = g->dim;
@@ -3902,14 +3922,19 @@ extern "C" int bv_graph_search(bv_graph *g, const float *queries, uint32_t nq, u
     }
     uint32_t seeds[8];
     const uint32_t ns = graph_seeds(entry, g->graph_rows, seeds);
-    rc = graph_run(g, queries, nq, seeds, ns, efA, efA, kk, k, false);
-    if (rc) return rc;
-    HIPX(g->dev, hipStreamSynchronize(g->stream), "graph search");
-    const size_t rb = HostIo::pad((size_t)nq * k * 4);
-    const char *out = (const char *)g->io.out.p;
-    std::memcpy(rows, out, (size_t)nq * k * 4);
-    std::memcpy(scores, out + rb, (size_t)nq * k * 4);
-    std::memcpy(n_out, out + 2 * rb, (size_t)nq * 4);
+    // (so many queries at a time that the pinned results stay within 8 MB)
+    const uint32_t chunk = (uint32_t)std::max<size_t>(1, HostIo::PINNED_MAX / ((size_t)k * 8 + 4));
+    for (uint32_t q0 = 0; q0 < nq; q0 += chunk) {
+        const uint32_t m = std::min(chunk, nq - q0);
+        rc = graph_run(g, queries + (size_t)q0 * g->dim, m, seeds, ns, efA, efA, kk, k, false);
+        if (rc) return rc;
+        HIPX(g->dev, hipStreamSynchronize(g->stream), "graph search");
+        const size_t rb = HostIo::pad((size_t)m * k * 4);
+        const char *out = (const char *)g->io.out.p;
+        std::memcpy(rows + (size_t)q0 * k, out, (size_t)m * k * 4);
+        std::memcpy(scores + (size_t)q0 * k, out + rb, (size_t)m * k * 4);
+        std::memcpy(n_out + q0, out + 2 * rb, (size_t)m * 4);
+    }
     return BV_OK;
 }
 
