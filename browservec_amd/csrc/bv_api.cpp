@@ -141,7 +141,7 @@ struct HostBuf {
 // the call write their results to pinned memory (coherent, so they are in
 // place when the stream is).  A pageable copy each way cost 8-12 us a piece:
 // 3,000 listed rows took 116 us a call, 36 of them kernels (42 now).  The buffers are
-// free again when the call has waited for its stream.  Inputs above
+// free again when the call has waited for its stream (IoCall).  Inputs above
 // 8 MB are copied from where they are: the pinned memory that stays with an
 // index or a graph is bounded.
 struct PinnedBuf {
@@ -199,6 +199,21 @@ struct HostIo {
         return d;
     }
     hipError_t send() { return err != hipSuccess ? err : launch_copy_in(dev.p, in.p, used, stream); }
+};
+// A host call from its first input to its last wait: one that fails in between
+// waits as well, since kernels and copies under way may still use the call's
+// buffers and its caller's.
+struct IoCall {
+    hipStream_t s;
+    bool waited = false;
+    explicit IoCall(hipStream_t s) : s(s) {}
+    ~IoCall() {
+        if (!waited) (void)hipStreamSynchronize(s);
+    }
+    int done(int rc) {
+        waited = rc == BV_OK;
+        return rc;
+    }
 };
 
 // Queries of a batch that are run again, and their results.
@@ -2758,6 +2773,7 @@ static int host_query(bv_index *idx, const float *q, uint32_t nq, uint32_t kprim
     hipStream_t st = idx->stream;
     const size_t qbytes = (size_t)nq * idx->dim * 4, mbytes = mask ? mask_words * 4 : 0;
     const size_t rbytes = HostIo::pad((size_t)nq * k_out * 4);
+    IoCall call(st);
     HIPX(idx->dev, idx->io.begin({qbytes, mbytes}, st), "query buffer");
     HIPX(idx->dev, idx->io.out.ensure(2 * rbytes + (size_t)nq * 4), "pinned buffer");
     uint32_t *o_rows = (uint32_t *)idx->io.out.p, *o_n = (uint32_t *)((char *)idx->io.out.p + 2 * rbytes);
@@ -2767,12 +2783,10 @@ static int host_query(bv_index *idx, const float *q, uint32_t nq, uint32_t kprim
     HIPX(idx->dev, hipEventRecord(idx->ev0, st), "event");
     HIPX(idx->dev, idx->io.send(), "query upload");
     rc = run_pipeline(idx, d_q, nq, kprime, k_out, rerank, d_mask, mask ? mask_words * 32 : 0, o_rows, o_scores, o_n);
-    if (rc) {
-        (void)hipStreamSynchronize(st);  // (launched kernels may still read the buffers)
-        return rc;
-    }
+    if (rc) return rc;
     HIPX(idx->dev, hipEventRecord(idx->ev1, st), "event");
     HIPX(idx->dev, hipStreamSynchronize(st), "query");
+    call.done(BV_OK);
     timing_collect(idx);
     float gms = 0;
     (void)hipEventElapsedTime(&gms, idx->ev0, idx->ev1);
@@ -3033,6 +3047,7 @@ extern "C" int bv_index_rerank(bv_index *idx, const float *q, const uint32_t *ca
         return BV_OK;
     }
     const size_t qb = (size_t)idx->dim * 4;
+    IoCall call(idx->stream);
     HIPX(idx->dev, idx->io.begin({qb, (size_t)n_cand * 4, 4}, idx->stream), "query buffer");
     const float *d_q = (const float *)idx->io.put(q, qb);
     const uint32_t *d_cand = (const uint32_t *)idx->io.put(cand, (size_t)n_cand * 4);
@@ -3060,6 +3075,7 @@ extern "C" int bv_index_rerank(bv_index *idx, const float *q, const uint32_t *ca
     r.out_n = (uint32_t *)(out + 2 * rb);
     HIPX(idx->dev, launch_rerank(r, 1, idx->stream), "rerank kernel");
     HIPX(idx->dev, hipStreamSynchronize(idx->stream), "rerank");
+    call.done(BV_OK);
     *n_out = *r.out_n;
     std::memcpy(rows, r.out_rows, (size_t)*n_out * 4);
     std::memcpy(scores, r.out_scores, (size_t)*n_out * 4);
@@ -3153,11 +3169,12 @@ extern "C" int bv_index_query_rows(bv_index *idx, const float *q, const uint32_t
         return BV_OK;
     }
     const size_t qb = (size_t)idx->dim * 4;
+    IoCall call(idx->stream);
     HIPX(idx->dev, idx->io.begin({qb, n_list * 4}, idx->stream), "query buffer");
     const float *d_q = (const float *)idx->io.put(q, qb);
     const uint32_t *d_list = (const uint32_t *)idx->io.put(list, n_list * 4);
     HIPX(idx->dev, idx->io.send(), "upload");
-    return exact_list_topk(idx, d_q, d_list, n_list, k, rows, scores, n_out);
+    return call.done(exact_list_topk(idx, d_q, d_list, n_list, k, rows, scores, n_out));
 }
 
 extern "C" int bv_index_query_rows_masked(bv_index *idx, const float *q, const uint32_t *mask_words, uint64_t n_words,
@@ -3176,6 +3193,7 @@ extern "C" int bv_index_query_rows_masked(bv_index *idx, const float *q, const u
     }
     hipStream_t s = idx->stream;
     const size_t qb = (size_t)idx->dim * 4;
+    IoCall call(s);
     HIPX(idx->dev, idx->io.begin({qb, words * 4}, s), "query buffer");
     const float *d_q = (const float *)idx->io.put(q, qb);
     const uint32_t *d_mask = (const uint32_t *)idx->io.put(mask_words, words * 4);
@@ -3203,9 +3221,9 @@ extern "C" int bv_index_query_rows_masked(bv_index *idx, const float *q, const u
     HIPX(idx->dev, hipStreamSynchronize(s), "mask rows");
     if (n_list == 0) {
         *n_out = 0;
-        return BV_OK;
+        return call.done(BV_OK);
     }
-    return exact_list_topk(idx, d_q, idx->sel_list.as<uint32_t>(), n_list, k, rows, scores, n_out);
+    return call.done(exact_list_topk(idx, d_q, idx->sel_list.as<uint32_t>(), n_list, k, rows, scores, n_out));
 }
 
 // Dense scores of one query for every row (the scan's score for each row),
@@ -3926,9 +3944,11 @@ extern "C" int bv_graph_search(bv_graph *g, const float *queries, uint32_t nq, u
     const uint32_t chunk = (uint32_t)std::max<size_t>(1, HostIo::PINNED_MAX / ((size_t)k * 8 + 4));
     for (uint32_t q0 = 0; q0 < nq; q0 += chunk) {
         const uint32_t m = std::min(chunk, nq - q0);
+        IoCall call(g->stream);
         rc = graph_run(g, queries + (size_t)q0 * g->dim, m, seeds, ns, efA, efA, kk, k, false);
         if (rc) return rc;
         HIPX(g->dev, hipStreamSynchronize(g->stream), "graph search");
+        call.done(BV_OK);
         const size_t rb = HostIo::pad((size_t)m * k * 4);
         const char *out = (const char *)g->io.out.p;
         std::memcpy(rows + (size_t)q0 * k, out, (size_t)m * k * 4);
@@ -3950,11 +3970,12 @@ extern "C" int bv_graph_search_beams(bv_graph *g, const float *queries, uint32_t
     if (g->corpus_rows == 0 || g->graph_rows == 0)
         return fail(BV_E_STATE, "graph search needs corpus rows and an uploaded adjacency");
     if (ef == 0 || ef > GRAPH_EF_CAP) return fail(BV_E_INVALID, "ef must be 1..%u, got %u", GRAPH_EF_CAP, ef);
+    IoCall call(g->stream);
     rc = graph_run(g, queries, nq, entries, std::min(n_entries, 64u), ef, iter_cap, 0, 0, true);
     if (rc) return rc;
     const size_t b = (size_t)nq * GRAPH_EF_CAP * 4;
     HIPX(g->dev, hipMemcpyAsync(beam_dist, g->beam_d.p, b, hipMemcpyDeviceToHost, g->stream), "download");
     HIPX(g->dev, hipMemcpyAsync(beam_id, g->beam_i.p, b, hipMemcpyDeviceToHost, g->stream), "download");
     HIPX(g->dev, hipStreamSynchronize(g->stream), "graph search");
-    return BV_OK;
+    return call.done(BV_OK);
 }
