@@ -1,6 +1,8 @@
-"""Query batches on the matrix-core paths against the same queries run one at
-a time through the fused single-query scan (src/index.ts:473-517: a batch
-must answer exactly as its queries would alone).  int8 / int4 keys are formed
+"""Query batches against the same queries run one at a time
+(src/index.ts:473-517: a batch must answer exactly as its queries would alone),
+whichever way each goes: at most of these sizes both are slot scans, and the
+matrix-core passes are held to at larger ones in test_gpu_batch_routes.py and
+test_gpu_batched_f32.py.  int8 / int4 keys are formed
 by the same f64 combine of exact int32 level dots in both paths; fp32 batches
 re-score the matrix-core survivors with the single-query arithmetic.  Rows
 and score bits must be identical, including re-ranked scores."""

@@ -9,6 +9,8 @@ from tests.helpers import need_gpu, say
 
 pytestmark = pytest.mark.gpu
 
+SAMPLE = 16384  # rows of the batch passes' sample
+
 
 @pytest.fixture(scope="module")
 def ctx():
@@ -22,6 +24,8 @@ def ctx():
 
 def same_as_singles(idx, qs, k, which):
     batch = idx.query_batch(qs, len(qs), k)
+    # (the prefilter's passes scan a sample besides the rows)
+    assert idx.stats()["last_scanned_rows"] > (idx.size + SAMPLE) * len(qs)
     for i in which:
         one = idx.query(qs[i], k)
         assert [h.row for h in batch[i]] == [h.row for h in one], i
@@ -113,9 +117,6 @@ def test_large_k_batches_bound_their_scratch(ctx):
         assert np.array_equal(r[0], rows[i].cpu().numpy().view(np.uint32)), i
         assert np.array_equal(s[0].view(np.uint32), scores[i].cpu().numpy().view(np.uint32)), i
     idx.destroy()
-
-
-SAMPLE = 16384  # rows of the batch passes' sample
 
 
 def device_rows(idx, q, nq, k, width):
