@@ -3095,9 +3095,10 @@ static int exact_list_topk(bv_index *idx, const float *d_q, const uint32_t *d_li
                     (unsigned long long)idx->rows);
     };
     // one wave per sixteen rows, then the selection of the slot scans: 3,000
-    // rows x 768, k 10, in 116 us a call against 134 with a lane per row and
-    // a sort of every key (100,000 rows: 172 / 273).  Larger k, longer lists
-    // and dimensions past LDS keep the sort.
+    // rows x 768, k 10, 116 us a call against 134 with a lane per row and a
+    // sort of every key (100,000 rows: 172 / 273), 42 since inputs and results
+    // go through pinned memory.  Larger k, longer lists and dimensions past LDS
+    // keep the sort.
     if (kk <= (uint32_t)MAX_KPRIME && n_list < (1ull << 30) && idx->dim <= 4096 && idx->rows > 0) {
         uint32_t rw = 16;
         while ((n_list + rw - 1) / rw > SLOTS_MAX / 2) rw *= 2;
@@ -3780,7 +3781,7 @@ extern "C" int bv_index_export_ivf(bv_index *idx, float *centroids, uint32_t *li
 // ------------------------------------------------------------ graph search
 // HNSWGpuSearcher (src/index/hnswGpu.ts:28-244): the corpus rows and the
 // layer-0 adjacency the host's HNSW build hands over, and the beam search of
-// a batch of queries in one launch (one wave per query).
+// a batch of queries in one launch (one workgroup per query).
 struct bv_graph {
     mutable std::mutex mu;
     bv_device *dev = nullptr;

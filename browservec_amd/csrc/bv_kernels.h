@@ -129,11 +129,10 @@ struct SlotArgs {
     float scale_mul;
     const void *q;            // prepared queries, q_stride bytes apart
     uint64_t q_stride;
-    const uint32_t *cand;     // indexed: query q scores rows cand[cand_off[q], cand_off[q + 1])
-    const uint64_t *cand_off; // (pick_topk: null for one query's rows cand[0, n))
+    const uint32_t *cand;     // rows_exact and its pick_topk: the rows are cand[0, n)
     const uint32_t *mask;     // row filter bits or null
     uint64_t mask_bits;
-    uint32_t n;               // rows (indexed: the most candidates of a query)
+    uint32_t n;               // rows
     uint32_t nq;
     uint32_t rw;              // rows per slot: a power of two, whole wave steps
     uint32_t nsub;            // parts per slot: a power of two; more than one: parts of whole step pairs

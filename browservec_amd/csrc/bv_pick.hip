@@ -19,6 +19,7 @@
 // Bound by latency: five dependent reads (best keys, slots, exact rows) of a
 // few hundred KB, 10-20 us a query, all queries at once.
 #include "bv_exact.h"
+#include "bv_mfma.h"
 #include "bv_scan.h"
 #include "bv_sort.h"
 
@@ -49,18 +50,8 @@ struct PickLds {
     uint32_t cnt, ns, np, sum, bin, excl, inbin;
 };
 
-// Inclusive prefix sum over the wave's lanes (DPP row shifts and broadcasts).
-__device__ __forceinline__ uint32_t pick_wave_scan(uint32_t x) {
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false);  // row_shr:1
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false);  // row_shr:2
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false);  // row_shr:4
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false);  // row_shr:8
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false);  // row_bcast:15
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false);  // row_bcast:31
-    return x;
-}
 __device__ __forceinline__ uint32_t pick_wave_sum(uint32_t x) {
-    return (uint32_t)__builtin_amdgcn_readlane((int)pick_wave_scan(x), 63);
+    return (uint32_t)__builtin_amdgcn_readlane((int)wave_incl_scan(x), 63);
 }
 
 // Lanes per row of the C_Q1P exact keys (0: another codec).
@@ -75,11 +66,7 @@ template <int LPR> __global__ __launch_bounds__(PICK_THREADS) void pick_topk(Pic
     const uint64_t *best = a.s.best + (uint64_t)q * nslots;
     const uint32_t *ord = a.s.ord + (uint64_t)q * nslots * a.s.rw;
     const uint32_t *cand = a.s.cand;
-    uint32_t n = a.s.n;
-    if (cand && a.s.cand_off) {
-        cand += a.s.cand_off[q];
-        n = (uint32_t)(a.s.cand_off[q + 1] - a.s.cand_off[q]);
-    }
+    const uint32_t n = a.s.n;
     const float *rq = a.rr_src ? a.rr_q + (uint64_t)q * a.rr_q_stride : nullptr;
 
     uint64_t kr[PICK_REG];
@@ -141,7 +128,7 @@ template <int LPR> __global__ __launch_bounds__(PICK_THREADS) void pick_topk(Pic
                 __syncthreads();
                 // thread t: bins 2047 - 2t and 2046 - 2t, counted from the top
                 const uint32_t h0 = L.hist[PICK_BINS - 1 - 2 * tid], h1 = L.hist[PICK_BINS - 2 - 2 * tid];
-                const uint32_t inc = pick_wave_scan(h0 + h1);
+                const uint32_t inc = wave_incl_scan(h0 + h1);
                 if (lane == 63) L.wsum[wave] = inc;
                 __syncthreads();
                 uint32_t run = inc - (h0 + h1);

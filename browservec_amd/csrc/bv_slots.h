@@ -1,6 +1,5 @@
 // The two-kernel search of short scans and small query batches: scan_slots
-// scores every row (or candidate) for up to NQ queries per pass over the
-// rows, pick_topk (bv_pick.hip) finds each query's best from what it left.
+// scores every row for up to NQ queries per pass over the rows, pick_topk (bv_pick.hip) finds each query's best from what it left.
 //
 // scan_slots cuts the rows into slots of a.rw rows, one wave per slot, and
 // writes every row's order word (the key's high word) and each slot's best
@@ -83,7 +82,7 @@ __device__ __forceinline__ void slots_step(const SlotArgs &a, const ScanRegs<C, 
     top = ord > top ? ord : top;
 }
 
-template <int C, int LPR, int UPL, bool IDX, int NQ>
+template <int C, int LPR, int UPL, int NQ>
 __global__ __launch_bounds__(SCAN_WG) void scan_slots(SlotArgs a) {
     using CD = Codec<C>;
     using QT = typename CD::QT;
@@ -93,12 +92,7 @@ __global__ __launch_bounds__(SCAN_WG) void scan_slots(SlotArgs a) {
     if (slot >= a.nslots) return;
     const uint32_t q0 = blockIdx.y * NQ;
     const int p = lane % LPR;
-    const uint32_t *cand = a.cand;
-    uint32_t n = a.n;
-    if (IDX) {
-        cand = a.cand + a.cand_off[q0];
-        n = (uint32_t)(a.cand_off[q0 + 1] - a.cand_off[q0]);
-    }
+    const uint32_t n = a.n;
     const uint32_t r0 = slot * a.rw;
     if (r0 >= n) {
 #pragma unroll
@@ -147,13 +141,13 @@ __global__ __launch_bounds__(SCAN_WG) void scan_slots(SlotArgs a) {
     // past the slot's end load its last row and are dropped: a load under a
     // condition would make the wave wait for both)
     StepData<C, LPR, UPL> A, B;
-    load_step<C, LPR, UPL, IDX>(la, R[0], cand, r0, r1, A, lane);
+    load_step<C, LPR, UPL, false>(la, R[0], nullptr, r0, r1, A, lane);
     for (uint32_t base = r0; base < r1; base += 2 * SH::RPS) {
-        load_step<C, LPR, UPL, IDX>(la, R[0], cand, base + SH::RPS, r1, B, lane);
+        load_step<C, LPR, UPL, false>(la, R[0], nullptr, base + SH::RPS, r1, B, lane);
 #pragma unroll
         for (int k = 0; k < NQ; ++k)
             slots_step<C, LPR, UPL>(a, R[k], A, base, r1, ordq[k], best[k], ptop[k], lane);
-        load_step<C, LPR, UPL, IDX>(la, R[0], cand, base + 2 * SH::RPS, r1, A, lane);
+        load_step<C, LPR, UPL, false>(la, R[0], nullptr, base + 2 * SH::RPS, r1, A, lane);
         if (base + SH::RPS < r1) {
 #pragma unroll
             for (int k = 0; k < NQ; ++k)
@@ -191,21 +185,18 @@ template <int C, int LPR, int UPL> hipError_t slots_go(const SlotArgs &a, hipStr
     using SH = ScanShape<C, LPR, UPL>;
     // slots of whole steps, parts of whole step pairs; row positions in 32 bits
     if (a.rw == 0 || a.rw % SH::RPS || a.nsub == 0 || a.rw % a.nsub || (a.nsub > 1 && a.rw / a.nsub % (2 * SH::RPS)) ||
-        a.nslots == 0 || a.nq == 0 || a.nq > SLOTS_MAX_NQ ||
+        a.cand || a.nslots == 0 || a.nq == 0 || a.nq > SLOTS_MAX_NQ ||
         (uint64_t)a.nslots * a.rw >= (1ull << 31) || (uint64_t)a.nslots * a.rw < a.n)
         return hipErrorInvalidValue;
     const uint32_t gx = (a.nslots + SH::WAVES - 1) / SH::WAVES;
     constexpr int MX = slots_nq_max<C, UPL>();
-    if (a.cand) {
-        if (!a.cand_off) return hipErrorInvalidValue;
-        hipLaunchKernelGGL((scan_slots<C, LPR, UPL, true, 1>), dim3(gx, a.nq), dim3(SCAN_WG), 0, s, a);
-    } else if (MX == 1 || a.nq == 1) {
-        hipLaunchKernelGGL((scan_slots<C, LPR, UPL, false, 1>), dim3(gx, a.nq), dim3(SCAN_WG), 0, s, a);
+    if (MX == 1 || a.nq == 1) {
+        hipLaunchKernelGGL((scan_slots<C, LPR, UPL, 1>), dim3(gx, a.nq), dim3(SCAN_WG), 0, s, a);
     } else if (MX == 2 || a.nq == 2) {
-        hipLaunchKernelGGL((scan_slots<C, LPR, UPL, false, MX == 1 ? 1 : 2>), dim3(gx, (a.nq + 1) / 2), dim3(SCAN_WG),
+        hipLaunchKernelGGL((scan_slots<C, LPR, UPL, MX == 1 ? 1 : 2>), dim3(gx, (a.nq + 1) / 2), dim3(SCAN_WG),
                            0, s, a);
     } else {
-        hipLaunchKernelGGL((scan_slots<C, LPR, UPL, false, MX>), dim3(gx, (a.nq + MX - 1) / MX), dim3(SCAN_WG), 0, s, a);
+        hipLaunchKernelGGL((scan_slots<C, LPR, UPL, MX>), dim3(gx, (a.nq + MX - 1) / MX), dim3(SCAN_WG), 0, s, a);
     }
     return hipGetLastError();
 }

@@ -404,7 +404,7 @@ class IVFQuantIndex(IVFIndex):
 class GraphSearcher:
     """HNSWGpuSearcher (src/index/hnswGpu.ts:28-244): corpus rows and the
     layer-0 adjacency on the device, beam search of query batches
-    (src/engine/wgsl/graphSearch.ts), one wave per query."""
+    (src/engine/wgsl/graphSearch.ts), one workgroup per query."""
 
     EF_CAP = 256
     EMPTY = 0xFFFFFFFF
