@@ -705,14 +705,16 @@ __global__ __launch_bounds__(256) void row_sqnorms(const float *rows, uint64_t n
         wmx[threadIdx.x >> 6] = __float_as_uint(ratio < 0x1p-8 ? (float)ratio : 0x1p-8f);
     }
     __syncthreads();
-    if (threadIdx.x == 0) {  // (two atomics per workgroup: they serialize)
+    if (threadIdx.x == 0) {  // (per workgroup: atomics serialize)
         uint32_t b = wmx[0], m = wsq[0];
         for (int i = 1; i < 4; ++i) {
             b = wmx[i] > b ? wmx[i] : b;
             m = wsq[i] > m ? wsq[i] : m;
         }
-        if (b) atomicMax(max_bits, b);
-        if (m) atomicMax(max_bits + 1, m);
+        // (the maxima only rise: what a plain read already passes need not be
+        // raised, and few workgroups hold a new maximum)
+        if (b > __hip_atomic_load(max_bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(max_bits, b);
+        if (m > __hip_atomic_load(max_bits + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(max_bits + 1, m);
     }
 }
 
