@@ -127,6 +127,9 @@ def test_overflow(ctx, kind, dim, n, nq):
     scanned = batch_equals_fused(idx, q.contiguous(), 100, 10)
     least = (n + SAMPLE) * nq + n * int(near.sum())
     assert least <= scanned < least + n * 8
+    rows, scores, cnt = idx.search(q.cpu().numpy(), 100, 10)  # (results in pinned memory)
+    again = search(idx, q.contiguous(), [0], nq, 100, 10)
+    assert np.array_equal(rows.view(np.int32), again[0]) and np.array_equal(scores.view(np.uint32), again[1])
     idx.destroy()
 
 
