@@ -531,7 +531,8 @@ hipError_t launch_ham_exact(const uint32_t *codes, uint32_t W, const uint32_t *q
 // Per query: its buckets joined into lk / uo [nq][cap] (after the list's
 // cnt[q] entries when append is set) and the length in cnt[q] (0xffffffff
 // when a bucket overflowed or the total exceeds cap).  spill_k (or null): the
-// entries of its spill list join them, and spill_n[q] is 0 again.
+// entries of its spill list join them (spill_cap and more: it overflowed), and
+// spill_n[q] is 0 again.
 hipError_t launch_mq1_compact(const uint64_t *bk, const uint32_t *bu, const uint32_t *bc, uint32_t nwg,
                               uint32_t capw, uint64_t cap, uint64_t *lk, uint32_t *uo, uint32_t *cnt, bool append,
                               uint32_t nq, hipStream_t s, const uint64_t *spill_k = nullptr,

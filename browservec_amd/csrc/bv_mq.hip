@@ -1093,7 +1093,7 @@ __global__ __launch_bounds__(1024) void mq1_compact(const uint64_t *bk, const ui
     const uint32_t base = append ? cnt[q] : 0u;  // entries already in the list
     if ((uint64_t)base > cap) return;             // already overflowed
     const uint32_t ns = spill_k ? spill_n[q] : 0u;
-    if (tid == 0) bad = ns > spill_cap;
+    if (tid == 0) bad = spill_k && ns >= spill_cap;  // (a list filled to the end may have been given up)
     __syncthreads();
     if (tid == 0 && spill_k) spill_n[q] = 0;
     // bucket lengths (one thread per bucket; nwg <= 1024) and their exclusive

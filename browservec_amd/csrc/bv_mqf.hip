@@ -379,7 +379,7 @@ __global__ __launch_bounds__(WAVES * 64) void mqf_scan(MqfArgs a) {
                     uint64_t at = 0;
                     if (m) at = atomicAdd(&a.cnt[nb + q], (uint32_t)__popc(m));
                     for (; m; m &= m - 1, ++at) {
-                        if (at >= a.cap) break;  // (a count past it tells mq1_compact)
+                        if (at >= a.cap) break;  // (a count of cap or more tells mq1_compact)
                         const uint64_t i = nb * a.capw + (uint64_t)q * a.cap + at;
                         entry(__builtin_ctz(m), a.cand[i], a.up_out[i]);
                     }

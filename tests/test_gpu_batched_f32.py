@@ -236,3 +236,35 @@ def test_only_overflowed_queries_are_run_again(ctx):
     least = (n + SAMPLE) * nq + (n + SAMPLE) * 100 + n * 50
     assert least < scanned < least + 50 * SAMPLE * 2 + nq * 4000
     idx.destroy()
+
+
+def test_a_spill_list_filled_to_its_end(ctx):
+    """All rows close to the queries lie in one workgroup's tiles, and one wave
+    fills the queries' spill lists with the first 512 of them to the last
+    entry; the closest rows lie in the tiles after those."""
+    import torch
+
+    from browservec_amd import FlatIndex
+
+    n, dim, nq, k = 5_000_000, 4, 64, 10
+    say("spill list full")
+    g = torch.Generator(device="cuda").manual_seed(4)
+    x = torch.randn(n, dim, generator=g, device="cuda") * 0.1
+    x[:, 0] = -1
+    wgs = ctx.info()["cu_count"] // 8 * 8  # one query block: every workgroup of the device
+    first = n // 8 // 32 * 32  # (the rows after the first eighth are a pass)
+    tile = torch.arange((n - first) // 32, device="cuda")
+    tile = tile[tile % wgs == 5]
+    assert len(tile) > 512
+    rows = (first + tile[:, None] * 32 + torch.arange(32, device="cuda")).flatten()
+    x[rows] = 0
+    x[rows, 0] = 1 + 0.0015 * torch.arange(len(rows), device="cuda") / len(rows)
+    q = torch.zeros(nq, dim, device="cuda")
+    q[:, 0] = 1
+    torch.cuda.synchronize()
+    idx = FlatIndex(ctx, dim, "dot")
+    idx.append_device(x.data_ptr(), n)
+    equals_fused(idx, q, nq, k)
+    best = idx.search(q[:1].cpu().numpy(), 0, k)[0][0]
+    assert (best > rows[512 * 32].item()).all()
+    idx.destroy()
